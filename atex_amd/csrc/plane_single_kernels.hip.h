@@ -152,8 +152,30 @@ __device__ __forceinline__ int plane_valid(int n_here) {
   return left <= 0 ? 0 : (n < U ? n : U);
 }
 
-// (mean, m2) of the chunk held in raw: exact two-pass per thread over its registers, Chan's merge
-// over the workgroup.  The same in every thread.
+// The triple of WIDTH lanes' triples, all of them merged at once (n > 0 somewhere).
+template <int WIDTH>
+__device__ __forceinline__ Wf plane_merge_lanes(const Wf& w) {
+#pragma clang fp contract(off)
+  const float n = group_sum<WIDTH>(w.n);
+  const float mean = n > 0.f ? group_sum<WIDTH>(w.mean * w.n) / n : 0.f;
+  const float d = w.mean - mean;
+  return Wf{mean, group_sum<WIDTH>(w.m2 + w.n * (d * d)), n};
+}
+// ... of the workgroup's threads.  buf: as for block_wf.
+__device__ __forceinline__ Wf plane_merge(const Wf& mine, Wf* buf) {
+  const Wf wave = plane_merge_lanes<kWave>(mine);
+  const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+  if (lane == 0) buf[threadIdx.x / kWave] = wave;
+  __syncthreads();
+  return plane_merge_lanes<kPlaneThreads / kWave>(buf[lane % (kPlaneThreads / kWave)]);
+}
+
+// (mean, m2) of the chunk held in raw, the same in every thread: exact two-pass per thread over its
+// registers, then Chan's merge over the workgroup, pairwise where every count is a power of two (FULL),
+// all lanes and then all waves at once otherwise: with counts of any size the pairwise merges, thirteen
+// approximate reciprocals one after another, pushed the mean of every plane of a shape the same way
+// (the mean's error against float64 at [4, 128, 50001] float32 3.7e-7, now 0.6e-7; [8, 64, 300001]
+// fp16 3.7e-7 and 0.5e-7; [2, 64, 157685] float32 1.26e-7 and 0.42e-7, at the same time).
 // edge: the thread's single element of a ragged plane, where it has one.
 template <typename T, int V, int U, bool FULL, bool RAGGED>
 __device__ __forceinline__ Wf plane_chunk_stats(Pack<T, V> (&raw)[U], int n_here, Wf* buf, bool has_edge, float edge) {
@@ -194,12 +216,12 @@ __device__ __forceinline__ Wf plane_chunk_stats(Pack<T, V> (&raw)[U], int n_here
       for (int i = 0; i < V; ++i) t += to_f32(raw[k].v[i]);
       s += k < nv ? t : 0.f;
     }
-    w.n = static_cast<float>(nv * V);
+    float n = static_cast<float>(nv * V);
     if (RAGGED && has_edge) {
       s += edge;
-      w.n += 1.f;
+      n += 1.f;
     }
-    w.mean = w.n > 0.f ? s / w.n : 0.f;
+    const float mean = n > 0.f ? s / n : 0.f;
     // (the second pass converts the elements again rather than keeping 64 floats alive)
 #pragma unroll
     for (int k = 0; k < U; ++k) forget_derived(raw[k]);
@@ -209,16 +231,16 @@ __device__ __forceinline__ Wf plane_chunk_stats(Pack<T, V> (&raw)[U], int n_here
       float t = 0.f;
 #pragma unroll
       for (int i = 0; i < V; ++i) {
-        const float d = to_f32(raw[k].v[i]) - w.mean;
+        const float d = to_f32(raw[k].v[i]) - mean;
         t += d * d;
       }
       q += k < nv ? t : 0.f;
     }
     if (RAGGED && has_edge) {
-      const float d = edge - w.mean;
+      const float d = edge - mean;
       q += d * d;
     }
-    w.m2 = q;
+    return plane_merge(Wf{mean, q, n}, buf);
   }
   return block_wf(w, buf, kPlaneThreads / kWave);
 }
@@ -387,10 +409,12 @@ __device__ __forceinline__ void plane_fwd_body(const T* __restrict__ x, cl_word*
   const PlaneEdge again = plane_edge<V, RAGGED>(g.s, S, rg, D);
   if (again.on) (y + g.row * D)[again.at] = from_f32<T>((to_f32(xe) - mean) * a + bt);
 }
-// (FULL: built for four workgroups per CU, 64 VGPRs, which the path that every launch takes needs
-// anyway; the fallback then keeps a few values in scratch memory)
+// (Built for four workgroups per CU, which the registers of the path that every launch takes allow
+// anyway, FULL in bf16 for three and other bf16 planes for two; the fallback then keeps a few values in
+// scratch memory.  Without the bound the float32 kernel of planes that do not fill their threads took 82
+// scalar registers instead of 78, which is another block of 16: [2, 32, 1000000] 86 us against 76.)
 template <typename T, int V, int U, bool FULL, bool NT>
-__global__ void __launch_bounds__(kPlaneThreads, FULL ? (__is_same(T, bf16_t) ? 6 : 8) : 4)
+__global__ void __launch_bounds__(kPlaneThreads, __is_same(T, bf16_t) ? (FULL ? 6 : 4) : 8)
 plane_fwd_single(const T* __restrict__ x, cl_word* tagged, unsigned* claims, const float* __restrict__ gamma,
                  const float* __restrict__ beta, T* __restrict__ y, float* __restrict__ mean_out,
                  float* __restrict__ rstd_out, int64_t n_rows, int n_vec, int S, int chunk_vec, int C, float eps,

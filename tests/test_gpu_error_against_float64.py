@@ -63,3 +63,31 @@ def test_weight_gradients_of_many_rows_per_workgroup(N, D, dtype):
     errors = _rel(dg, dg_ref), _rel(db, db_ref)
     print(f"LN bwd [{N}, {D}] {dtype}: {rows:.0f} rows per group, dgamma {errors[0]:.3e} dbeta {errors[1]:.3e} bound {bound:.3e}", flush=True)
     assert max(errors) <= bound
+
+
+@pytest.mark.parametrize("N,C,D,dtype", [(4, 64, 50001, "f32"), (2, 64, 157685, "f32"), (1, 300, 100003, "f16"), (5, 33, 110001, "bf16"),
+                                         (2, 32, 1500000, "f16"), (3, 64, 16388, "f32")])
+def test_means_of_planes_over_several_workgroups(N, C, D, dtype):
+    """Planes of a length that no power of two divides into (plane_fwd_ragged, and plane_fwd_single where
+    a thread holds fewer vectors than it could).  From a thread's mean on there are 22 roundings on the
+    way of every element: a product, six additions and a division in the wave, a product, three
+    additions and a division in the workgroup, a product, six additions and a product with 1 / D (itself
+    rounded) over the chunks.  Unbiased, as many leave sqrt(22) of one.  (That those of a wave or of a
+    chunk average out over 8 waves or S chunks is the bound's margin.)"""
+    import torch
+
+    bound = ROUNDING * 22 ** 0.5
+    capi = util.Capi()
+    g = torch.Generator(device="cuda").manual_seed(12)
+    x = torch.empty((N * C, D), device="cuda", dtype=util.torch_dtype(dtype))
+    ref = torch.empty(N * C, device="cuda", dtype=torch.float64)
+    for s in _in_slices(N * C, D):
+        offset = torch.rand((x[s].shape[0], 1), device="cuda", generator=g) * 4 - 2
+        x[s] = (torch.randn(x[s].shape, device="cuda", generator=g) + offset).to(x.dtype)
+        ref[s] = x[s].double().mean(1)
+    one, zero = torch.ones(C, device="cuda"), torch.zeros(C, device="cuda")
+    _, mean, _ = capi.in_fwd(x.view(N, C, D), one, zero, EPS, dtype, True)
+    torch.cuda.synchronize()
+    error = _rel(mean.view(-1), ref)
+    print(f"IN fwd channel-first [{N}, {C}, {D}] {dtype}: mean {error:.3e} bound {bound:.3e}", flush=True)
+    assert error <= bound
