@@ -6,6 +6,7 @@
 #include <cstdio>
 #include <cstring>
 
+#include "call_tag.h"
 #include "norm_common.hip.h"
 #include "plan.h"
 #include "rows_kernels.hip.h"
@@ -57,13 +58,13 @@ bool exchange_disabled() {
 
 __device__ unsigned g_recorded_calls;  // replays of recorded launches on this device so far
 __global__ void recorded_tag_kernel(unsigned origin, unsigned* word) {
-  *word = (origin + atomicAdd(&g_recorded_calls, 1u)) << 1;
+  *word = recorded_call_tag(origin, [] { return atomicAdd(&g_recorded_calls, 1u); });
 }
 }  // namespace
 
 unsigned next_call_tag() {
   static std::atomic<unsigned> counter{tag_origin()};
-  return counter.fetch_add(1, std::memory_order_relaxed) << 1 | 1u;
+  return host_call_tag(counter.fetch_add(1, std::memory_order_relaxed));
 }
 
 bool exchange_allowed(void* st) {
