@@ -5,7 +5,8 @@
 Each .hip translation unit is compiled to an object (in parallel), then linked into
 atex_amd/lib/libatex_norms_hip.so.  No CMake, no torch: the library depends only on the HIP
 runtime.  The host side of the op and layer calls on torch tensors is a Python extension of its own
-on top of that library's C ABI (csrc/torch_host.cc -> nv_norms/_torch_host.so).
+on top of that library's C ABI (csrc/torch_host.cc -> nv_norms/_torch_host.so), built where a ROCm
+torch is installed.
 
 A second library, libatex_norms_hip_bench.so, is the same sources compiled with
 -DATEXN_BENCH_BUILD: it adds the entry points of csrc/bench_hooks.h (launch-planning switches,
@@ -147,32 +148,55 @@ def _link(objs, path: str, force: bool) -> None:
             raise RuntimeError("link failed:\n" + r.stderr)
 
 
-def _build_torch_host(force: bool) -> None:
-    """nv_norms/_torch_host.so against the installed torch (found, not imported)."""
-    header = os.path.join(HERE, "..", "include", "atex_norms.h")
-    if not force and os.path.exists(TORCH_HOST_PATH) and \
-            os.path.getmtime(TORCH_HOST_PATH) >= max(os.path.getmtime(TORCH_HOST_SRC), os.path.getmtime(header)):
-        return
+def _torch_host_command(out: str):
+    """(command that builds nv_norms/_torch_host.so as `out` against the installed torch, which is found
+    and not imported; what the result depends on besides the sources), or None without a ROCm torch."""
     spec = importlib.util.find_spec("torch")
-    if spec is None:
-        raise RuntimeError("torch is not installed: nv_norms needs it")
+    if spec is None or not spec.submodule_search_locations:
+        return None
     torch_dir = spec.submodule_search_locations[0]
+    if not os.path.exists(os.path.join(torch_dir, "lib", "libtorch_hip.so")):
+        return None
     include = os.path.join(torch_dir, "include")
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     libs = ["torch", "torch_cpu", "torch_hip", "torch_python", "c10", "c10_hip"]
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            *(a for d in (include, os.path.join(include, "torch", "csrc", "api", "include"), os.path.join(rocm, "include"),
                          sysconfig.get_paths()["include"]) for a in ("-isystem", d)),
-           TORCH_HOST_SRC, "-o", TORCH_HOST_PATH, "-L" + os.path.join(torch_dir, "lib"), *("-l" + l for l in libs)]
+           TORCH_HOST_SRC, "-o", out, "-L" + os.path.join(torch_dir, "lib"), *("-l" + l for l in libs)]
+    with open(os.path.join(torch_dir, "version.py")) as f:
+        key = "\n".join([torch_dir, sysconfig.get_config_var("SOABI") or "", f.read()])
+    return cmd, key
+
+
+def _build_torch_host(force: bool) -> None:
+    """nv_norms/_torch_host.so; nothing, with a message, where there is no ROCm torch to build it for (the
+    C library needs none)."""
+    tmp = f"{TORCH_HOST_PATH}.{os.getpid()}"
+    found = _torch_host_command(tmp)
+    if found is None:
+        sys.stderr.write("no ROCm build of torch: nv_norms/_torch_host.so is left out\n")
+        return
+    cmd, key = found
+    header = os.path.join(HERE, "..", "include", "atex_norms.h")
+    stamp = os.path.join(OBJ_DIR, "torch_host.key")
+    if not force and os.path.exists(TORCH_HOST_PATH) and os.path.exists(stamp) and \
+            os.path.getmtime(TORCH_HOST_PATH) >= max(os.path.getmtime(TORCH_HOST_SRC), os.path.getmtime(header)):
+        with open(stamp) as f:
+            if f.read() == key:
+                return
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("g++ failed for torch_host.cc:\n" + r.stderr)
+    os.replace(tmp, TORCH_HOST_PATH)  # (a process that has the old one loaded keeps it)
+    with open(stamp, "w") as f:
+        f.write(key)
     if r.stderr.strip():
         sys.stderr.write(r.stderr)
 
 
 def build(force: bool = False, jobs: int = 8, bench: bool = True) -> str:
-    """Compiles the product library and (bench=True) the benchmark variant."""
+    """Compiles the product library and (bench=True) the benchmark variant, and the extension for torch."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     dep_m = _deps_mtime()
@@ -180,7 +204,6 @@ def build(force: bool = False, jobs: int = 8, bench: bool = True) -> str:
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
         host = ex.submit(_build_torch_host, force)
         objs = list(ex.map(lambda u: _compile(u[0], force, dep_m, u[1]), units))
-        host.result()
     _link(objs[:len(SOURCES)], LIB_PATH, force)
     merged = {}
     for o in objs[:len(SOURCES)]:
@@ -191,6 +214,7 @@ def build(force: bool = False, jobs: int = 8, bench: bool = True) -> str:
         json.dump(merged, f, indent=0, sort_keys=True)
     if bench:
         _link(objs[len(SOURCES):], BENCH_LIB_PATH, force)
+    host.result()  # (what is wrong there does not keep the libraries from being built)
     return LIB_PATH
 
 
