@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.normpath(os.path.join(_HERE, "..", "lib", "libatex_norms_hip.so"))
@@ -107,6 +108,14 @@ def lib() -> ctypes.CDLL:
 _host = None
 
 
+class _NoExtension:
+    """Stands in for the extension where it is not built or does not load (another torch than it was
+    built for): declines every call, so that it goes through ctypes."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def torch_host():
     """The host side of the op calls on torch GPU tensors (csrc/torch_host.cc), bound to lib()."""
     global _host
@@ -114,11 +123,13 @@ def torch_host():
         lib()
         try:
             from . import _torch_host
+            _torch_host.load(LIB_PATH)
+            _host = _torch_host
         except ImportError as e:
-            raise ImportError("atex_amd/nv_norms/_torch_host.so is missing or does not load: build it with "
-                              f"`python -m atex_amd.build` ({e})") from e
-        _torch_host.load(LIB_PATH)
-        _host = _torch_host
+            warnings.warn(f"atex_amd/nv_norms/_torch_host.so is missing or does not load ({e}): calls on GPU tensors go "
+                          "through ctypes, which costs small ones several times the host time; build it with "
+                          "`python -m atex_amd.build`", RuntimeWarning, stacklevel=2)
+            _host = _NoExtension()
     return _host
 
 

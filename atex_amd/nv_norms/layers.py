@@ -89,17 +89,19 @@ class _FusedInstanceNormFn(torch.autograd.Function):
 def fused_layer_norm(x, gamma, beta, axis=(-1,), epsilon=0.001):
     """Differentiable fused_layer_norm_op: returns (y, mean, inv_std)."""
     axis = tuple(axis)
-    out = ops._capi.torch_host().layer_norm_apply(x, gamma, beta, axis, float(epsilon))
-    if out is not None:
-        return ops._checked(out)
+    if x.is_cuda:
+        out = ops._capi.torch_host().layer_norm_apply(x, gamma, beta, axis, float(epsilon))
+        if out is not None:
+            return ops._checked(out)
     return _FusedLayerNormFn.apply(x, gamma, beta, axis, float(epsilon))
 
 
 def fused_instance_norm(x, gamma, beta, data_format="N...C", epsilon=0.001):
     """Differentiable fused_instance_norm_op: returns (y, mean, inv_std)."""
-    out = ops._capi.torch_host().instance_norm_apply(x, gamma, beta, data_format, float(epsilon))
-    if out is not None:
-        return ops._checked(out)
+    if x.is_cuda:
+        out = ops._capi.torch_host().instance_norm_apply(x, gamma, beta, data_format, float(epsilon))
+        if out is not None:
+            return ops._checked(out)
     return _FusedInstanceNormFn.apply(x, gamma, beta, data_format, float(epsilon))
 
 

@@ -113,9 +113,10 @@ def _checked(out):
 
 def fused_layer_norm_op(x: torch.Tensor, scale: torch.Tensor, offset: torch.Tensor,
                         axis: Sequence[int] = (-1,), epsilon: float = 0.001):
-    out = _capi.torch_host().layer_norm_fwd(x, scale, offset, axis, float(epsilon))
-    if out is not None:
-        return _checked(out)
+    if x.is_cuda:
+        out = _capi.torch_host().layer_norm_fwd(x, scale, offset, axis, float(epsilon))
+        if out is not None:
+            return _checked(out)
     L = _capi.lib()
     ax, n_ax = _axis_array(axis)
     xd, sd, od = _desc(x, "x"), _desc(scale, "scale"), _desc(offset, "offset")
@@ -138,9 +139,10 @@ def fused_layer_norm_grad_op(y_backprop: torch.Tensor, x: torch.Tensor, scale: t
                              reserve_space_1: torch.Tensor, reserve_space_2: torch.Tensor,
                              axis: Sequence[int] = (-1,), epsilon: float = 0.001):
     del epsilon  # attr of the op, unused by the gradient math (norm_ops.cc:172)
-    out = _capi.torch_host().layer_norm_bwd(y_backprop, x, scale, reserve_space_1, reserve_space_2, axis)
-    if out is not None:
-        return _checked(out)
+    if x.is_cuda:
+        out = _capi.torch_host().layer_norm_bwd(y_backprop, x, scale, reserve_space_1, reserve_space_2, axis)
+        if out is not None:
+            return _checked(out)
     L = _capi.lib()
     ax, n_ax = _axis_array(axis)
     dyd, xd, sd = _desc(y_backprop, "y_backprop"), _desc(x, "x"), _desc(scale, "scale")
@@ -167,9 +169,10 @@ def _fmt(data_format) -> bytes:
 
 def fused_instance_norm_op(x: torch.Tensor, scale: torch.Tensor, offset: torch.Tensor,
                            data_format: str = "N...C", epsilon: float = 0.001):
-    out = _capi.torch_host().instance_norm_fwd(x, scale, offset, data_format, float(epsilon))
-    if out is not None:
-        return _checked(out)
+    if x.is_cuda:
+        out = _capi.torch_host().instance_norm_fwd(x, scale, offset, data_format, float(epsilon))
+        if out is not None:
+            return _checked(out)
     L = _capi.lib()
     fmt = _fmt(data_format)
     xd, sd, od = _desc(x, "x"), _desc(scale, "scale"), _desc(offset, "offset")
@@ -194,9 +197,10 @@ def fused_instance_norm_grad_op(y_backprop: torch.Tensor, x: torch.Tensor, scale
                                 reserve_space_1: torch.Tensor, reserve_space_2: torch.Tensor,
                                 data_format: str = "N...C", epsilon: float = 0.001):
     del epsilon
-    out = _capi.torch_host().instance_norm_bwd(y_backprop, x, scale, reserve_space_1, reserve_space_2, data_format)
-    if out is not None:
-        return _checked(out)
+    if x.is_cuda:
+        out = _capi.torch_host().instance_norm_bwd(y_backprop, x, scale, reserve_space_1, reserve_space_2, data_format)
+        if out is not None:
+            return _checked(out)
     L = _capi.lib()
     fmt = _fmt(data_format)
     dyd, xd, sd = _desc(y_backprop, "y_backprop"), _desc(x, "x"), _desc(scale, "scale")

@@ -68,6 +68,7 @@ def test_same_bits_as_through_ctypes(kind, dtype, monkeypatch):
         assert not outs[-1].requires_grad
         return outs
 
+    assert _capi.torch_host().__file__.endswith("_torch_host.so")
     host = everything()
     monkeypatch.setattr(_capi, "_host", _NeverPlain())
     for i, (a, b) in enumerate(zip(host, everything())):
