@@ -10,7 +10,7 @@ from atex_amd.nv_norms import _capi
 
 
 def _calls():
-    x = torch.randn(3, 4, 8, requires_grad=True)
+    x = torch.randn(3, 4, 5, 8, requires_grad=True)
     g, b = torch.ones(8), torch.zeros(8)
     y, m, r = nv_norms.fused_layer_norm_op(x, g, b, axis=[-1])
     nv_norms.fused_layer_norm_grad_op(y, x, g, m, r, axis=[-1])
