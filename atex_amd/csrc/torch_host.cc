@@ -24,12 +24,14 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <dlfcn.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/autograd/variable.h>
 
+#include <algorithm>
 #include <array>
 #include <string>
 #include <vector>
@@ -66,6 +68,22 @@ struct Attr {
   std::vector<int> axes;
   std::string format;
 };
+
+// A valid attribute as a number that a saved_data entry holds without an allocation, and back: how many
+// axes, which are the last ones, or whether the channels come first.
+int64_t as_number(const Attr& a, int rank) {
+  if (!a.layer_norm) return a.format[1] == 'C';
+  unsigned seen = 0;
+  for (const int v : a.axes) seen |= 1u << (v < 0 ? v + rank : v);
+  return __builtin_popcount(seen);
+}
+Attr from_number(bool layer_norm, int64_t n) {
+  Attr a;
+  a.layer_norm = layer_norm;
+  if (!layer_norm) a.format = n != 0 ? "NC..." : "N...C";
+  else for (int64_t i = n; i > 0; --i) a.axes.push_back(static_cast<int>(-i));
+  return a;
+}
 
 // False: not the plain case.
 bool describe(const at::Tensor& t, const c10::Device& device, atexn_tensor& d) {
@@ -176,27 +194,77 @@ Result backward(const Attr& a, const at::Tensor& dy, const at::Tensor& x, const 
   return r;
 }
 
-// The gradient: one node for y; mean and inv_std are not differentiable.
+// What the gradient's nodes return: n tensors, the first three defined.
+torch::autograd::variable_list gradients(const Attr& a, const at::Tensor& grad, const at::Tensor& x, const at::Tensor& gamma,
+                                         const at::Tensor& mean, const at::Tensor& inv_std, size_t n) {
+  Result r = backward(a, grad.defined() ? grad.contiguous() : at::zeros_like(x), x, gamma, mean, inv_std);
+  const char* const name = a.layer_norm ? "FusedLayerNormBackward" : "FusedInstanceNormBackward";
+  TORCH_CHECK(r.plain, name, ": the gradient must be a dense tensor like the output");
+  TORCH_CHECK(r.status == ATEXN_OK, name, ": ", g_abi.last_error());
+  torch::autograd::variable_list out(n);
+  std::move(r.out.begin(), r.out.end(), out.begin());
+  return out;
+}
+
+// The gradient of y (mean and inv_std are not differentiable) as torch's own C++ autograd function.  It is
+// what compiled autograd can take apart; eager backwards go through the node below, which does the same
+// in 5 us less (an autograd step of a small layer: 34 us, 40 with this function's node).
+template <bool LAYER_NORM>
+struct FusedNorm : torch::autograd::Function<FusedNorm<LAYER_NORM>> {
+  static constexpr bool is_traceable = false;  // the backward calls the C ABI: data, not proxies
+
+  // y: what the node is attached to
+  static at::Tensor forward(torch::autograd::AutogradContext* ctx, const at::Tensor& x, const at::Tensor& gamma,
+                            const at::Tensor& /*beta*/, const Attr* a, const at::Tensor* y, const at::Tensor* mean,
+                            const at::Tensor* inv_std) {
+    ctx->save_for_backward({x, gamma, *mean, *inv_std});
+    ctx->set_materialize_grads(false);
+    ctx->saved_data["attr"] = as_number(*a, static_cast<int>(x.dim()));
+    return *y;
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    const torch::autograd::variable_list saved = ctx->get_saved_variables();
+    const Attr a = from_number(LAYER_NORM, ctx->saved_data["attr"].toInt());
+    return gradients(a, grads[0], saved[0], saved[1], saved[2], saved[3], /*n=*/7);
+  }
+};
+
+template <bool LAYER_NORM>
 struct FusedNormBackward : public torch::autograd::Node {
   Attr attr;
   torch::autograd::SavedVariable x, gamma, mean, inv_std;
+  mutable std::shared_ptr<torch::autograd::Node> compiled;  // FusedNorm's node over the same tensors, if asked for
 
-  std::string name() const override { return attr.layer_norm ? "FusedLayerNormBackward" : "FusedInstanceNormBackward"; }
+  std::string name() const override { return LAYER_NORM ? "FusedLayerNormBackward" : "FusedInstanceNormBackward"; }
   void release_variables() override {
     std::lock_guard<std::mutex> lock(mutex_);
     x.reset_data();
     gamma.reset_data();
     mean.reset_data();
     inv_std.reset_data();
+    if (compiled) compiled->release_variables();
   }
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
     const at::Tensor xv = x.unpack(), gv = gamma.unpack(), mv = mean.unpack(), rv = inv_std.unpack();
-    const at::Tensor dy = grads[0].defined() ? grads[0].contiguous() : at::zeros_like(xv);
-    Result r = backward(attr, dy, xv, gv, mv, rv);
-    TORCH_CHECK(r.plain, name(), ": the gradient must be a dense tensor like the output");
-    TORCH_CHECK(r.status == ATEXN_OK, name(), ": ", g_abi.last_error());
-    return {std::move(r.out[0]), std::move(r.out[1]), std::move(r.out[2])};
+    return gradients(attr, grads[0], xv, gv, mv, rv, /*n=*/3);
+  }
+  void compiled_args(torch::dynamo::autograd::CompiledNodeArgs& args) const override {
+    if (!compiled) {
+      const at::Tensor xv = x.unpack(), gv = gamma.unpack(), mv = mean.unpack(), rv = inv_std.unpack();
+      // y and beta stand for tensors that no longer exist: one element in the shape of x, and a value
+      // that has a gradient whatever x and gamma have
+      const at::Tensor y = at::empty_strided(xv.sizes(), std::vector<int64_t>(xv.dim(), 0), xv.options());
+      const at::AutoGradMode on(true);
+      compiled = FusedNorm<LAYER_NORM>::apply(xv, gv, at::empty_like(gv).requires_grad_(true), &attr, &y, &mv, &rv).grad_fn();
+      compiled->set_next_edges(torch::autograd::edge_list(next_edges()));
+    }
+    compiled->compiled_args(args);
+  }
+  torch::autograd::variable_list apply_with_saved(const torch::autograd::variable_list& inputs,
+                                                  torch::dynamo::autograd::SwapSavedVariables& saved) override {
+    return compiled->apply_with_saved(inputs, saved);
   }
 };
 
@@ -329,7 +397,7 @@ PyObject* norm_apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
     pybind11::gil_scoped_release no_gil;
     r = forward(a, x, gamma, beta, eps);
     if (r.plain && r.status == ATEXN_OK && torch::autograd::compute_requires_grad(x, gamma, beta)) {
-      auto node = std::shared_ptr<FusedNormBackward>(new FusedNormBackward(), torch::autograd::deleteNode);
+      auto node = std::shared_ptr<FusedNormBackward<LAYER_NORM>>(new FusedNormBackward<LAYER_NORM>(), torch::autograd::deleteNode);
       node->set_next_edges(torch::autograd::collect_next_edges(x, gamma, beta));
       node->attr = std::move(a);
       node->x = torch::autograd::SavedVariable(x, false);

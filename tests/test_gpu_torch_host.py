@@ -156,3 +156,22 @@ def test_tracers_modes_and_transforms_see_the_call(kind):
     assert seen.calls > 0
     with pytest.raises(RuntimeError, match="setup_context"):
         torch.vmap(lambda a: a + diff(x, gamma, beta)[0].sum())(dy)
+
+
+@pytest.mark.parametrize("kind", ["ln", "cl", "cf"])
+def test_compiled_autograd_takes_the_gradient(kind):
+    import torch
+    from torch._dynamo import compiled_autograd
+
+    x, gamma, beta, dy = _inputs(kind, torch.float32, grad=True)
+    diff = _ops(kind)[2]
+
+    def grads():
+        y = diff(x * 2.0, gamma, beta)[0]
+        return torch.autograd.grad(y * 3.0, [x, gamma, beta], dy)
+
+    eager = grads()
+    with compiled_autograd._enable(lambda graph: torch.compile(graph, backend="eager")):
+        compiled = grads()
+    for i, (a, b) in enumerate(zip(eager, compiled)):
+        assert torch.equal(a, b), f"gradient {i}"
