@@ -9,7 +9,8 @@
 // contiguous, on one GPU, of a storage type and rank that the C ABI has, with nobody listening to the
 // calls (a tracer, a dispatch mode, a functorch transform).  For anything else it
 // returns None and the caller goes the way it went before, which words the errors; a status of the
-// C ABI that is not OK comes back as an int, and the caller raises it.
+// C ABI that is not OK comes back as an int, and the caller raises it.  The autograd node, which has no
+// such caller, goes that way itself.
 //
 // Counterpart in the reference: the OpKernels' Compute methods (fused_layer_norm_op.cc:295-458,
 // fused_instance_norm_op.cc:328-534) and the registered gradients (nv_norm_ops.py:27-67).
@@ -24,6 +25,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <dlfcn.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -34,6 +36,7 @@
 #include <algorithm>
 #include <array>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/atex_norms.h"
@@ -194,13 +197,40 @@ Result backward(const Attr& a, const at::Tensor& dy, const at::Tensor& x, const 
   return r;
 }
 
+// The gradient op through nv_norms/ops.py, for what is not the plain case and for errors, which it words.
+std::array<at::Tensor, 3> gradients_in_python(const Attr& a, const at::Tensor& dy, const at::Tensor& x, const at::Tensor& gamma,
+                                              const at::Tensor& mean, const at::Tensor& inv_std) {
+  const pybind11::gil_scoped_acquire gil;
+  auto raise = [] {
+    python_error e;
+    e.persist();
+    throw python_error(std::move(e));
+  };
+  THPObjectPtr ops(PyImport_ImportModule("atex_amd.nv_norms.ops"));
+  if (!ops) raise();
+  THPObjectPtr attr(a.layer_norm ? PyList_New(static_cast<Py_ssize_t>(a.axes.size())) : PyUnicode_FromString(a.format.c_str()));
+  if (!attr) raise();
+  for (size_t i = 0; i < a.axes.size(); ++i) PyList_SET_ITEM(attr.get(), static_cast<Py_ssize_t>(i), PyLong_FromLong(a.axes[i]));
+  std::array<THPObjectPtr, 5> t;
+  const at::Tensor* const from[5] = {&dy, &x, &gamma, &mean, &inv_std};
+  for (int i = 0; i < 5; ++i) {
+    t[i] = THPObjectPtr(THPVariable_Wrap(*from[i]));
+    if (!t[i]) raise();
+  }
+  THPObjectPtr out(PyObject_CallMethod(ops.get(), a.layer_norm ? "fused_layer_norm_grad_op" : "fused_instance_norm_grad_op",
+                                             "OOOOOO", t[0].get(), t[1].get(), t[2].get(), t[3].get(), t[4].get(), attr.get()));
+  if (!out) raise();
+  std::array<at::Tensor, 3> r;
+  for (int i = 0; i < 3; ++i) r[i] = THPVariable_Unpack(PyTuple_GetItem(out.get(), i));
+  return r;
+}
+
 // What the gradient's nodes return: n tensors, the first three defined.
 torch::autograd::variable_list gradients(const Attr& a, const at::Tensor& grad, const at::Tensor& x, const at::Tensor& gamma,
                                          const at::Tensor& mean, const at::Tensor& inv_std, size_t n) {
-  Result r = backward(a, grad.defined() ? grad.contiguous() : at::zeros_like(x), x, gamma, mean, inv_std);
-  const char* const name = a.layer_norm ? "FusedLayerNormBackward" : "FusedInstanceNormBackward";
-  TORCH_CHECK(r.plain, name, ": the gradient must be a dense tensor like the output");
-  TORCH_CHECK(r.status == ATEXN_OK, name, ": ", g_abi.last_error());
+  const at::Tensor dy = grad.defined() ? grad.contiguous() : at::zeros_like(x);
+  Result r = backward(a, dy, x, gamma, mean, inv_std);
+  if (!r.plain || r.status != ATEXN_OK) r.out = gradients_in_python(a, dy, x, gamma, mean, inv_std);
   torch::autograd::variable_list out(n);
   std::move(r.out.begin(), r.out.end(), out.begin());
   return out;

@@ -175,3 +175,31 @@ def test_compiled_autograd_takes_the_gradient(kind):
         compiled = grads()
     for i, (a, b) in enumerate(zip(eager, compiled)):
         assert torch.equal(a, b), f"gradient {i}"
+
+
+@pytest.mark.parametrize("kind", ["ln", "cf"])
+def test_errors_of_the_backward_are_those_of_the_op(kind, monkeypatch):
+    """Saved-tensor hooks may hand the backward anything; what the op refuses raises the op's error."""
+    import torch
+
+    from atex_amd.nv_norms import InvalidArgumentError, _capi
+
+    x, gamma, beta, dy = _inputs(kind, torch.float32, grad=True)
+    diff = _ops(kind)[2]
+    swaps = [lambda t: t.transpose(0, 1).contiguous().transpose(0, 1), lambda t: t.double(), lambda t: t.cpu(),
+             lambda t: t[:1].contiguous()]
+
+    def errors():
+        got = []
+        for swap in swaps:
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: swap(t) if t.shape == x.shape else t):
+                y = diff(x, gamma, beta)[0]
+            with pytest.raises(Exception) as e:
+                torch.autograd.grad(y, [x, gamma, beta], dy)
+            got.append((type(e.value), str(e.value)))
+        return got
+
+    here = errors()
+    assert all(t is InvalidArgumentError for t, _ in here), here
+    monkeypatch.setattr(_capi, "_host", _NeverPlain())
+    assert here == errors()
