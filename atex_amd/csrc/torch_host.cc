@@ -7,7 +7,7 @@
 //
 // Every function here takes the plain case only: exact torch.Tensor (or Parameter) objects,
 // contiguous, on one GPU, of a storage type and rank that the C ABI has, with nobody listening to the
-// calls (a tracer, a dispatch mode, a functorch transform).  For anything else it
+// calls (a tracer, a dispatch or torch-function mode, a functorch transform).  For anything else it
 // returns None and the caller goes the way it went before, which words the errors; a status of the
 // C ABI that is not OK comes back as an int, and the caller raises it.  The autograd node, which has no
 // such caller, goes that way itself.
@@ -15,6 +15,7 @@
 // Counterpart in the reference: the OpKernels' Compute methods (fused_layer_norm_op.cc:295-458,
 // fused_instance_norm_op.cc:328-534) and the registered gradients (nv_norm_ops.py:27-67).
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TracerMode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/HIPContextLight.h>
@@ -25,6 +26,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <dlfcn.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/utils/object_ptr.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/function.h>
@@ -299,12 +301,26 @@ struct FusedNormBackward : public torch::autograd::Node {
 };
 
 // ------------------------------------------------------------------------------ arguments
+PyTypeObject* g_device_context = nullptr;  // torch.utils._device.DeviceContext
+
+// Whether a torch-function mode is on that may want to see the calls.  A default device (a with-block of
+// torch.device, torch.set_default_device) is such a mode, but one that only completes calls that name no
+// device, and there are none.
+bool function_mode_watches() {
+  if (!at::impl::torch_function_mode_enabled()) return false;
+  for (int64_t i = 0; i < at::impl::PythonTorchFunctionTLS::stack_len(); ++i) {
+    PyObject* const mode = at::impl::PythonTorchFunctionTLS::get_stack_at(i)->ptr(getPyInterpreter());
+    if (Py_TYPE(mode) != g_device_context) return true;
+  }
+  return false;
+}
 // False: somebody records, intercepts or transforms the calls of this thread.  What is done here
 // never reaches the dispatcher, so they would not see it (a traced layer would come out as a
 // constant).
 bool unobserved() {
   return !at::tracer::impl::is_dispatch_enabled() && !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
-         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+         !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
+         !function_mode_watches();
 }
 bool tensor_arg(PyObject* o, at::Tensor& t) {
   if (!THPVariable_CheckExact(o)) return false;
@@ -458,6 +474,10 @@ PyObject* load(PyObject*, PyObject* path) {
                   bind(lib, "atexn_fused_instance_norm_grad_workspace_bytes", g_abi.in_bwd_ws) &&
                   bind(lib, "atexn_fused_instance_norm_grad", g_abi.in_bwd);
   if (!ok) return nullptr;
+  THPObjectPtr device(PyImport_ImportModule("torch.utils._device"));
+  PyObject* const context = device ? PyObject_GetAttrString(device.get(), "DeviceContext") : nullptr;  // (kept)
+  if (context == nullptr) return nullptr;
+  g_device_context = reinterpret_cast<PyTypeObject*>(context);
   Py_RETURN_NONE;
 }
 

@@ -133,6 +133,7 @@ def test_tracers_modes_and_transforms_see_the_call(kind):
     """They never see what the extension does, so it leaves these calls to Python: a traced layer
     stays a function of its input."""
     import torch
+    from torch.overrides import TorchFunctionMode
     from torch.utils._python_dispatch import TorchDispatchMode
 
     from atex_amd import nv_norms as n
@@ -154,6 +155,18 @@ def test_tracers_modes_and_transforms_see_the_call(kind):
     with Seen() as seen:
         fwd(x, gamma, beta)
     assert seen.calls > 0
+
+    class Functions(TorchFunctionMode):
+        calls = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.calls += func in (torch.empty, torch.empty_like)
+            return func(*args, **(kwargs or {}))
+
+    for call in (fwd, diff):
+        with Functions() as seen, torch.device("cuda"):
+            call(x, gamma, beta)
+        assert seen.calls > 0
     with pytest.raises(RuntimeError, match="setup_context"):
         torch.vmap(lambda a: a + diff(x, gamma, beta)[0].sum())(dy)
 
@@ -203,3 +216,19 @@ def test_errors_of_the_backward_are_those_of_the_op(kind, monkeypatch):
     assert all(t is InvalidArgumentError for t, _ in here), here
     monkeypatch.setattr(_capi, "_host", _NeverPlain())
     assert here == errors()
+
+
+def test_a_default_device_is_not_in_the_way(monkeypatch):
+    """... though it is a torch-function mode: the extension takes the call."""
+    import torch
+
+    from atex_amd.nv_norms import ops
+
+    x, gamma, beta, _ = _inputs("ln", torch.float16)
+    fwd, _, _ = _ops("ln")
+    plain = fwd(x, gamma, beta)
+    monkeypatch.setattr(ops, "_desc", None)  # what the way through Python starts with
+    with torch.device("cuda"):
+        got = fwd(x, gamma, beta)
+    for a, b in zip(got, plain):
+        assert torch.equal(a, b)
