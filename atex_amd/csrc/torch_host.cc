@@ -16,11 +16,13 @@
 // fused_instance_norm_op.cc:328-534) and the registered gradients (nv_norm_ops.py:27-67).
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/SequenceNumber.h>
 #include <ATen/TracerMode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/HIPContextLight.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/record_function.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -441,6 +443,18 @@ PyObject* norm_apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Result r;
   {
     pybind11::gil_scoped_release no_gil;
+    // (what a profiler shows of the Python autograd function)
+    at::RecordFunction record(at::RecordScope::FUNCTION);
+    if (record.isActive()) {
+      const char* const name = LAYER_NORM ? "_FusedLayerNormFn" : "_FusedInstanceNormFn";
+      const int64_t sequence = static_cast<int64_t>(at::sequence_number::peek());  // the node's, below
+      if (record.needsInputs()) {
+        const std::array<c10::IValue, 3> inputs{x, gamma, beta};
+        record.before(name, c10::ArrayRef<const c10::IValue>(inputs.data(), inputs.size()), sequence);
+      } else {
+        record.before(name, sequence);
+      }
+    }
     r = forward(a, x, gamma, beta, eps);
     if (r.plain && r.status == ATEXN_OK && torch::autograd::compute_requires_grad(x, gamma, beta)) {
       auto node = std::shared_ptr<FusedNormBackward<LAYER_NORM>>(new FusedNormBackward<LAYER_NORM>(), torch::autograd::deleteNode);

@@ -232,3 +232,28 @@ def test_a_default_device_is_not_in_the_way(monkeypatch):
         got = fwd(x, gamma, beta)
     for a, b in zip(got, plain):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("kind", ["ln", "cl"])
+def test_a_profiler_sees_the_call(kind, monkeypatch):
+    """By the name, the inputs and the link from the backward that the Python autograd function has."""
+    import torch
+
+    from atex_amd.nv_norms import _capi
+
+    x, gamma, beta, dy = _inputs(kind, torch.float32, grad=True)
+    diff = _ops(kind)[2]
+    name = "_FusedLayerNormFn" if kind == "ln" else "_FusedInstanceNormFn"
+
+    def seen():
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU], record_shapes=True) as p:
+            y = diff(x, gamma, beta)[0]
+            torch.autograd.grad(y, [x, gamma, beta], dy)
+        calls = [e for e in p.events() if e.name == name]
+        backward = [e for e in p.events() if "evaluate_function" in e.name and e.sequence_nr == calls[0].sequence_nr]
+        return [e.input_shapes[:3] for e in calls], len(backward)
+
+    here = seen()
+    assert len(here[0]) == 1 and here[1] == 1, here
+    monkeypatch.setattr(_capi, "_host", _NeverPlain())
+    assert here == seen()
