@@ -295,6 +295,10 @@ int atexn_bench_describe_bwd(int op, int dtype, int layout, int64_t N, int64_t C
       if (p.lr.on)
         n = snprintf(out, out_bytes, "long_rows_bwd (S=%d chunks of %d vectors, %d groups, grid %d x %d threads) + col_reduce over %d partial rows; alone=0",
                      p.lr.S, p.lr.chunk_vec, p.lr.groups, p.lr.grid, kPlanLongThreads, p.lr.part_rows);
+      else if (p.plane_ragged)
+        n = snprintf(out, out_bytes, "plane_bwd_ragged (S=%d chunks of %d vectors, grid %d x %d threads; %s when dx == dy)%s; alone=0",
+                     p.ps_S, p.ps_chunk_vec, p.ps_grid, kPlanPlaneThreads, two,
+                     p.ps_fold ? ", plane sums folded over the batch in the kernel" : " + col_reduce");
       else if (p.plane_single)
         n = snprintf(out, out_bytes, "plane_bwd_single (S=%d chunks of %d vectors, grid %d x %d threads; %s when dx == dy or under capture)%s; alone=0",
                      p.ps_S, p.ps_chunk_vec, p.ps_grid, kPlanPlaneThreads, two,

@@ -276,6 +276,10 @@ def test_every_planning_parameter_is_settable_in_the_benchmark_build():
     assert b"cl_bwd_sums" in buf.value and b"alone=0" in buf.value
     assert L.atexn_bench_describe_bwd(1, 1, 0, 2, 32, 2097152, buf, 256) > 0
     assert b"plane_bwd_single (S=64" in buf.value and b"folded over the batch" in buf.value
+    # planes of any length: the split kernels' plan (few planes) and the staged kernels' (many) carry it
+    for n, c, d in ((2, 8, 300001), (8, 64, 36865)):
+        assert L.atexn_bench_describe_bwd(1, 1, 0, n, c, d, buf, 256) > 0
+        assert buf.value.startswith(b"plane_bwd_ragged") and buf.value.endswith(b"alone=0"), buf.value
 
 
 def test_workspace_queries_without_gpu(L):
