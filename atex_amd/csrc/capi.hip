@@ -144,7 +144,7 @@ int atexn_abi_version(void) { return kAbiVersion; }
 int atexn_set_tuning(const char* name, int value) {
   ATEXN_REQUIRE(name != nullptr && value >= 0, "bad tuning request");
   ATEXN_REQUIRE(value >= 1 || !strcmp(name, "reverse_second_pass") || !strcmp(name, "cl_fused") ||
-                    !strcmp(name, "cl_fold_cap") || !strcmp(name, "cl_single") || !strcmp(name, "affine_fold") || !strcmp(name, "affine_fold_polls") || !strcmp(name, "cl_single_polls") || !strcmp(name, "cl_single_xm") || !strcmp(name, "cl_single_occ") || !strcmp(name, "plane_single") || !strcmp(name, "plane_single_occ") || !strcmp(name, "plane_single_polls") || !strcmp(name, "bwd_lds_rows") || !strcmp(name, "staged_rows") || !strcmp(name, "cl_narrow_tiles") || !strcmp(name, "cl_fused_split") || !strcmp(name, "long_rows") || !strcmp(name, "long_rows_polls") || !strcmp(name, "long_rows_vpt") || !strcmp(name, "long_rows_chunks"),
+                    !strcmp(name, "cl_fold_cap") || !strcmp(name, "cl_single") || !strcmp(name, "affine_fold") || !strcmp(name, "affine_fold_polls") || !strcmp(name, "cl_single_polls") || !strcmp(name, "cl_single_xm") || !strcmp(name, "cl_single_occ") || !strcmp(name, "plane_single") || !strcmp(name, "plane_single_occ") || !strcmp(name, "plane_single_polls") || !strcmp(name, "bwd_lds_rows") || !strcmp(name, "staged_rows") || !strcmp(name, "cl_narrow_tiles") || !strcmp(name, "cl_fused_split") || !strcmp(name, "long_rows") || !strcmp(name, "long_rows_polls"),
                 "value must be >= 1");
   Tuning& t = tuning();
   if (!strcmp(name, "fwd_waves_per_cu")) t.fwd_waves_per_cu = value;
@@ -214,20 +214,11 @@ int atexn_set_tuning(const char* name, int value) {
   } else if (!strcmp(name, "plane_single_occ")) {
     ATEXN_REQUIRE(value == 0 || value == 1, "plane_single_occ must be 0 or 1");
     t.plane_single_occ = value;
-  } else if (!strcmp(name, "bwd_resident_max_vec")) {
-    ATEXN_REQUIRE(value >= 192 && value <= 2048, "bwd_resident_max_vec must be in [192, 2048]");
-    t.bwd_resident_max_vec = value;
   } else if (!strcmp(name, "long_rows")) {
     ATEXN_REQUIRE(value == 0 || value == 1, "long_rows must be 0 or 1");
     t.long_rows = value;
   } else if (!strcmp(name, "long_rows_polls")) {
     t.long_rows_polls = value;
-  } else if (!strcmp(name, "long_rows_vpt")) {
-    ATEXN_REQUIRE(value == 0 || value == 1 || value == 2 || value == 4, "long_rows_vpt must be 0 (the planner's choice), 1, 2 or 4");
-    t.long_rows_vpt = value;
-  } else if (!strcmp(name, "long_rows_chunks")) {
-    ATEXN_REQUIRE(value <= 64, "long_rows_chunks must be in [0, 64]");
-    t.long_rows_chunks = value;
   } else if (!strcmp(name, "plane_nt_min_mb")) {
     t.plane_nt_min_mb = value;
   } else if (!strcmp(name, "cl_single")) {

@@ -75,10 +75,7 @@ struct Tuning {
   TuneInt plane_single_occ{1};
   TuneInt long_rows{1};           // LayerNorm rows beyond one workgroup: one launch, one pass (long_rows_kernels.hip.h)
   TuneInt long_rows_polls{500};   //   and its polls
-  TuneInt long_rows_vpt{0};       //   vectors per thread: 0: by plan_long_rows, else at least that many
-  TuneInt long_rows_chunks{0};    //   workgroups per row: 0: by plan_long_rows
   TuneInt plane_nt_min_mb{256};  // forward: non-temporal loads of x from this many MiB (what no cache level retains anyway)
-  TuneInt bwd_resident_max_vec{2048};  // LayerNorm backward: longest register-resident row, in vectors
   TuneInt bwd_wave_groups{1};  // LayerNorm backward, 129..512 vectors per row: rows on 2 / 4 waves
   // Block-wide resident rows: longest row (in vectors) that uses 2 vectors per thread (more,
   // smaller-register threads) before switching to 4; forward <= 2048, backward <= 1536.
@@ -158,13 +155,11 @@ inline LongPlan plan_long_rows(bool bwd, int V, int64_t n_rows, int64_t D, int c
   const int64_t s_max = std::min<int64_t>(kPlanLongMaxChunks, slots);
   const int64_t rows8 = div_up(n_rows, kPlanXcdCount);
   double best = 1e300;
-  for (int vpt = std::max(1, t.long_rows_vpt.load()); vpt <= long_rows_max_vpt(bwd, V); vpt *= 2) {
+  for (int vpt = 1; vpt <= long_rows_max_vpt(bwd, V); vpt *= 2) {
     const int64_t s_min = div_up(n_vec, int64_t(kPlanLongThreads) * vpt);
     if (s_min > s_max) continue;
     for (int64_t g = 1; g <= std::min(rows8, slots / s_min); ++g) {
       int64_t S = std::max(s_min, std::min(std::min(s_max, slots / g), div_up(n_vec, 64)));
-      if (t.long_rows_chunks > 0) S = std::max(s_min, std::min<int64_t>(s_max, t.long_rows_chunks));
-      if (S * g > slots) continue;
       const int64_t chunk = div_up(n_vec, S);
       S = div_up(n_vec, chunk);
       LongPlan q;
@@ -267,7 +262,7 @@ constexpr int kPlanPlaneThreads = 512, kPlanPlaneVpt = 8, kPlanPlaneMaxChunks = 
 // dgamma / dbeta accumulators of its columns).
 // The channel-first InstanceNorm backward has no such accumulators and goes as far as the
 // forward.
-inline int64_t resident_limit(RowsKind kind) { return kind == RowsKind::kBwdCols ? tuning().bwd_resident_max_vec.load() : 4096; }
+inline int64_t resident_limit(RowsKind kind) { return kind == RowsKind::kBwdCols ? 2048 : 4096; }
 
 // LayerNorm backward beyond that: one more single-pass kernel keeps the dgamma / dbeta
 // accumulators of a workgroup's columns in LDS (rows_bwd_lds: 8 bytes per column, 8 vectors per
