@@ -8,16 +8,14 @@
 #include "plan.h"
 
 namespace atexn {
-// the product library's planner: its parameters are constants
-const Tuning& tuning() {
-  static const Tuning t;
-  return t;
-}
+// the product library's planner: its parameters are constants (but for long_rows, below)
+static Tuning g_tuning;
+const Tuning& tuning() { return g_tuning; }
 }  // namespace atexn
 
 using namespace atexn;
 
-static long g_checked = 0, g_failed = 0;
+static long g_checked = 0, g_failed = 0, g_long = 0, g_ragged = 0;
 
 #define EXPECT(cond, ...)                                   \
   do {                                                      \
@@ -30,6 +28,33 @@ static long g_checked = 0, g_failed = 0;
       }                                                     \
     }                                                       \
   } while (0)
+
+// What long_rows_fwd / long_rows_bwd and their launchers assume.  ws: the whole plan's workspace;
+// without: the workspace of the kernels that serve y == x (dx == dy), which share it.
+static void check_long(bool bwd, int V, int64_t n_rows, int64_t D, int cus, const LongPlan& p, size_t ws, size_t without) {
+  const int64_t n_vec = div_up(D, V), slots = cus / 8 * 2;
+  EXPECT(V > 1 && D >= V && D < (int64_t(1) << 29), "long rows: D=%lld V=%d", (long long)D, V);
+  const bool built = p.vpt == 1 || (p.vpt == 2 && !(bwd && V == 8)) || (p.vpt == 4 && V == 4 && !bwd);
+  EXPECT(built, "long rows: no kernel with %d vectors per thread, V=%d bwd=%d", p.vpt, V, int(bwd));
+  EXPECT(p.chunk_vec >= 1 && p.chunk_vec <= 512 * p.vpt, "long rows: chunks of %d vectors, vpt=%d", p.chunk_vec, p.vpt);
+  EXPECT(p.S >= 1 && p.S <= 64 && int64_t(p.S - 1) * p.chunk_vec < n_vec && n_vec <= int64_t(p.S) * p.chunk_vec,
+         "long rows: S=%d chunk=%d n_vec=%lld", p.S, p.chunk_vec, (long long)n_vec);
+  // every workgroup on the chip at once, the groups of an XCD on that XCD
+  EXPECT(p.groups >= 8 && p.groups % 8 == 0 && p.groups / 8 * int64_t(p.S) <= slots && p.grid == p.groups * p.S,
+         "long rows: S=%d groups=%d grid=%d cus=%d", p.S, p.groups, p.grid, cus);
+  EXPECT(p.groups / 8 <= div_up(n_rows, 8), "long rows: %d groups for %lld rows", p.groups, (long long)n_rows);
+  int64_t with_rows = 0;
+  for (int g = 0; g < p.groups; ++g) with_rows += g < n_rows;  // group g's first row is g
+  EXPECT(p.part_rows == with_rows, "long rows: %d partial rows of %lld groups with rows", p.part_rows, (long long)with_rows);
+  const size_t pairs = size_t(n_rows) * size_t(p.S);
+  EXPECT(p.off_tagged == 0 && p.off_claims >= 16 * pairs && p.off_tag >= p.off_claims + 4 * pairs && p.off_part >= p.off_tag + 4,
+         "long rows: workspace sections");
+  EXPECT(p.off_claims % 256 == 0 && p.off_tag % 256 == 0 && p.off_part % 256 == 0, "long rows: section alignment");
+  EXPECT(p.ws_bytes >= p.off_part + (bwd ? size_t(8) * size_t(D) * size_t(p.part_rows) : 0), "long rows: partial rows");
+  EXPECT(ws >= p.ws_bytes && ws >= without, "long rows: workspace");
+  // a backward that fits the static scratch buffer does so with this plan too
+  EXPECT(!bwd || without > kPlanStaticScratch || ws <= kPlanStaticScratch, "long rows: %zu bytes instead of %zu", ws, without);
+}
 
 static void check_rows(RowsKind kind, bool layer_norm, int vec, int64_t n_rows, int64_t D, int C, int cus) {
   ++g_checked;
@@ -66,24 +91,52 @@ static void check_rows(RowsKind kind, bool layer_norm, int vec, int64_t n_rows, 
       EXPECT(p.off_part >= p.off_rowsum + sizeof(float) * 2 * size_t(n_rows), "rowsum section");
       EXPECT(p.ws_bytes >= p.off_part + (p.sums_RS > 1 ? sizeof(float) * 2 * size_t(D) * size_t(p.sums_RS) : 0), "part section");
     }
+    if (p.lr.on) {
+      g_tuning.long_rows = 0;
+      const size_t without = plan_tiles(bwd, r.V, n_rows, D, cus).ws_bytes;
+      g_tuning.long_rows = 1;
+      check_long(bwd, r.V, n_rows, D, cus, p.lr, p.ws_bytes, without);
+      ++g_long;
+    }
     return;
   }
   const RowsPlan p = plan_rows(kind, r.V, n_rows, D, layer_norm ? 0 : C, cus);
   EXPECT(p.ragged == (D % r.V != 0), "ragged");
+  if (p.lr.on) {
+    g_tuning.long_rows = 0;
+    const size_t without = plan_rows(kind, r.V, n_rows, D, 0, cus).ws_bytes;
+    g_tuning.long_rows = 1;
+    EXPECT(kind == RowsKind::kBwdCols && p.resident, "long rows instead of another kernel than one for resident rows");
+    check_long(true, r.V, n_rows, D, cus, p.lr, p.ws_bytes, without);
+    ++g_long;
+  }
   // the one-launch plan for channel-first planes, where a plan carries one (`before`: bytes of the
   // workspace sections that precede its tagged pairs)
   auto check_plane_single = [&](size_t before) {
-  if (p.plane_single) {
+  EXPECT(!(p.plane_single && p.plane_ragged), "one plan for planes over several workgroups");
+  if (p.plane_single || p.plane_ragged) {
     // what plane_fwd_single / plane_bwd_single assume: whole vectors, chunks of at most 8
     // vectors per thread of 512, no more chunks than lanes in a wave or than an XCD holds such
-    // workgroups, a grid of whole planes per XCD, the tagged pairs behind the other sections
+    // workgroups, a grid of whole planes per XCD, the tagged pairs behind the other sections;
+    // plane_*_ragged: the same for whatever a plane that starts off a 16-byte boundary has left
     const int64_t n_vec = D / r.V;
-    EXPECT(D % r.V == 0 && r.V > 1 && C > 0, "plane single: D=%lld V=%d", (long long)D, r.V);
+    EXPECT((D % r.V == 0) == p.plane_single && r.V > 1 && C > 0, "plane single: D=%lld V=%d", (long long)D, r.V);
+    if (p.plane_ragged) {
+      ++g_ragged;
+      EXPECT(!p.ps_full, "ragged planes have no full chunks");
+      for (int head = 0; head < r.V; ++head) {
+        const int64_t last = (D - head) / r.V - int64_t(p.ps_S - 1) * p.ps_chunk_vec;
+        EXPECT(last >= 1 && last <= p.ps_chunk_vec, "ragged plane: %lld vectors in the last chunk of %d, head=%d, D=%lld", (long long)last, p.ps_chunk_vec, head, (long long)D);
+      }
+      EXPECT(p.off_ps_tag % 256 == 0 && p.off_ps_tag >= p.off_ps_claims + size_t(4) * size_t(n_rows) * size_t(p.ps_S) &&
+                 p.ws_bytes >= p.off_ps_tag + 4 && (!p.ps_fold || p.off_ps_fold >= p.off_ps_tag + 4),
+             "ragged plane: the tag's word");
+    }
     EXPECT(p.ps_S >= 2 && p.ps_S <= 64 && p.ps_S <= cus / 8 * 2, "plane single: S=%d cus=%d", p.ps_S, cus);
     EXPECT(p.ps_chunk_vec >= 1 && p.ps_chunk_vec <= 512 * 8, "plane single: chunk of %d vectors", p.ps_chunk_vec);
     EXPECT(int64_t(p.ps_S - 1) * p.ps_chunk_vec < n_vec && n_vec <= int64_t(p.ps_S) * p.ps_chunk_vec,
            "plane single: S=%d chunk=%d n_vec=%lld", p.ps_S, p.ps_chunk_vec, (long long)n_vec);
-    EXPECT(p.ps_full == (n_vec == int64_t(p.ps_S) * 4096), "plane single: full=%d", int(p.ps_full));
+    if (p.plane_single) EXPECT(p.ps_full == (n_vec == int64_t(p.ps_S) * 4096), "plane single: full=%d", int(p.ps_full));
     EXPECT(int64_t(p.ps_grid) == (n_rows + 7) / 8 * 8 * p.ps_S, "plane single: grid=%d", p.ps_grid);
     EXPECT(p.off_ps_tagged % 256 == 0 && p.off_ps_tagged >= before &&
                p.ws_bytes >= p.off_ps_tagged + size_t(16) * size_t(n_rows) * size_t(p.ps_S),
@@ -271,6 +324,13 @@ int main() {
           check_rows(RowsKind::kBwdCols, true, vec, n_rows, D, 1, cus);
         }
       }
+      // rows of about as many vectors as 64 workgroups hold, and longer ones
+      for (int64_t D : {262143, 262144, 262145, 524287, 524288, 524289, 1000003, 10000000}) {
+        for (int64_t n_rows : {1, 7, 8, 9, 100, 1000}) {
+          check_rows(RowsKind::kFwd, true, vec, n_rows, D, 1, cus);
+          check_rows(RowsKind::kBwdCols, true, vec, n_rows, D, 1, cus);
+        }
+      }
       // channel-first InstanceNorm: rows = N * C planes
       for (int64_t N : {1, 2, 8, 64, 100}) {
         for (int C : {1, 3, 32, 64, 100, 1024}) {
@@ -297,6 +357,6 @@ int main() {
     std::printf("%ld of %ld plans violate an invariant\n", g_failed, g_checked);
     return 1;
   }
-  std::printf("ok %ld\n", g_checked);
+  std::printf("ok %ld %ld %ld\n", g_checked, g_long, g_ragged);
   return 0;
 }

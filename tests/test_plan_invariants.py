@@ -17,4 +17,5 @@ def test_every_plan_satisfies_the_kernels_assumptions(tmp_path):
     run = subprocess.run([exe], capture_output=True, text=True)
     assert run.returncode == 0, run.stdout[-4000:]
     assert run.stdout.startswith("ok ")
-    assert int(run.stdout.split()[1]) > 1_000_000
+    checked, long_rows, ragged_planes = (int(v) for v in run.stdout.split()[1:])
+    assert checked > 1_000_000 and long_rows > 10_000 and ragged_planes > 10_000
