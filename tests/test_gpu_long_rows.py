@@ -65,8 +65,14 @@ def test_rows_over_several_workgroups(coracle, N, D, dtype):
             got = _step(capi, *dev, dtype)
             for name, a, b in zip(("y", "mean", "inv_std", "dx", "dgamma", "dbeta"), got, ref):
                 assert bool((a == b).all()), f"{polls} polls: {name} differs"
+        # as after a call whose waits ran out: patient waits are cut short
+        assert L.atexn_set_tuning(b"long_rows_polls", DEFAULT_POLLS) == 0
+        assert L.atexn_bench_mark_exchange_trouble(1) == 0
+        for name, a, b in zip(("y", "mean", "inv_std", "dx", "dgamma", "dbeta"), _step(capi, *dev, dtype), ref):
+            assert bool((a == b).all()), f"waits cut short: {name} differs"
     finally:
         L.atexn_set_tuning(b"long_rows_polls", DEFAULT_POLLS)
+        L.atexn_bench_mark_exchange_trouble(0)
 
 
 def test_in_place_rows_keep_to_one_workgroup_or_two_passes(coracle):

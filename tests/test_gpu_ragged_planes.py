@@ -64,8 +64,14 @@ def test_planes_of_any_length_over_several_workgroups(coracle, N, C, D, dtype):
             got = _step(capi, *dev, dtype)
             for name, a, b in zip(("y", "mean", "inv_std", "dx", "dgamma", "dbeta"), got, ref):
                 assert bool((a == b).all()), f"{polls} polls: {name} differs"
+        # as after a call whose waits ran out: patient waits are cut short
+        assert L.atexn_set_tuning(b"plane_single_polls", 500) == 0
+        assert L.atexn_bench_mark_exchange_trouble(1) == 0
+        for name, a, b in zip(("y", "mean", "inv_std", "dx", "dgamma", "dbeta"), _step(capi, *dev, dtype), ref):
+            assert bool((a == b).all()), f"waits cut short: {name} differs"
     finally:
         L.atexn_set_tuning(b"plane_single_polls", 500)
+        L.atexn_bench_mark_exchange_trouble(0)
 
 
 @pytest.mark.parametrize("shift_x,shift_dy", [(1, 0), (3, 3), (0, 5)])
@@ -87,3 +93,31 @@ def test_in_place(coracle):
     dx, dg, db = capi.in_bwd(dyd, x_keep, gd, m, r, "f16", True, dx=dyd)
     torch.cuda.synchronize()
     _check(coracle, host, (y, m, r, dx, dg, db), "f16")
+
+
+@pytest.mark.parametrize("N,C,D", [(2, 8, 40001), (3, 5, 70003)])
+def test_replays_of_a_recorded_launch_take_new_data(N, C, D):
+    """Every replay draws its own tag; with the fold over the batch in the kernel (C = 8) and without."""
+    import torch
+
+    capi = util.Capi()
+    dtype = "f16"
+    _, (xd, gd, bd, dyd) = _device(N, C, D, dtype, 63)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _step(capi, xd, gd, bd, dyd, dtype)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y, m, r = capi.in_fwd(xd, gd, bd, EPS, dtype, True)
+        outs = (y, m, r) + tuple(capi.in_bwd(dyd, xd, gd, m, r, dtype, True))
+    for replay in range(4):
+        xd.copy_(torch.randn(xd.shape, device="cuda").to(xd.dtype) * (replay + 1))
+        for t in outs:
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(outs, _step(capi, xd, gd, bd, dyd, dtype)):
+            assert torch.equal(a, b), f"replay {replay}"

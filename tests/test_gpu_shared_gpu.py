@@ -72,6 +72,52 @@ def test_results_do_not_depend_on_who_else_runs(N, C, S, cf):
           f"{recorded} of 4 runs beside the occupier recorded a wait that ran out", flush=True)
 
 
+@pytest.mark.parametrize("kind,shape,dtype", [("ln", (300, 40001), "f16"), ("ln", (30, 200000), "bf16"), ("ln", (20, 60001), "f32"),
+                                              ("cf", (2, 8, 300001), "f16"), ("cf", (1, 8, 1500001), "f16"), ("cf", (2, 3, 700001), "f32")])
+def test_long_rows_and_ragged_planes_beside_the_occupier(kind, shape, dtype):
+    """LayerNorm rows over several workgroups, one row after another, and planes of any length: on fewer
+    workgroups than an XCD still has places for, and on more, where waits run out."""
+    import torch
+
+    capi = util.Capi(bench=True)
+    L = capi.L
+    gen = torch.Generator(device="cuda").manual_seed(78)
+    x = torch.randn(shape, device="cuda", generator=gen).to(util.torch_dtype(dtype))
+    dy = torch.randn(shape, device="cuda", generator=gen).to(util.torch_dtype(dtype))
+    width = shape[1]
+    gamma = torch.rand(width, device="cuda", generator=gen) + 0.5
+    beta = torch.randn(width, device="cuda", generator=gen) * 0.1
+    side = torch.cuda.Stream()
+    print(kind, shape, dtype, flush=True)
+
+    def run():
+        if kind == "ln":
+            y, m, r = capi.ln_fwd(x, gamma, beta, EPS, dtype)
+            return (y, m, r) + tuple(capi.ln_bwd(dy, x, gamma, m, r, dtype))
+        y, m, r = capi.in_fwd(x, gamma, beta, EPS, dtype, True)
+        return (y, m, r) + tuple(capi.in_bwd(dy, x, gamma, m, r, dtype, True))
+
+    assert L.atexn_bench_mark_exchange_trouble(0) == 0
+    alone = run()
+    recorded = 0
+    try:
+        for wgs in (192, 128):
+            for rep in range(2):
+                torch.cuda.synchronize()
+                assert L.atexn_bench_occupy(wgs, 20.0, side.cuda_stream) == 0
+                torch.cuda._sleep(400000)  # the occupier gets its CUs first
+                shared = run()
+                torch.cuda.synchronize()
+                for n_, a, b in zip(("y", "mean", "inv_std", "dx", "dgamma", "dbeta"), alone, shared):
+                    assert torch.equal(_bits(a), _bits(b)), f"beside {wgs} occupied CUs, run {rep}: {n_} differs"
+                age = L.atexn_bench_exchange_trouble_age()
+                recorded += 0 <= age < 64
+    finally:
+        torch.cuda.synchronize()
+        L.atexn_bench_mark_exchange_trouble(0)
+    print(f"{recorded} of 4 runs beside the occupier recorded a wait that ran out", flush=True)
+
+
 @pytest.mark.parametrize("seed", range(N_SEEDS))
 def test_random_shapes_beside_the_occupier(seed):
     """Shapes of every kernel family that exchanges results (and a few that do not), in the three

@@ -257,3 +257,121 @@ def test_a_profiler_sees_the_call(kind, monkeypatch):
     assert len(here[0]) == 1 and here[1] == 1, here
     monkeypatch.setattr(_capi, "_host", _NeverPlain())
     assert here == seen()
+
+
+@pytest.mark.parametrize("kind", ["ln", "cl", "cf"])
+def test_side_streams_and_threads(kind):
+    """The current stream of the calling thread, for the outputs and the scratch memory too: what the
+    allocator hands out again is not written by a call that is still running on another stream."""
+    import threading
+
+    import torch
+
+    _, _, diff = _ops(kind)
+    inputs = [[t.detach().clone().requires_grad_(i < 3) for i, t in enumerate(_inputs(kind, torch.float16))] for _ in range(3)]
+    for i, (x, _, _, dy) in enumerate(inputs):
+        with torch.no_grad():
+            x.add_(i)
+            dy.mul_(i + 1)
+
+    def step(x, gamma, beta, dy):
+        y = diff(x * 2.0, gamma, beta)[0]
+        return [y.detach(), *torch.autograd.grad(y, [x, gamma, beta], dy)]
+
+    want = [step(*i) for i in inputs]
+    torch.cuda.synchronize()
+    got = [None] * 3
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                got[i] = step(*inputs[i])
+        stream.synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, b in zip(want, got):
+        for p, q in zip(a, b):
+            assert torch.equal(p, q)
+
+
+@pytest.mark.parametrize("kind", ["ln", "cf"])
+def test_captured_steps(kind):
+    import torch
+
+    x, gamma, beta, dy = _inputs(kind, torch.float16, grad=True)
+    diff = _ops(kind)[2]
+
+    def step():
+        y = diff(x, gamma, beta)[0]
+        return [y, *torch.autograd.grad(y, [x, gamma, beta], dy)]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = step()
+    for replay in range(3):
+        with torch.no_grad():
+            x.mul_(1.5).add_(0.25)
+        want = [t.detach().clone() for t in step()]
+        for t in outs:
+            t.detach().fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(outs, want):
+            assert torch.equal(a.detach(), b), f"replay {replay}"
+
+
+def test_saved_tensor_hooks_and_checkpoints():
+    import torch
+    from torch.utils.checkpoint import checkpoint
+
+    x, gamma, beta, dy = _inputs("ln", torch.float32, grad=True)
+    diff = _ops("ln")[2]
+    want = torch.autograd.grad(diff(x, gamma, beta)[0], [x, gamma, beta], dy)
+    packed = []
+
+    def pack(t):
+        packed.append(t.shape)
+        return t.cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        y = diff(x, gamma, beta)[0]
+    assert sorted(packed) == sorted([x.shape, gamma.shape, torch.Size([30]), torch.Size([30])])
+    for a, b in zip(want, torch.autograd.grad(y, [x, gamma, beta], dy)):
+        assert torch.equal(a, b)
+    y = checkpoint(lambda t: diff(t, gamma, beta)[0], x, use_reentrant=False)
+    for a, b in zip(want, torch.autograd.grad(y, [x, gamma, beta], dy)):
+        assert torch.equal(a, b)
+
+
+def test_inference_mode_and_forward_mode(monkeypatch):
+    import torch
+    from torch.autograd import forward_ad
+
+    from atex_amd.nv_norms import _capi
+
+    x, gamma, beta, dy = _inputs("cl", torch.float32)
+    diff = _ops("cl")[2]
+    want = diff(x, gamma, beta)[0]
+    with torch.inference_mode():
+        y = diff(x, gamma, beta)[0]
+        assert y.is_inference() and torch.equal(y, want)
+
+    def refusal():  # no forward-mode formula: refused, not silently without a tangent
+        with forward_ad.dual_level(), pytest.raises(Exception) as e:
+            diff(forward_ad.make_dual(x, dy), gamma, beta)
+        return type(e.value), str(e.value)
+
+    here = refusal()
+    monkeypatch.setattr(_capi, "_host", _NeverPlain())
+    assert here == refusal()

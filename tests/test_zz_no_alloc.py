@@ -63,6 +63,20 @@ def test_static_scratch_matches_workspace_entry(dtype, shapes):
         assert _same_bits(db, db_ref), "dbeta differs"
 
 
+@pytest.mark.parametrize("dtype,shapes", [("f16", [(8, 70001), (24, 18432)]), ("f32", [(40, 16385), (12, 9001)])])
+def test_static_scratch_matches_workspace_entry_on_long_rows(dtype, shapes):
+    """Rows over several workgroups (long_rows_bwd): tagged words and claims of an earlier call are in the
+    scratch array when the next one polls it."""
+    from oracle import oracle as O
+
+    L = util.Capi(bench=True).L
+    for N, D in shapes:
+        text = ctypes.create_string_buffer(512)
+        assert L.atexn_bench_describe_bwd(0, O.DTYPE_CODE[dtype], 0, N, 1, D, text, 512) > 0
+        assert text.value.startswith(b"long_rows_bwd"), text.value
+    test_static_scratch_matches_workspace_entry(dtype, shapes + shapes)
+
+
 def test_static_scratch_limit_and_empty():
     import torch
 
