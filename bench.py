@@ -94,6 +94,8 @@ CASES = {
     "ln_8192x12288_f32": ("ln", "f32", (8192, 12288)),
     # 1024 channel-first planes of 256 x 256: staged in registers + LDS, single pass
     "in_16x64x256x256_cf": ("in", "f16", (16, 64, 256 * 256, True)),
+    # channel-first planes of an odd length: over several workgroups each, off every alignment
+    "in_2x64x157685_cf_f32": ("in", "f32", (2, 64, 157685, True)),
     # more instances than the chip holds workgroups for at once: the channels-last single-launch
     # kernels on their XCD-major grid
     "in_16x128x128x64_cl": ("in", "f16", (16, 64, 128 * 128, False)),
