@@ -421,7 +421,7 @@ inline RowsPlan plan_rows(RowsKind kind, int V, int64_t n_rows, int64_t D, int C
     }
     // (the one-launch kernels over the workgroups of an XCD, where they apply, are faster:
     // [16, 64, 256, 256] fp16 44.7 / 86.1 us staged, 41.9 / 74.8 us so; the staged kernels then
-    // serve y == x, stream capture and ragged planes)
+    // serve y == x and, for planes of whole vectors, stream capture)
     plan_plane_single(p, kind, V, n_rows, D, C, cus, p.ws_bytes);
     return p;
   }

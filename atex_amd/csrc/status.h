@@ -15,16 +15,16 @@ const char* last_error();
 // queried, so that the workspace queries stay usable on a host without a GPU.
 int cu_count();
 
-// A tag that no earlier call of this process has used (never 0): the single-launch
-// channels-last kernels mark the partial results they exchange with it, so that whatever an
-// earlier call left in the caller's workspace is never taken for data of this one.  A
-// process-wide atomic counter, started from the clock.
+// A tag that no earlier call of this process has used (odd, so never 0): kernels whose workgroups
+// exchange partial results mark them with it, so that whatever an earlier call left in the caller's
+// workspace is never taken for data of this one.  A process-wide atomic counter, started from the clock.
 unsigned next_call_tag();
 
-// Whether a call on stream `st` may take the kernels whose workgroups exchange partial results
-// while they run.  Not while the stream is being captured (a graph replay would repeat the call's
-// tag), and not in a process started with ATEXN_NO_EXCHANGE set to anything but "0": those
-// kernels need the workgroups of one instance / plane on the chip together, which a process that
+// Whether a call on stream `st` may take the InstanceNorm kernels whose workgroups exchange partial
+// results under a tag from the host.  Not while the stream is being captured (a graph replay would
+// repeat the call's tag; LayerNorm's long rows and ragged planes take theirs from exchange_tag below and
+// are recorded as they are), and neither these nor those in a process started with ATEXN_NO_EXCHANGE set
+// to anything but "0": such kernels need the workgroups of one instance / plane on the chip together, which a process that
 // keeps other kernels resident on the same GPU (communication kernels overlapped with compute)
 // may never give them; every wait then runs out and every workgroup recomputes its peers' share.
 // The results are the same; the time is not.  The variable is read once, at the first call.
@@ -60,7 +60,7 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // is being captured gets no number of its own, since every replay would repeat it: a one-thread
 // kernel is recorded ahead of the launch that takes the next number of a device-wide counter and
 // leaves it at `word` (device memory, 4 bytes, part of the caller's workspace), and the launch reads
-// its tag there (`at`).  Host tags are odd, recorded ones even.  Eager calls and replays thus run the
+// its tag there (`at`).  Host tags are odd, recorded ones even and not 0 (call_tag.h).  Eager calls and replays thus run the
 // same kernels, to the same bits.
 struct ExchangeTag {
   bool ok = false;

@@ -29,12 +29,12 @@
  *     in vain, and only makes the next calls give such waits up sooner); the library has no
  *     process-wide settings: launch plans depend on the sizes and the device alone.  One
  *     environment variable is read, once, at the first call: ATEXN_NO_EXCHANGE=1 keeps every
- *     InstanceNorm call on kernels that need no group of workgroups resident on the GPU
- *     together (two launches per direction instead of one for some shapes; same results up to
- *     the order of a few float32 additions in the statistics, same workspace sizes) -- for
- *     processes that keep other kernels running on more than half of the GPU's compute units
- *     all the time, under which the one-launch kernels are correct but two to three times slower
- *     than the two launches;
+ *     call on kernels that need no group of workgroups resident on the GPU together (for some
+ *     InstanceNorm shapes two launches per direction instead of one, for LayerNorm rows of more
+ *     than one workgroup three or four; same results up to the order of a few float32 additions,
+ *     same workspace sizes) -- for processes that keep other kernels running on more than half
+ *     of the GPU's compute units all the time, under which the one-launch kernels are correct but
+ *     two to three times slower than the others;
  *   - the device the stream belongs to must be the calling thread's current device: launch
  *     plans and workspace sizes are made for the current device's compute-unit count;
  *   - data pointers need only the alignment of their element type (2 or 4 bytes): the
@@ -113,7 +113,8 @@ int atexn_layer_norm_bwd(int dtype, const void* dy, const void* x, const float* 
  * ATEXN_INVALID_ARGUMENT.  All calls on one GPU share the one array: calls that overlap in
  * time on the same GPU (two streams, two threads) race; serialise them or use
  * atexn_layer_norm_bwd with separate workspaces.  Nothing has to be cleared between calls
- * (the kernels write every scratch word before they read it).  The first call on a device
+ * (kernels whose workgroups exchange results do read words that an earlier call has left, and
+ * recognise their own by the call's tag; every other word is written before it is read).  The first call on a device
  * looks the array's address up (hipGetSymbolAddress); make that call outside stream capture.
  * Results are bit-identical to atexn_layer_norm_bwd. */
 #define ATEXN_STATIC_SCRATCH_BYTES (8u << 20)

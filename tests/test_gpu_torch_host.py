@@ -375,3 +375,22 @@ def test_inference_mode_and_forward_mode(monkeypatch):
     here = refusal()
     monkeypatch.setattr(_capi, "_host", _NeverPlain())
     assert here == refusal()
+
+
+@pytest.mark.parametrize("kind", ["ln", "cf"])
+def test_a_compiled_model_breaks_its_graph_at_the_call(kind):
+    import torch
+
+    from atex_amd import nv_norms as n
+
+    x, _, _, dy = _inputs(kind, torch.float32, grad=True)
+    layer = n.LayerNormalization(axis=-1) if kind == "ln" else n.InstanceNormalization(axis=1)
+    layer.build(x.shape, device="cuda")
+    model = torch.nn.Sequential(torch.nn.ReLU(), layer, torch.nn.ReLU())
+
+    def step(f):
+        y = f(x)
+        return [y.detach(), *torch.autograd.grad(y, [x, layer.gamma, layer.beta], dy)]
+
+    for a, b in zip(step(model), step(torch.compile(model, backend="eager"))):
+        assert torch.equal(a, b)
