@@ -158,8 +158,9 @@ int fill_zero(float* out, int64_t n, hipStream_t st) {
   return ATEXN_OK;
 }
 
-int launch_col_reduce(const float* part, float* out0, float* out1, int G, int64_t W,
-                      hipStream_t st, int batch, int64_t part_stride, int64_t out_stride) {
+template <typename SUM>
+static int col_reduce_in(const float* part, float* out0, float* out1, int G, int64_t W, hipStream_t st, int batch,
+                         int64_t part_stride, int64_t out_stride) {
   ATEXN_REQUIRE(2 * W < (int64_t(1) << 31), "column count %lld too large", (long long)W);
   const int Wi = static_cast<int>(W);
   // Column groups per block (CX): the more, the longer the contiguous run a wave reads per
@@ -170,7 +171,7 @@ int launch_col_reduce(const float* part, float* out0, float* out1, int G, int64_
     return div_up(2 * W, int64_t(cw) * cx) * batch >= cus && (256 / cx) * 2 <= std::max(G, 2);
   };
 #define ATEXN_COL_REDUCE(CW_, CX_)                                                              \
-  col_reduce<CW_, CX_><<<dim3(static_cast<unsigned>(div_up(2 * W, int64_t(CW_) * CX_)), batch),  \
+  col_reduce<CW_, CX_, SUM><<<dim3(static_cast<unsigned>(div_up(2 * W, int64_t(CW_) * CX_)), batch),  \
                          kColReduceThreads, 0, st>>>(part, out0, out1, G, Wi, part_stride,      \
                                                      out_stride)
   if (W % 4 == 0) {
@@ -193,6 +194,13 @@ int launch_col_reduce(const float* part, float* out0, float* out1, int G, int64_
 #undef ATEXN_COL_REDUCE
   ATEXN_CHECK_LAUNCH("col_reduce");
   return ATEXN_OK;
+}
+int launch_col_reduce(const float* part, float* out0, float* out1, int G, int64_t W,
+                      hipStream_t st, int batch, int64_t part_stride, int64_t out_stride) {
+  return col_reduce_in<float>(part, out0, out1, G, W, st, batch, part_stride, out_stride);
+}
+int launch_col_reduce_double(const float* part, float* out0, float* out1, int G, int64_t W, hipStream_t st) {
+  return col_reduce_in<double>(part, out0, out1, G, W, st, 1, 0, 0);
 }
 
 // --------------------------------------------------------------------- dtype dispatch

@@ -1385,13 +1385,15 @@ rows_bwd_staged(const T* dy, const T* __restrict__ x, const float* __restrict__ 
 // Block of 256 threads = CX column groups of CW floats x (256 / CX) slices of g; a block
 // owns CX * CW adjacent columns of the concatenated [2W] row, so the grid has
 // 2W / (CX * CW) blocks (128 for W = 1024).  Slices are folded by a lane butterfly and a
-// 4-entry LDS step.  A thread's slice, up to G additions one after another, is summed in double:
-// the partial rows are read once whatever the sum is held in, and float32 there made up a third of
-// the weights' error against float64 ([500, 68001] float32 dgamma 0.96e-7, now 0.77e-7; [804, 16844]
-// fp16 0.96e-7, now 0.87e-7), at the same time.
+// 4-entry LDS step.  SUM: what a thread sums its slice in, up to G additions one after another.  float,
+// as the kernels do that fold the same sums themselves (a captured channel-first call, which ends in
+// a column reduction, has the bits of an eager one); double for the partial rows of long_rows_bwd, of
+// whose weight gradients' error against float64 float32 here made up up to a third ([500, 68001] float32
+// dgamma 0.96e-7 -> 0.77e-7, [804, 16844] fp16 0.96e-7 -> 0.87e-7), at the same time: the rows are read
+// once either way.
 constexpr int kColReduceThreads = 256;
 
-template <int CW, int CX>
+template <int CW, int CX, typename SUM>
 __global__ void __launch_bounds__(kColReduceThreads)
 col_reduce(const float* __restrict__ part, float* __restrict__ out0, float* __restrict__ out1,
            int G, int W, int64_t part_stride, int64_t out_stride) {
@@ -1411,7 +1413,7 @@ col_reduce(const float* __restrict__ part, float* __restrict__ out0, float* __re
   const int W2 = 2 * W;
   const int col = (blockIdx.x * CX + cx) * CW;  // column in the concatenated [2W] row
   float acc[CW];
-  double sum[CW];
+  SUM sum[CW];
 #pragma unroll
   for (int i = 0; i < CW; ++i) sum[i] = 0;
   if (col < W2) {
@@ -1424,13 +1426,13 @@ col_reduce(const float* __restrict__ part, float* __restrict__ out0, float* __re
       load_f32<CW>(p + static_cast<int64_t>(g + 2 * CY) * W2, t2);
       load_f32<CW>(p + static_cast<int64_t>(g + 3 * CY) * W2, t3);
 #pragma unroll
-      for (int i = 0; i < CW; ++i) sum[i] += (double(t0[i]) + t1[i]) + (double(t2[i]) + t3[i]);
+      for (int i = 0; i < CW; ++i) sum[i] += (SUM(t0[i]) + SUM(t1[i])) + (SUM(t2[i]) + SUM(t3[i]));
     }
     for (; g < G; g += CY) {
       float t[CW];
       load_f32<CW>(p + static_cast<int64_t>(g) * W2, t);
 #pragma unroll
-      for (int i = 0; i < CW; ++i) sum[i] += t[i];
+      for (int i = 0; i < CW; ++i) sum[i] += SUM(t[i]);
     }
   }
 #pragma unroll

@@ -183,7 +183,7 @@ int long_rows_bwd_launch(const LongPlan& p, const ExchangeTag& tag, const T* dy,
                                         static_cast<int>(D), p.S, p.chunk_vec, p.groups,
                                         exchange_args(tag, tuning().long_rows_polls));
     ATEXN_CHECK_LAUNCH("long_rows_bwd");
-    return launch_col_reduce(part, dgamma, dbeta, p.part_rows, D, st);
+    return launch_col_reduce_double(part, dgamma, dbeta, p.part_rows, D, st);
   };
   const bool rg = D % V != 0;
   if (p.vpt == 1) return launch(rg ? long_rows_bwd<T, V, 1, true> : long_rows_bwd<T, V, 1, false>);
