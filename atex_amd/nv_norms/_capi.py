@@ -105,7 +105,7 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
-_host = None
+_host = None  # what torch_host() has returned, once it has been asked
 
 
 class _NoExtension:

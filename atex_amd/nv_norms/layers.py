@@ -89,8 +89,9 @@ class _FusedInstanceNormFn(torch.autograd.Function):
 def fused_layer_norm(x, gamma, beta, axis=(-1,), epsilon=0.001):
     """Differentiable fused_layer_norm_op: returns (y, mean, inv_std)."""
     axis = tuple(axis)
-    if x.is_cuda:
-        out = ops._capi.torch_host().layer_norm_apply(x, gamma, beta, axis, float(epsilon))
+    host = ops._capi._host or (x.is_cuda and ops._capi.torch_host())
+    if host:
+        out = host.layer_norm_apply(x, gamma, beta, axis, float(epsilon))
         if out is not None:
             return ops._checked(out)
     return _FusedLayerNormFn.apply(x, gamma, beta, axis, float(epsilon))
@@ -98,8 +99,9 @@ def fused_layer_norm(x, gamma, beta, axis=(-1,), epsilon=0.001):
 
 def fused_instance_norm(x, gamma, beta, data_format="N...C", epsilon=0.001):
     """Differentiable fused_instance_norm_op: returns (y, mean, inv_std)."""
-    if x.is_cuda:
-        out = ops._capi.torch_host().instance_norm_apply(x, gamma, beta, data_format, float(epsilon))
+    host = ops._capi._host or (x.is_cuda and ops._capi.torch_host())
+    if host:
+        out = host.instance_norm_apply(x, gamma, beta, data_format, float(epsilon))
         if out is not None:
             return ops._checked(out)
     return _FusedInstanceNormFn.apply(x, gamma, beta, data_format, float(epsilon))

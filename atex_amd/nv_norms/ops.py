@@ -113,8 +113,9 @@ def _checked(out):
 
 def fused_layer_norm_op(x: torch.Tensor, scale: torch.Tensor, offset: torch.Tensor,
                         axis: Sequence[int] = (-1,), epsilon: float = 0.001):
-    if x.is_cuda:
-        out = _capi.torch_host().layer_norm_fwd(x, scale, offset, axis, float(epsilon))
+    host = _capi._host or (x.is_cuda and _capi.torch_host())
+    if host:
+        out = host.layer_norm_fwd(x, scale, offset, axis, float(epsilon))
         if out is not None:
             return _checked(out)
     L = _capi.lib()
@@ -139,8 +140,9 @@ def fused_layer_norm_grad_op(y_backprop: torch.Tensor, x: torch.Tensor, scale: t
                              reserve_space_1: torch.Tensor, reserve_space_2: torch.Tensor,
                              axis: Sequence[int] = (-1,), epsilon: float = 0.001):
     del epsilon  # attr of the op, unused by the gradient math (norm_ops.cc:172)
-    if x.is_cuda:
-        out = _capi.torch_host().layer_norm_bwd(y_backprop, x, scale, reserve_space_1, reserve_space_2, axis)
+    host = _capi._host or (x.is_cuda and _capi.torch_host())
+    if host:
+        out = host.layer_norm_bwd(y_backprop, x, scale, reserve_space_1, reserve_space_2, axis)
         if out is not None:
             return _checked(out)
     L = _capi.lib()
@@ -169,8 +171,9 @@ def _fmt(data_format) -> bytes:
 
 def fused_instance_norm_op(x: torch.Tensor, scale: torch.Tensor, offset: torch.Tensor,
                            data_format: str = "N...C", epsilon: float = 0.001):
-    if x.is_cuda:
-        out = _capi.torch_host().instance_norm_fwd(x, scale, offset, data_format, float(epsilon))
+    host = _capi._host or (x.is_cuda and _capi.torch_host())
+    if host:
+        out = host.instance_norm_fwd(x, scale, offset, data_format, float(epsilon))
         if out is not None:
             return _checked(out)
     L = _capi.lib()
@@ -197,8 +200,9 @@ def fused_instance_norm_grad_op(y_backprop: torch.Tensor, x: torch.Tensor, scale
                                 reserve_space_1: torch.Tensor, reserve_space_2: torch.Tensor,
                                 data_format: str = "N...C", epsilon: float = 0.001):
     del epsilon
-    if x.is_cuda:
-        out = _capi.torch_host().instance_norm_bwd(y_backprop, x, scale, reserve_space_1, reserve_space_2, data_format)
+    host = _capi._host or (x.is_cuda and _capi.torch_host())
+    if host:
+        out = host.instance_norm_bwd(y_backprop, x, scale, reserve_space_1, reserve_space_2, data_format)
         if out is not None:
             return _checked(out)
     L = _capi.lib()
