@@ -75,7 +75,7 @@ OUTLIER_CASES = {
     "channels-last, C not a multiple of the vector, merge launch": ("cl", 2, 6, 50000),
     "channels-last, single pass": ("cl", 512, 32, 256),
     "channel-first, planes split over workgroups": ("cf", 1, 3, 1 << 19),
-    "LayerNorm tiles (rows too long for registers)": ("ln", 6, 1, 70001),
+    "LayerNorm rows over several workgroups": ("ln", 6, 1, 70001),
 }
 
 

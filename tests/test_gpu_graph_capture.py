@@ -17,6 +17,8 @@ EPS = 1e-3
 def test_graph_replay_matches_eager(case):
     import torch
 
+    # (ln_tiles and ln_accumulators_in_lds are named for the kernels that in-place calls of their sizes
+    # take, tests/test_gpu_in_place_rows.py runs them so; here both run long_rows_*)
     # (two cases through the benchmark build with the kernels that would take their shapes in
     # eager mode, but not under capture, switched off: eager and replay then run the same ones;
     # test_graph_capture_of_a_single_launch_shape covers what happens otherwise)

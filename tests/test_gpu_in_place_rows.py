@@ -52,7 +52,7 @@ def test_a_non_finite_row_stays_alone(capi, N, D, row, col):
 
 
 def test_outlier_samples_in_tiles(capi, coracle):
-    test_gpu_conditioning.test_outlier_samples(coracle, "LayerNorm tiles (rows too long for registers)", 1000.0)
+    test_gpu_conditioning.test_outlier_samples(coracle, "LayerNorm rows over several workgroups", 1000.0)
 
 
 @pytest.mark.parametrize("case", ["ln_tiles", "ln_accumulators_in_lds"])

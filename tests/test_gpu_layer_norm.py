@@ -134,9 +134,9 @@ def test_unaligned_pointers(capi, coracle, N, D, dtype):
 def test_backward_accumulators_in_lds(capi, coracle, N, D, dtype, in_place):
     """Rows of more than 2048 vectors whose dgamma / dbeta accumulators still fit a CU's LDS
     (up to 20416 elements: every 16-bit row from 16385 on, every float32 row from 8193 on)
-    take a single-pass backward with the accumulators in LDS; ragged row ends (an overlapping
-    last vector), a row count that is not a multiple of the workgroups, one row, the largest
-    row, and dx written over dy."""
+    take a single-pass backward with the accumulators in LDS where dx is written over dy; the others are
+    spread over several workgroups (tests/test_gpu_in_place_rows.py has such on the LDS kernel too).  Ragged row ends (an overlapping
+    last vector), a row count that is not a multiple of the workgroups, one row, the largest row."""
     run_case(capi, coracle, "plain", N, D, dtype, 19, in_place=in_place)
 
 

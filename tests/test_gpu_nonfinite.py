@@ -28,7 +28,7 @@ def _rows_equal(a, b, keep):
     (5000, 10, 17, 3),
     (33, 4096, 32, 5),       # wave groups (backward)
     (9, 12288, 4, 12287),    # one workgroup per row
-    (5, 70001, 2, 70000),    # 2-D tiles, the ragged tail element
+    (5, 70001, 2, 70000),    # several workgroups per row, the ragged tail element
     (5, 70001, 4, 8191),
 ])
 def test_layer_norm_row_isolation(N, D, row, col, bad):
