@@ -434,7 +434,7 @@ PyObject* norm_apply(PyObject*, PyObject* const* args, Py_ssize_t n) {
   at::Tensor x, gamma, beta;
   Attr a;
   if (n != 5 || !unobserved() || !PyFloat_CheckExact(args[4]) || !tensor_arg(args[0], x) || !tensor_arg(args[1], gamma) ||
-      !tensor_arg(args[2], beta) || !attr_arg<LAYER_NORM>(args[3], a)) {
+      !tensor_arg(args[2], beta) || !attr_arg<LAYER_NORM>(args[3], a) || !x.is_cuda()) {
     Py_RETURN_NONE;
   }
   // (forward-mode derivatives are not the node's business: the way round Python refuses them)

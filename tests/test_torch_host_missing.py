@@ -37,3 +37,13 @@ def test_a_missing_extension_declines_every_call(monkeypatch):
         host = _capi.torch_host()
     assert host.layer_norm_fwd(1, 2, 3) is None and host.instance_norm_apply() is None
     assert _capi.torch_host() is host  # warned once
+
+
+def test_host_tensors_beside_the_extension():
+    """Where it is loaded for other calls: it declines these before it leaves a trace in a profile."""
+    assert _capi.torch_host().__file__.endswith("_torch_host.so")
+    _calls()
+    x = torch.randn(6, 8)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as p:
+        nv_norms.fused_layer_norm(x, torch.ones(8), torch.zeros(8))
+    assert [e.name for e in p.events()].count("_FusedLayerNormFn") == 1
