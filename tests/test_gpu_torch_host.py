@@ -394,3 +394,22 @@ def test_a_compiled_model_breaks_its_graph_at_the_call(kind):
 
     for a, b in zip(step(model), step(torch.compile(model, backend="eager"))):
         assert torch.equal(a, b)
+
+
+def test_anomaly_mode_and_node_hooks():
+    import torch
+
+    x, gamma, beta, dy = _inputs("ln", torch.float32, grad=True)
+    diff = _ops("ln")[2]
+    seen = []
+    with torch.autograd.detect_anomaly(check_nan=True):
+        y = diff(x, gamma, beta)[0]
+        y.grad_fn.register_hook(lambda into, out: seen.append(len(into)))
+        want = torch.autograd.grad(y, [x, gamma, beta], dy, retain_graph=True)
+        bad = dy.clone()
+        bad.view(-1)[0] = float("nan")
+        with pytest.raises(RuntimeError, match="FusedLayerNormBackward.* returned nan"):
+            torch.autograd.grad(y, [x, gamma, beta], bad)
+    assert seen[0] == 3
+    for a, b in zip(want, torch.autograd.grad(diff(x, gamma, beta)[0], [x, gamma, beta], dy)):
+        assert torch.equal(a, b)
