@@ -1385,12 +1385,11 @@ rows_bwd_staged(const T* dy, const T* __restrict__ x, const float* __restrict__ 
 // Block of 256 threads = CX column groups of CW floats x (256 / CX) slices of g; a block
 // owns CX * CW adjacent columns of the concatenated [2W] row, so the grid has
 // 2W / (CX * CW) blocks (128 for W = 1024).  Slices are folded by a lane butterfly and a
-// 4-entry LDS step.  SUM: what a thread sums its slice in, up to G additions one after another.  float,
-// as the kernels do that fold the same sums themselves (a captured channel-first call, which ends in
-// a column reduction, has the bits of an eager one); double for the partial rows of long_rows_bwd, of
-// whose weight gradients' error against float64 float32 here made up up to a third ([500, 68001] float32
-// dgamma 0.96e-7 -> 0.77e-7, [804, 16844] fp16 0.96e-7 -> 0.87e-7), at the same time: the rows are read
-// once either way.
+// 4-entry LDS step.  SUM: what the sums are made in.  float, as the kernels do that fold the same sums
+// themselves (a captured channel-first call, which ends in a column reduction, has the bits of an
+// eager one); double for the partial rows of long_rows_bwd, of whose weight gradients' error against
+// float64 float32 here made up a fifth to a third ([500, 68001] float32 dgamma 0.96e-7 -> 0.76e-7,
+// [770, 5635] 0.98e-7 -> 0.61e-7, [804, 16844] fp16 0.96e-7 -> 0.69e-7), at the same time: the rows are read once either way.
 constexpr int kColReduceThreads = 256;
 
 template <int CW, int CX, typename SUM>
@@ -1407,15 +1406,14 @@ col_reduce(const float* __restrict__ part, float* __restrict__ out0, float* __re
   constexpr int CY = kColReduceThreads / CX;
   constexpr int NW = kColReduceThreads / kWave;
   constexpr int HOLD = CX < kWave ? NW : CY;  // partial sums per column group after the wave fold
-  __shared__ float buf[HOLD > 1 ? HOLD : 1][CX][CW];
+  __shared__ SUM buf[HOLD > 1 ? HOLD : 1][CX][CW];
   const int cx = threadIdx.x % CX;
   const int cy = threadIdx.x / CX;
   const int W2 = 2 * W;
   const int col = (blockIdx.x * CX + cx) * CW;  // column in the concatenated [2W] row
-  float acc[CW];
-  SUM sum[CW];
+  SUM acc[CW];
 #pragma unroll
-  for (int i = 0; i < CW; ++i) sum[i] = 0;
+  for (int i = 0; i < CW; ++i) acc[i] = 0;
   if (col < W2) {
     const float* p = part + col;
     int g = cy;
@@ -1426,23 +1424,21 @@ col_reduce(const float* __restrict__ part, float* __restrict__ out0, float* __re
       load_f32<CW>(p + static_cast<int64_t>(g + 2 * CY) * W2, t2);
       load_f32<CW>(p + static_cast<int64_t>(g + 3 * CY) * W2, t3);
 #pragma unroll
-      for (int i = 0; i < CW; ++i) sum[i] += (SUM(t0[i]) + SUM(t1[i])) + (SUM(t2[i]) + SUM(t3[i]));
+      for (int i = 0; i < CW; ++i) acc[i] += (SUM(t0[i]) + SUM(t1[i])) + (SUM(t2[i]) + SUM(t3[i]));
     }
     for (; g < G; g += CY) {
       float t[CW];
       load_f32<CW>(p + static_cast<int64_t>(g) * W2, t);
 #pragma unroll
-      for (int i = 0; i < CW; ++i) sum[i] += SUM(t[i]);
+      for (int i = 0; i < CW; ++i) acc[i] += SUM(t[i]);
     }
   }
-#pragma unroll
-  for (int i = 0; i < CW; ++i) acc[i] = static_cast<float>(sum[i]);
   if constexpr (CX < kWave) {
     // lanes l, l + CX, ... of a wave hold slices of the same columns
 #pragma unroll
     for (int i = 0; i < CW; ++i) {
 #pragma unroll
-      for (int m = CX; m < kWave; m <<= 1) acc[i] += lane_xor(acc[i], m);
+      for (int m = CX; m < kWave; m <<= 1) acc[i] += __shfl_xor(acc[i], m, kWave);
     }
   }
   if constexpr (HOLD > 1) {
@@ -1456,7 +1452,7 @@ col_reduce(const float* __restrict__ part, float* __restrict__ out0, float* __re
     if (threadIdx.x < CX) {
 #pragma unroll
       for (int i = 0; i < CW; ++i) {
-        float s = buf[0][cx][i];
+        SUM s = buf[0][cx][i];
 #pragma unroll
         for (int k = 1; k < HOLD; ++k) s += buf[k][cx][i];
         acc[i] = s;
@@ -1469,9 +1465,9 @@ col_reduce(const float* __restrict__ part, float* __restrict__ out0, float* __re
       // CW divides W on the vector path, so a column group never straddles the two halves
       const int j = col + i;
       if (j < W) {
-        out0[j] = acc[i];
+        out0[j] = static_cast<float>(acc[i]);
       } else if (j < W2) {
-        out1[j - W] = acc[i];
+        out1[j - W] = static_cast<float>(acc[i]);
       }
     }
   }

@@ -98,7 +98,7 @@ int fill_zero(float* out, int64_t n, hipStream_t st);
 int launch_col_reduce(const float* part, float* out0, float* out1, int G, int64_t W,
                       hipStream_t st, int batch = 1, int64_t part_stride = 0,
                       int64_t out_stride = 0);
-// The same, each thread's share of the G rows summed in double.
+// The same, summed in double.
 int launch_col_reduce_double(const float* part, float* out0, float* out1, int G, int64_t W, hipStream_t st);
 
 inline int elem_size(int dtype) { return dtype == ATEXN_F32 ? 4 : 2; }
