@@ -45,6 +45,9 @@ SOURCES = [
     "rows_launch_f16.hip",
     "rows_launch_bf16.hip",
     "cl_launch.hip",
+    "cl_flat_launch_f32.hip",
+    "cl_flat_launch_f16.hip",
+    "cl_flat_launch_bf16.hip",
     "cpu_kernels.cc",
 ]
 

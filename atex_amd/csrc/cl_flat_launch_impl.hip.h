@@ -1,0 +1,108 @@
+// Launchers of the flat channels-last kernels, templated on the storage type.
+#pragma once
+
+#include "cl_flat_kernels.hip.h"
+#include "plan.h"
+#include "status.h"
+
+namespace atexn {
+
+static_assert(kPlanFlatMaxSlabs == kFlatMaxSlabs && kPlanFlatMaxThreads == kFlatMaxThreads,
+              "the planner and the flat kernels must agree on their limits");
+
+inline FlatArgs flat_args(const FlatPlan& p, int64_t N, int64_t C, int64_t D, void* ws, const ExchangeTag& e) {
+  char* w = static_cast<char*>(ws);
+  FlatArgs a;
+  a.N = N;
+  a.D = D;
+  a.E = D * C;
+  a.C = static_cast<int>(C);
+  a.P = p.P;
+  a.A = p.A;
+  a.S = p.S;
+  a.base = p.base;
+  a.extra = p.extra;
+  a.pix = p.pix;
+  a.width = std::min(64, pow2_ceil(p.S));
+  a.inv_d = 1.0f / static_cast<float>(D);
+  a.px_base = static_cast<float>(int64_t(p.base) * p.pix);
+  a.px_more = static_cast<float>((int64_t(p.base) + 1) * p.pix);
+  a.px_last = static_cast<float>(D - (int64_t(p.S - 1) * p.base + p.extra) * p.pix);
+  a.local = p.local;
+  a.k_at = p.k_at;
+  a.ex = ExchangeArgs{e.tag, e.at, tuning().cl_flat_polls, e.trouble};
+  a.tagged = reinterpret_cast<cl_word*>(w + p.off_tagged);
+  a.finals = reinterpret_cast<cl_word*>(w + p.off_finals);
+  a.claims = reinterpret_cast<unsigned*>(w + p.off_claims);
+  return a;
+}
+
+// Launches the call's kernel unless its workgroups may not exchange results (taken: it did).
+template <typename T, int V>
+int flat_fwd_v(const FlatPlan& p, const T* x, const float* gamma, const float* beta, int64_t N, int64_t C, int64_t D,
+               float eps, T* y, float* mean, float* rstd, void* ws, hipStream_t st, bool& taken) {
+  ExchangeTag e;
+  e.ok = true;
+  if (p.S > 1) ATEXN_TRY(exchange_tag(st, static_cast<char*>(ws) + p.off_tag, e));
+  taken = e.ok;
+  if (!taken) return ATEXN_OK;
+  const FlatArgs a = flat_args(p, N, C, D, ws, e);
+  const unsigned grid = static_cast<unsigned>(p.grid);
+#define ATEXN_FLAT_FWD(U_) \
+  case U_: cl_flat_fwd<T, V, U_><<<grid, p.threads, p.lds, st>>>(x, gamma, beta, y, mean, rstd, a, eps); break
+  switch (p.U) {
+    ATEXN_FLAT_FWD(1);
+    ATEXN_FLAT_FWD(2);
+    ATEXN_FLAT_FWD(3);
+    ATEXN_FLAT_FWD(4);
+    ATEXN_FLAT_FWD(6);
+    ATEXN_FLAT_FWD(8);
+    ATEXN_FLAT_FWD(12);
+    ATEXN_FLAT_FWD(16);
+    default: return set_error(ATEXN_INVALID_ARGUMENT, "no kernel for %d vectors per thread", p.U);
+  }
+#undef ATEXN_FLAT_FWD
+  ATEXN_CHECK_LAUNCH("cl_flat_fwd");
+  return ATEXN_OK;
+}
+
+template <typename T, int V>
+int flat_bwd_v(const FlatPlan& p, const T* dy, const T* x, const float* gamma, const float* mean, const float* rstd,
+               int64_t N, int64_t C, int64_t D, T* dx, float* dgamma, float* dbeta, void* ws, hipStream_t st,
+               bool& taken) {
+  ExchangeTag e;
+  e.ok = true;
+  if (p.S > 1) ATEXN_TRY(exchange_tag(st, static_cast<char*>(ws) + p.off_tag, e));
+  taken = e.ok;
+  if (!taken) return ATEXN_OK;
+  const FlatArgs a = flat_args(p, N, C, D, ws, e);
+  const unsigned grid = static_cast<unsigned>(p.grid);
+  float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + p.off_part);
+  float* o0 = N == 1 ? dgamma : part;
+  float* o1 = N == 1 ? dbeta : part + C;
+#define ATEXN_FLAT_BWD(U_) \
+  case U_: cl_flat_bwd<T, V, U_><<<grid, p.threads, p.lds, st>>>(dy, x, gamma, mean, rstd, dx, o0, o1, 2 * C, a); break
+  switch (p.U) {
+    ATEXN_FLAT_BWD(1);
+    ATEXN_FLAT_BWD(2);
+    ATEXN_FLAT_BWD(3);
+    ATEXN_FLAT_BWD(4);
+    ATEXN_FLAT_BWD(6);
+    ATEXN_FLAT_BWD(8);
+    default: return set_error(ATEXN_INVALID_ARGUMENT, "no kernel for %d vectors per thread", p.U);
+  }
+#undef ATEXN_FLAT_BWD
+  ATEXN_CHECK_LAUNCH("cl_flat_bwd");
+  if (N > 1) return launch_col_reduce(part, dgamma, dbeta, static_cast<int>(N), C, st);
+  return ATEXN_OK;
+}
+
+#define ATEXN_INSTANTIATE_FLAT(T)                                                                                \
+  template int flat_fwd_v<T, VecOf<T>::value>(const FlatPlan&, const T*, const float*, const float*, int64_t,    \
+                                              int64_t, int64_t, float, T*, float*, float*, void*, hipStream_t,   \
+                                              bool&);                                                            \
+  template int flat_bwd_v<T, VecOf<T>::value>(const FlatPlan&, const T*, const T*, const float*, const float*,   \
+                                              const float*, int64_t, int64_t, int64_t, T*, float*, float*,       \
+                                              void*, hipStream_t, bool&);
+
+}  // namespace atexn

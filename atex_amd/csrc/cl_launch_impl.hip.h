@@ -14,6 +14,14 @@ static_assert(kPlanClSingleMaxCap == kClSingleMaxCap && kPlanClSingleMaxSlabs ==
 
 static_assert(kPlanClFoldRegs == 2 * kClFoldRegs, "the planner and the kernels must agree on the fold's register limit");
 
+// cl_flat_launch_impl.hip.h
+template <typename T, int V>
+int flat_fwd_v(const FlatPlan&, const T*, const float*, const float*, int64_t, int64_t, int64_t, float, T*, float*,
+               float*, void*, hipStream_t, bool&);
+template <typename T, int V>
+int flat_bwd_v(const FlatPlan&, const T*, const T*, const float*, const float*, const float*, int64_t, int64_t,
+               int64_t, T*, float*, float*, void*, hipStream_t, bool&);
+
 // Whether every register-resident slab of the plan holds exactly U pixels per pixel slot and
 // every channel tile is complete (the kernels' FULL instantiations: no lane is ever masked).
 inline bool cl_slabs_full(const ClPlan& p, int64_t C, int64_t D) {
@@ -58,6 +66,11 @@ int cl_fwd_v(const T* x, const float* gamma, const float* beta, int64_t N, int64
     ATEXN_CHECK_LAUNCH("cl_fwd_apply");                                                       \
   } while (0)
   if constexpr (V > 1) {
+    if (p.flat.on && static_cast<const void*>(y) != static_cast<const void*>(x)) {
+      bool taken = false;
+      ATEXN_TRY((flat_fwd_v<T, V>(p.flat, x, gamma, beta, N, C, D, eps, y, mean, rstd, ws, st, taken)));
+      if (taken) return ATEXN_OK;
+    }
     if (p.fused) {
       const dim3 fgrid(static_cast<unsigned>(N), 1, p.CT);
 #define ATEXN_CL_FWD_FUSED(U_)                                                                 \
@@ -176,6 +189,11 @@ int cl_bwd_v(const T* dy, const T* x, const float* gamma, const float* mean, con
     ATEXN_CHECK_LAUNCH("cl_bwd_apply");                                                       \
   } while (0)
   if constexpr (V > 1) {
+    if (p.flat.on && static_cast<const void*>(dx) != static_cast<const void*>(dy)) {
+      bool taken = false;
+      ATEXN_TRY((flat_bwd_v<T, V>(p.flat, dy, x, gamma, mean, rstd, N, C, D, dx, dgamma, dbeta, ws, st, taken)));
+      if (taken) return ATEXN_OK;
+    }
     if (p.fused) {
       const dim3 fgrid(static_cast<unsigned>(N), 1, p.CT);
       // a single instance: its sums are dgamma / dbeta; else per-instance rows for col_reduce

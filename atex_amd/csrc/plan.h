@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <atomic>
 #include <climits>
+#include <cmath>
 
 namespace atexn {
 
@@ -65,6 +66,8 @@ struct Tuning {
   TuneInt cl_single_xm{1};  //   also on the XCD-major grid (any batch size, any number of workgroups)
   TuneInt cl_single_occ{1};  //   on that grid, when the launch does not fit the chip: the kernels compiled for more workgroups per CU
   TuneInt cl_single_polls{300};
+  TuneInt cl_flat{1};          // channels-last, flat instances (cl_flat_kernels.hip.h); 2: wherever they can
+  TuneInt cl_flat_polls{300};  //   their polls
   TuneInt affine_fold{1};      // channel-first backward, a workgroup per plane: dgamma / dbeta folded over the batch in the row kernel
   TuneInt affine_fold_polls{2000};  //   polls before a workgroup recomputes its peers' plane sums (0: at once)
   // channel-first planes too long for a workgroup: the chunks of a plane on the workgroups of one
@@ -636,6 +639,89 @@ inline TilePlan plan_tiles(bool bwd, int V, int64_t n_rows, int64_t D, int cus) 
   return p;
 }
 
+// Channels-last instances as flat arrays, one launch per direction (cl_flat_kernels.hip.h).
+struct FlatPlan {
+  bool on = false;
+  int U = 0, threads = 0, P = 0, A = 0, S = 1, base = 0, extra = 0, pix = 1, local = 0, k_at = 0;
+  int64_t grid = 0;
+  size_t lds = 0, off_tagged = 0, off_finals = 0, off_claims = 0, off_part = 0, off_tag = 0, ws_bytes = 0;
+};
+constexpr int kPlanFlatMaxSlabs = 512, kPlanFlatMaxThreads = 512, kPlanFlatMaxChannels = 2048;
+constexpr int kPlanFlatUs[] = {16, 12, 8, 6, 4, 3, 2, 1};  // vectors per thread that have a kernel (backward: up to 8)
+
+// The plan with U vectors per thread on `threads` threads and S slabs per instance, if there is one: the
+// slabs get the instance's periods evenly, and every step of a slab but its last must be whole.
+inline FlatPlan plan_flat_as(bool bwd, int V, int64_t N, int64_t C, int64_t D, int U, int threads, int64_t S, bool local) {
+  FlatPlan p;
+  int64_t g = V;
+  while (C % g != 0) g /= 2;
+  const int64_t P = C / g, pix = V / g;
+  const int64_t m = threads / P, periods = div_up(D, pix);
+  if (m < 1 || S < 1 || S > kPlanFlatMaxSlabs || S > periods) return p;
+  const int64_t base = periods / S, extra = periods % S;
+  const int64_t last_px = D - (periods - base) * pix;  // the last slab has the fewest pixels
+  if (base + (extra > 0 ? 1 : 0) > U * m || last_px < 1 || last_px < (U - 1) * m * pix) return p;
+  p.U = U;
+  p.threads = threads;
+  p.P = static_cast<int>(P);
+  p.A = static_cast<int>(m * P);
+  p.pix = static_cast<int>(pix);
+  p.S = static_cast<int>(S);
+  p.base = static_cast<int>(base);
+  p.extra = static_cast<int>(extra);
+  p.local = local ? 1 : 0;
+  p.grid = (local ? round_up(N, kPlanXcdCount) : N) * S;
+  if (p.grid >= (int64_t(1) << 31) / threads) return p;
+  // LDS: the threads' sums, the threads' shares of the channels', the channels' parameters
+  const int64_t sums = 2 * int64_t(p.A) * V + 2 * std::max<int64_t>(threads, C);
+  p.k_at = static_cast<int>(sums);
+  p.lds = sizeof(float) * size_t(sums + (bwd ? 4 : 3) * C);
+  if (p.lds > 65000) return p;
+  p.off_finals = S > 1 ? align256(size_t(16) * size_t(N) * size_t(S) * size_t(C)) : 0;
+  p.off_claims = p.off_finals + (S > 1 ? align256(size_t(16) * size_t(N) * size_t(C)) : 0);
+  p.off_part = p.off_claims + (S > 1 ? align256(size_t(4) * size_t(N) * size_t(S)) : 0);
+  p.off_tag = p.off_part + (bwd && N > 1 ? align256(sizeof(float) * 2 * size_t(N) * size_t(C)) : 0);
+  p.ws_bytes = p.off_tag + 256;
+  p.on = true;
+  return p;
+}
+
+// The flat kernels' plan, whether or not they are the better ones.
+//
+// Threads: 256 unless 512 leave clearly fewer lanes without a vector (C = 137: 274 of 512 or 137 of 256).
+// (384 threads, six waves, do not pack the SIMDs: launches that should have fitted the chip did not.)
+// Vectors per thread: as many as leave the chip three quarters of a wave per SIMD of 256 threads.  Slabs
+// are held at 128 registers, four waves per SIMD, and a launch costs most where its workgroups come in
+// more than one round (fp16 [59, 16896, 17] forward with 8 / 12 / 16 vectors, 1152 / 767 / 590 workgroups:
+// 18.8 / 17.2 / 18.1 us; [17, 30940, 57] bf16 41 / 38.7 / 29.5), and every slab is C pairs to exchange.
+// Instances stay on one XCD each where that keeps the XCDs busy alike: a hop through its L2 costs 1 to 2 us
+// less than one through memory ([38, 3328, 85] fp16 14.1 against 17.8 us).
+inline FlatPlan plan_flat(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+  FlatPlan p;
+  if (V == 1 || C > kPlanFlatMaxChannels || D * C >= (int64_t(1) << 31) || cus < kPlanXcdCount) return p;
+  int64_t g = V;
+  while (C % g != 0) g /= 2;
+  const int64_t P = C / g, pix = V / g, periods = div_up(D, pix);
+  if (P > kPlanFlatMaxThreads) return p;
+  const bool wide = P > 256 || 256 / P * 8 < 512 / P * 3;
+  const int threads = wide ? 512 : 256;
+  const int64_t m = threads / P;
+  const int64_t slots = int64_t(cus) * (1024 / threads);
+  const bool near = N >= kPlanXcdCount ? round_up(N, kPlanXcdCount) * 2 <= N * 3 : N * C * D * 16 / V <= (int64_t(5) << 20);
+  for (const bool local : {near, !near}) {
+    const int64_t fit = (local ? slots / kPlanXcdCount : slots) * 15 / 16;  // an instance's slabs are on the chip together
+    for (const int U : kPlanFlatUs) {
+      if (bwd && U > 8) continue;
+      const int64_t S = div_up(periods, U * m);
+      if (S > fit || (p.on && N * p.S * threads >= int64_t(cus) * 192)) break;
+      const FlatPlan q = plan_flat_as(bwd, V, N, C, D, U, threads, S, local);
+      if (q.on) p = q;
+    }
+    if (p.on) return p;
+  }
+  return p;
+}
+
 // Channels-last InstanceNorm, x as [N, D, C].
 struct ClPlan {
   int V = 1;
@@ -678,6 +764,7 @@ struct ClPlan {
   // other grid
   bool xm_fold = false;
   bool xm_resident = false;  // every workgroup of the XCD-major grid on the chip at once
+  FlatPlan flat;  // instead of all of the above, except in place
 };
 constexpr int kClFoldAbove = 64;
 constexpr int kPlanClSingleMaxCap = 64, kPlanClSingleMaxSlabs = 64, kPlanClSingleMaxOwned = 4;
@@ -840,7 +927,7 @@ inline ClPlan plan_cl_with(bool bwd, int V, int64_t N, int64_t C, int64_t D, int
   return p;
 }
 
-inline ClPlan plan_cl(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+inline ClPlan plan_cl_slabs(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
   const ClPlan p = plan_cl_with(bwd, V, N, C, D, cus, 0);
   const Tuning& t = tuning();
   if (p.single || p.fused || !t.cl_single || !t.cl_single_xm || V == 1) return p;
@@ -854,6 +941,48 @@ inline ClPlan plan_cl(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus)
   if (s_x < 2 || s_x > kPlanClSingleMaxSlabs) return p;
   const ClPlan q = plan_cl_with(bwd, V, N, C, D, cus, s_x);
   return q.single ? q : p;
+}
+
+// Whether the flat kernels take a call that would otherwise run plan p: the classes of drawn shapes where
+// they were faster (us of the old kernels against theirs).
+// 16-bit pixels that are no whole number of vectors, which the other kernels read in overlapping pieces and
+// twice.  Forward from 2 MB of x ([22, 14280, 17] fp16 20.1 -> 11.2, [51, 7684, 87] bf16 49.1 -> 32.3,
+// [28, 1275, 162] 16.2 -> 13.5; [48, 304, 74], 2.2 MB with few pixels, 7.5 -> 9.0); over all XCDs from 5 MB and
+// while the pairs that are exchanged are few ([1, 598464, 17] 31.1 -> 20.2, [2, 85000, 133] 37.4 -> 32.4;
+// [4, 1664, 428] 14.4 -> 17.1, [3, 14016, 428] 31.0 -> 41.0, [5, 75264, 116] 48 -> 53).  Backward, which holds half as much and leaves
+// the fold over the instances to a launch, from 7 MB on one XCD each ([24, 9384, 57] 28.8 -> 20.4,
+// [36, 36288, 29] 104 -> 61; [50, 1248, 53], 6.6 MB, 13.3 -> 13.6), not where a few workgroups are left for
+// another round or there are several rounds of many channels ([20, 2920, 175] 26.8 -> 30.0, [11, 7104, 190]
+// 33.0 -> 39.5).
+// Other pixels: forward in place of two stages from 20 MB ([28, 92880, 16] 47.3 -> 34.3, f32
+// [15, 5488, 104] 24.7 -> 17.5; [12, 3408, 448] 27.9 -> 29.2, [11, 20592, 128] 35.6 -> 37.9); and where even
+// the kernels of resident slabs need several rounds, both ways ([33, 23808, 64] bf16 55.9 / 89.1 ->
+// 39.2 / 77.3, [36, 30000, 32] 35.9 / 58.0 -> 26.9 / 50.2; [32, 6976, 64] 15.0 -> 15.1).
+inline bool flat_instead(const ClPlan& p, const FlatPlan& f, bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+  if (!f.on || p.fused || f.S < 2) return false;
+  if (int64_t(f.S) * 32 > D) return false;  // a slab's pairs: more than a sixteenth (f32: an eighth) of its bytes
+  const int64_t x2 = N * C * D / (V / 2) >> 16;  // MiB of x, times two
+  const int64_t slots = int64_t(cus) * (1024 / f.threads);
+  if (C % V != 0 && V == 8) {
+    if (bwd) return f.local && x2 >= 14 && (f.grid <= slots || C <= 64 || (C <= 160 && f.grid * 20 > slots * 23));
+    if (f.local) return N >= kPlanXcdCount && x2 >= 4;
+    return x2 >= 10 && (f.grid <= slots ? C <= 300 : C <= 80 && f.grid <= slots * 2);
+  }
+  if (!f.local || C > 128 || (f.grid > slots && f.grid * 2 < slots * 3)) return false;
+  if (!bwd && !p.single) return x2 >= 40;
+  return V == 8 && p.single && C <= 64 && x2 >= 96;
+}
+
+inline ClPlan plan_cl(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+  ClPlan p = plan_cl_slabs(bwd, V, N, C, D, cus);
+  const int how = tuning().cl_flat;
+  if (how == 0 || (how == 1 && (p.fused || N * C * D < (int64_t(1) << 19)))) return p;  // (flat_instead wants more)
+  const FlatPlan f = plan_flat(bwd, V, N, C, D, cus);
+  if (how == 2 ? f.on : flat_instead(p, f, bwd, V, N, C, D, cus)) {
+    p.flat = f;
+    p.ws_bytes = std::max(p.ws_bytes, f.ws_bytes);
+  }
+  return p;
 }
 
 }  // namespace atexn

@@ -1,0 +1,85 @@
+// Host-only check of the plans of the flat channels-last kernels (atex_amd/csrc/plan.h): what the kernels
+// assume of them, and that threads, steps and slabs cover every element of an instance once.  Built and run
+// by tests/test_flat_plans.py.  "ok <plans> <with several slabs>" on success.
+#include <cstdio>
+#include <vector>
+
+#include "plan.h"
+
+namespace atexn {
+static Tuning g_tuning;
+const Tuning& tuning() { return g_tuning; }
+}  // namespace atexn
+using namespace atexn;
+
+static long g_plans = 0, g_split = 0, g_failed = 0;
+#define EXPECT(cond)                                                                                              \
+  do {                                                                                                            \
+    if (!(cond) && ++g_failed < 50)                                                                               \
+      std::printf("FAIL %s: bwd=%d V=%d N=%lld C=%lld D=%lld cus=%d U=%d threads=%d S=%d\n", #cond, int(bwd), V,  \
+                  (long long)N, (long long)C, (long long)D, cus, p.U, p.threads, p.S);                            \
+  } while (0)
+
+static void check(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+  const FlatPlan p = plan_flat(bwd, V, N, C, D, cus);
+  if (!p.on) return;
+  ++g_plans;
+  if (p.S > 1) ++g_split;
+  EXPECT(p.threads == 256 || p.threads == 512);
+  EXPECT(p.A <= p.threads && p.A % p.P == 0 && int64_t(p.P) * V == C * p.pix && V % p.pix == 0);
+  bool built = false;
+  for (const int u : kPlanFlatUs) built = built || (p.U == u && (u <= 8 || !bwd));
+  EXPECT(built);
+  // the slabs are the instance's periods; every step of every slab but the last is whole
+  const int64_t E = D * C, step = int64_t(p.A) * V;
+  int64_t at = 0, least = E;
+  for (int s = 0; s < p.S; ++s) {
+    const int64_t p0 = int64_t(s) * p.base + std::min(s, p.extra), k = p.base + (s < p.extra ? 1 : 0);
+    const int64_t px0 = p0 * p.pix, px1 = std::min(px0 + k * p.pix, D);
+    EXPECT(px0 * C == at && px1 > px0);
+    const int64_t n = (px1 - px0) * C;
+    EXPECT(n <= p.U * step && n >= (p.U - 1) * step && n < (int64_t(1) << 24));
+    // pixel counts as the fold takes them
+    const int64_t said = s == p.S - 1 ? D - (int64_t(p.S - 1) * p.base + p.extra) * p.pix
+                                      : (int64_t(p.base) + (s < p.extra ? 1 : 0)) * p.pix;
+    EXPECT(said == px1 - px0);
+    at += n;
+    least = std::min(least, n);
+  }
+  EXPECT(at == E && least > 0);
+  // an instance's slabs are on the chip (the XCD) together; 32-bit positions in its pairs
+  const int64_t slots = int64_t(cus) * (1024 / p.threads);
+  EXPECT(p.S <= (p.local ? slots / 8 : slots) && 4 * int64_t(p.S) * C < (int64_t(1) << 32));
+  EXPECT(p.grid == (p.local ? round_up(N, 8) : N) * p.S && p.grid * p.threads < (int64_t(1) << 32));
+  EXPECT(size_t(p.k_at) >= 2 * size_t(step) + 2 * size_t(std::max<int64_t>(p.threads, C)));
+  EXPECT(p.lds >= sizeof(float) * (size_t(p.k_at) + size_t(bwd ? 4 : 3) * size_t(C)) && p.lds + 2048 <= 65536 + 1536);
+  const size_t pairs = p.S > 1 ? size_t(16) * N * p.S * C : 0, finals = p.S > 1 ? size_t(16) * N * C : 0;
+  EXPECT(p.off_tagged == 0 && p.off_finals >= pairs && p.off_claims >= p.off_finals + finals);
+  EXPECT(p.off_part >= p.off_claims + (p.S > 1 ? size_t(4) * N * p.S : 0));
+  EXPECT(p.off_tag >= p.off_part + (bwd && N > 1 ? size_t(8) * N * C : 0) && p.ws_bytes >= p.off_tag + 4);
+  EXPECT(p.off_finals % 16 == 0 && p.off_claims % 16 == 0 && p.off_part % 16 == 0 && p.off_tag % 4 == 0);
+  // the call's plan has room for it and for the kernels that serve y == x
+  const ClPlan c = plan_cl(bwd, V, N, C, D, cus);
+  EXPECT(!c.flat.on || (c.ws_bytes >= c.flat.ws_bytes && c.ws_bytes >= plan_cl_slabs(bwd, V, N, C, D, cus).ws_bytes));
+}
+
+int main() {
+  std::vector<int64_t> channels;
+  for (int64_t c = 4; c <= 80; ++c) channels.push_back(c);
+  for (int64_t c = 81; c <= 2100; c += c < 600 ? 5 : 61) channels.push_back(c);
+  for (const int64_t c : {127, 128, 129, 255, 256, 257, 511, 512, 513, 1024, 2047, 2048, 2049, 4096}) channels.push_back(c);
+  const int64_t pixels[] = {1, 2, 7, 8, 9, 31, 100, 441, 1000, 2047, 4096, 5917, 16384, 30940, 100003, 268800, 1000000, 2097152, 6782976};
+  const int64_t batches[] = {1, 2, 3, 7, 8, 9, 13, 17, 24, 59, 64, 300, 5000};
+  for (const int64_t C : channels)
+    for (const int64_t D : pixels)
+      for (const int64_t N : batches)
+        for (const int cus : {256, 304, 64, 8, 7})
+          for (const int V : {8, 4}) {
+            if (C < V) continue;
+            check(false, V, N, C, D, cus);
+            check(true, V, N, C, D, cus);
+          }
+  if (g_failed) return 1;
+  std::printf("ok %ld %ld\n", g_plans, g_split);
+  return 0;
+}
