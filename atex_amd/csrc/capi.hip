@@ -144,7 +144,7 @@ int atexn_abi_version(void) { return kAbiVersion; }
 int atexn_set_tuning(const char* name, int value) {
   ATEXN_REQUIRE(name != nullptr && value >= 0, "bad tuning request");
   ATEXN_REQUIRE(value >= 1 || !strcmp(name, "reverse_second_pass") || !strcmp(name, "cl_fused") ||
-                    !strcmp(name, "cl_fold_cap") || !strcmp(name, "cl_single") || !strcmp(name, "affine_fold") || !strcmp(name, "affine_fold_polls") || !strcmp(name, "cl_single_polls") || !strcmp(name, "cl_single_xm") || !strcmp(name, "cl_single_occ") || !strcmp(name, "plane_single") || !strcmp(name, "plane_single_occ") || !strcmp(name, "plane_single_polls") || !strcmp(name, "bwd_lds_rows") || !strcmp(name, "staged_rows") || !strcmp(name, "cl_narrow_tiles") || !strcmp(name, "cl_fused_split") || !strcmp(name, "long_rows") || !strcmp(name, "long_rows_polls") || !strcmp(name, "cl_flat") || !strcmp(name, "cl_flat_polls"),
+                    !strcmp(name, "cl_fold_cap") || !strcmp(name, "cl_single") || !strcmp(name, "affine_fold") || !strcmp(name, "affine_fold_polls") || !strcmp(name, "cl_single_polls") || !strcmp(name, "cl_single_xm") || !strcmp(name, "cl_single_occ") || !strcmp(name, "plane_single") || !strcmp(name, "plane_single_occ") || !strcmp(name, "plane_single_polls") || !strcmp(name, "bwd_lds_rows") || !strcmp(name, "staged_rows") || !strcmp(name, "cl_narrow_tiles") || !strcmp(name, "cl_fused_split") || !strcmp(name, "long_rows") || !strcmp(name, "long_rows_polls") || !strcmp(name, "pair_rows") || !strcmp(name, "cl_flat") || !strcmp(name, "cl_flat_polls"),
                 "value must be >= 1");
   Tuning& t = tuning();
   if (!strcmp(name, "fwd_waves_per_cu")) t.fwd_waves_per_cu = value;
@@ -214,6 +214,9 @@ int atexn_set_tuning(const char* name, int value) {
   } else if (!strcmp(name, "plane_single_occ")) {
     ATEXN_REQUIRE(value == 0 || value == 1, "plane_single_occ must be 0 or 1");
     t.plane_single_occ = value;
+  } else if (!strcmp(name, "pair_rows")) {
+    ATEXN_REQUIRE(value >= 0 && value <= 2, "pair_rows must be 0, 1 or 2");
+    t.pair_rows = value;
   } else if (!strcmp(name, "long_rows")) {
     ATEXN_REQUIRE(value == 0 || value == 1, "long_rows must be 0 or 1");
     t.long_rows = value;
@@ -287,6 +290,10 @@ int atexn_bench_describe_bwd(int op, int dtype, int layout, int64_t N, int64_t C
       else
         n = snprintf(out, out_bytes, "tile_bwd_sums + merge_row_sums + tile_bwd_apply%s; alone=0",
                      p.sums_RS > 1 ? " + col_reduce" : "");
+    } else if (!affine && plan_pair(r.V, rows, D).on) {
+      const PairPlan p = plan_pair(r.V, rows, D);
+      n = snprintf(out, out_bytes, "rows_bwd_pair (%d workgroups of rows, %d lanes x %d vectors each; %d of columns; the row kernels when dx == dy); alone=0",
+                   p.row_blocks, p.tpr, p.vpt, p.grid - p.row_blocks);
     } else {
       const RowsPlan p = plan_rows(kind, r.V, rows, D, affine ? static_cast<int>(C) : 0, cus);
       const char* k = p.acc_lds ? "rows_bwd_lds" : p.staged ? "rows_bwd_staged" : p.resident ? "rows_bwd_resident" : "";

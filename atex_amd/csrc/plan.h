@@ -76,6 +76,7 @@ struct Tuning {
   TuneInt plane_single_polls{500};
   // 1: plane_bwd_single built for three workgroups per CU when a plane has more than 32 chunks
   TuneInt plane_single_occ{1};
+  TuneInt pair_rows{1};           // LayerNorm backward of few rows in one launch (pair_rows_kernels.hip.h); 2: wherever it can
   TuneInt long_rows{1};           // LayerNorm rows beyond one workgroup: one launch, one pass (long_rows_kernels.hip.h)
   TuneInt long_rows_polls{500};   //   and its polls
   TuneInt plane_nt_min_mb{256};  // forward: non-temporal loads of x from this many MiB (what no cache level retains anyway)
@@ -209,6 +210,38 @@ inline bool long_rows_instead(int V, int64_t n_rows, int64_t D, int cus) {
   const int64_t n_vec = div_up(D, V);
   if (V == 8) return n_vec > 1536 && n_rows < int64_t(20) * cus;
   return n_vec > 2048 || (n_vec > 1408 && n_rows >= int64_t(3) * cus);
+}
+
+// LayerNorm backward of few rows, dx and dgamma / dbeta by workgroups of their own in one launch
+// (pair_rows_kernels.hip.h).
+struct PairPlan {
+  bool on = false;
+  int tpr = 0, vpt = 0;  // lanes of a row (64 or 512), vectors per lane (1, 2 or 4)
+  int strip = 4;         // vectors of a column workgroup (4 or 8)
+  int row_blocks = 0, grid = 0;
+};
+// How many rows: the second read of x and dy against the partial rows of the row kernels and the launch
+// that folds them (us, row kernels -> this).  Up to 512: fp16 [32, 1024] 7.7 -> 4.9, [128, 10501] 20.1 ->
+// 8.4, [256, 13845] 22.2 -> 11.0, [512, 4096] 11.4 -> 10.4, float32 [512, 1024] 8.3 -> 8.1, [512, 7575] 22.0 ->
+// 21.0; more where a row of 16-bit data is long ([768, 10501] 31.0 -> 23.6; [768, 4096] 12.5 -> 12.9, float32
+// [768, 7575] 25.3 -> 30.2) or so short that the launches are all there is ([1024, 256] 8.9 -> 8.1;
+// [1024, 1024] 8.6 -> 10.1).  Strips of 8 vectors, whole cache lines, where that leaves enough workgroups:
+// [256, 10501] 13.5 -> 9.8.
+inline PairPlan plan_pair(int V, int64_t n_rows, int64_t D) {
+  PairPlan p;
+  const int how = tuning().pair_rows;
+  const int64_t n_vec = div_up(D, V);
+  if (how == 0 || V == 1 || D < V || n_vec > 2048) return p;
+  if (!tuning().long_rows && n_vec > 1536) return p;  // (a switch: such rows on the kernels that serve dx == dy)
+  const int64_t most = n_vec <= 32 ? 1024 : (V == 8 && n_vec > 512 ? 768 : 512);
+  if (n_rows > (how == 2 ? 65536 : most)) return p;
+  p.tpr = n_vec <= 256 ? 64 : 512;
+  p.vpt = n_vec <= p.tpr ? 1 : (n_vec <= 2 * p.tpr ? 2 : 4);
+  p.strip = n_vec > 512 ? 8 : 4;
+  p.row_blocks = static_cast<int>(div_up(n_rows, 512 / p.tpr));
+  p.grid = p.row_blocks + static_cast<int>(div_up(n_vec, p.strip));
+  p.on = true;
+  return p;
 }
 
 struct RowsPlan {

@@ -8,6 +8,7 @@
 #include "small_kernels.hip.h"
 #include "tiles_kernels.hip.h"
 #include "long_rows_kernels.hip.h"
+#include "pair_rows_kernels.hip.h"
 
 #include <atomic>
 #include "status.h"
@@ -373,6 +374,27 @@ int tiles_bwd(const T* dy, const T* x, const float* gamma, const float* mean, co
   return launch_col_reduce(part, dgamma, dbeta, p.sums_RS, D, st);
 }
 
+template <typename T>
+int pair_bwd_launch(const PairPlan& p, const T* dy, const T* x, const float* gamma, const float* mean, const float* rstd,
+                    int64_t n_rows, int64_t D, T* dx, float* dgamma, float* dbeta, hipStream_t st) {
+  constexpr int V = VecOf<T>::value;
+#define ATEXN_PAIR(TPR_, VPT_, STRIP_)                                                                            \
+  rows_bwd_pair<T, V, TPR_, VPT_, STRIP_><<<p.grid, kPairThreads, 0, st>>>(dy, x, gamma, mean, rstd, dx, dgamma,  \
+                                                                           dbeta, n_rows, static_cast<int>(D), p.row_blocks)
+  if (p.tpr == 64) {
+    if (p.vpt == 1) ATEXN_PAIR(64, 1, 4);
+    else if (p.vpt == 2) ATEXN_PAIR(64, 2, 4);
+    else ATEXN_PAIR(64, 4, 4);
+  } else {
+    if (p.vpt == 1) ATEXN_PAIR(512, 1, 4);
+    else if (p.vpt == 2) ATEXN_PAIR(512, 2, 8);
+    else ATEXN_PAIR(512, 4, 8);
+  }
+#undef ATEXN_PAIR
+  ATEXN_CHECK_LAUNCH("rows_bwd_pair");
+  return ATEXN_OK;
+}
+
 template <typename T, int V, bool AFF>
 int rows_bwd_v(const T* dy, const T* x, const float* gamma, const float* mean, const float* rstd,
                int64_t n_rows, int64_t D, int C, T* dx, float* dgamma, float* dbeta, void* ws,
@@ -542,6 +564,10 @@ int rows_bwd_t(bool affine, const void* dy_, const void* x_, const float* gamma,
   }
   if (route.tiles) {
     return tiles_bwd<T>(dy, x, gamma, mean, rstd, n_rows, D, dx, dgamma, dbeta, ws, ws_bytes, st);
+  }
+  if (!affine && route.V > 1 && static_cast<const void*>(dx) != static_cast<const void*>(dy) && bwd_stage_mask() == 3) {
+    const PairPlan p = plan_pair(VEC, n_rows, D);
+    if (p.on) return pair_bwd_launch<T>(p, dy, x, gamma, mean, rstd, n_rows, D, dx, dgamma, dbeta, st);
   }
   if (route.V > 1) {
     return affine ? rows_bwd_v<T, VEC, true>(dy, x, gamma, mean, rstd, n_rows, D, C, dx, dgamma, dbeta, ws, ws_bytes, st)
