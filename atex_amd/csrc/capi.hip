@@ -144,7 +144,7 @@ int atexn_abi_version(void) { return kAbiVersion; }
 int atexn_set_tuning(const char* name, int value) {
   ATEXN_REQUIRE(name != nullptr && value >= 0, "bad tuning request");
   ATEXN_REQUIRE(value >= 1 || !strcmp(name, "reverse_second_pass") || !strcmp(name, "cl_fused") ||
-                    !strcmp(name, "cl_fold_cap") || !strcmp(name, "cl_single") || !strcmp(name, "affine_fold") || !strcmp(name, "affine_fold_polls") || !strcmp(name, "cl_single_polls") || !strcmp(name, "cl_single_xm") || !strcmp(name, "cl_single_occ") || !strcmp(name, "plane_single") || !strcmp(name, "plane_single_occ") || !strcmp(name, "plane_single_polls") || !strcmp(name, "bwd_lds_rows") || !strcmp(name, "staged_rows") || !strcmp(name, "cl_narrow_tiles") || !strcmp(name, "cl_fused_split") || !strcmp(name, "long_rows") || !strcmp(name, "long_rows_polls") || !strcmp(name, "pair_rows") || !strcmp(name, "cl_flat") || !strcmp(name, "cl_flat_polls"),
+                    !strcmp(name, "cl_fold_cap") || !strcmp(name, "cl_single") || !strcmp(name, "affine_fold") || !strcmp(name, "affine_fold_polls") || !strcmp(name, "cl_single_polls") || !strcmp(name, "cl_single_xm") || !strcmp(name, "cl_single_occ") || !strcmp(name, "plane_single") || !strcmp(name, "plane_single_occ") || !strcmp(name, "plane_single_polls") || !strcmp(name, "bwd_lds_rows") || !strcmp(name, "staged_rows") || !strcmp(name, "cl_narrow_tiles") || !strcmp(name, "cl_fused_split") || !strcmp(name, "long_rows") || !strcmp(name, "long_rows_polls") || !strcmp(name, "pair_rows") || !strcmp(name, "cl_flat") || !strcmp(name, "cl_flat_polls") || !strcmp(name, "cl_hold"),
                 "value must be >= 1");
   Tuning& t = tuning();
   if (!strcmp(name, "fwd_waves_per_cu")) t.fwd_waves_per_cu = value;
@@ -238,6 +238,9 @@ int atexn_set_tuning(const char* name, int value) {
   } else if (!strcmp(name, "cl_flat")) {
     ATEXN_REQUIRE(value >= 0 && value <= 2, "cl_flat must be 0, 1 or 2");
     t.cl_flat = value;
+  } else if (!strcmp(name, "cl_hold")) {
+    ATEXN_REQUIRE(value >= 0 && value <= 2, "cl_hold must be 0, 1 or 2");
+    t.cl_hold = value;
   } else if (!strcmp(name, "cl_flat_polls")) {
     t.cl_flat_polls = value;
   } else if (!strcmp(name, "cl_fold_cap")) {
@@ -263,7 +266,10 @@ int atexn_bench_describe_bwd(int op, int dtype, int layout, int64_t N, int64_t C
   int n = 0;
   if (op == 1 && layout == ATEXN_LAYOUT_N_C) {
     const ClPlan p = plan_cl(true, C >= vec ? vec : 1, N, C, D, cus);
-    if (p.flat.on)
+    if (p.flat.on && p.flat.hold)
+      n = snprintf(out, out_bytes, "cl_hold_bwd (S=%d slabs, U=%d, %d read twice, grid %lld x %d threads; cl_bwd_sums and two stages when dx == dy)%s; alone=0",
+                   p.flat.S, p.flat.U, p.flat.R, (long long)p.flat.grid, p.flat.threads, N > 1 ? " + col_reduce" : "");
+    else if (p.flat.on)
       n = snprintf(out, out_bytes, "cl_flat_bwd (S=%d slabs, U=%d, grid %lld x %d threads%s; two stages when dx == dy)%s; alone=0", p.flat.S,
                    p.flat.U, (long long)p.flat.grid, p.flat.threads, p.flat.local ? ", instances on one XCD" : "", N > 1 ? " + col_reduce" : "");
     else if (p.fused)

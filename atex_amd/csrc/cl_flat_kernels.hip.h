@@ -45,11 +45,11 @@ __device__ __forceinline__ int flat_uniform(int v) { return __builtin_amdgcn_rea
 struct FlatArgs {
   int64_t N, D, E;     // instances, pixels and elements (D * C) of one
   int C, P, A;         // channels; vectors per period; lanes that hold data
-  int S, base, extra;  // slabs per instance; periods of a slab, the first `extra` have one more
+  int S, base, extra;  // slabs per instance; periods of a slab, the last `extra` have one more
   int pix;             // pixels per period
   int width;           // lanes that share the fold of a channel: a power of two, at least S if S < 64, else 64
   float inv_d;         // 1 / D
-  float px_more, px_base, px_last;  // pixels of the first `extra` slabs, of the others, of the last one
+  float px_more, px_base, px_last;  // pixels of the last `extra` slabs, of the others, of the very last one
   int local;           // the slabs of an instance on one XCD
   int k_at;            // where in LDS the channels' parameters, then constants, are: behind the sums
   ExchangeArgs ex;
@@ -65,8 +65,9 @@ struct FlatSlab {
 };
 template <int V>
 __device__ __forceinline__ FlatSlab flat_slab(const FlatArgs& a, int s) {
-  const int64_t p0 = static_cast<int64_t>(s) * a.base + (s < a.extra ? s : a.extra);
-  const int k = a.base + (s < a.extra ? 1 : 0);
+  const int more = s - (a.S - a.extra);
+  const int64_t p0 = static_cast<int64_t>(s) * a.base + (more > 0 ? more : 0);
+  const int k = a.base + (more >= 0 ? 1 : 0);
   const int64_t px0 = p0 * a.pix, px1 = px0 + static_cast<int64_t>(k) * a.pix;
   const int64_t px = (px1 < a.D ? px1 : a.D) - px0;
   FlatSlab f;
@@ -76,7 +77,7 @@ __device__ __forceinline__ FlatSlab flat_slab(const FlatArgs& a, int s) {
 }
 
 __device__ __forceinline__ float flat_pixels(const FlatArgs& a, int s) {
-  return s == a.S - 1 ? a.px_last : (s < a.extra ? a.px_more : a.px_base);
+  return s == a.S - 1 ? a.px_last : (s < a.S - a.extra ? a.px_base : a.px_more);
 }
 
 // Which slab of which instance the workgroup takes.  local: unit by unit on each XCD (cl_single_place
@@ -344,8 +345,8 @@ __device__ __forceinline__ float flat_group_sum(float v, int width) {
   if (width >= 64) v = swap_add<32>(v);
   return v;
 }
-// Channel c of instance n (want: there is one) from all slabs' pairs, by a.width lanes, each taking every
-// width-th slab; false when a wait of the wave runs out.  STATS: (mean, m2) by Chan's merge of all slabs at
+// Channel c of instance n (want: there is one) from the pairs of at most 64 slabs, by a.width lanes; false
+// when a wait of the wave runs out.  STATS: (mean, m2) by Chan's merge of all slabs at
 // once; else sums.
 template <bool STATS>
 __device__ __forceinline__ bool flat_fold(const FlatArgs& a, unsigned tag, int64_t n, int c, bool want, int polls,
@@ -355,36 +356,76 @@ __device__ __forceinline__ bool flat_fold(const FlatArgs& a, unsigned tag, int64
   const unsigned stride = static_cast<unsigned>(a.C) * 2;
   const cl_word* const at = a.tagged + n * a.S * a.C * 2;
   const unsigned col = want ? 2u * c : 0u;
-  r0 = r1 = 0.f;
-  float p = 0.f, q = 0.f;  // of the lane's first slab
-#pragma unroll 1
-  for (int l0 = 0; l0 < a.S; l0 += a.width) {
-    const int l = l0 + sub;
-    const bool mine = want && l < a.S;
-    float lp, lq;
-    if (!exchange_wait_pair(at + (mine ? l * stride + col : 0u), mine, tag, polls, trouble, lp, lq)) return false;
-    r0 += mine ? (STATS ? lp * flat_pixels(a, l) : lp) : 0.f;
-    if constexpr (!STATS) r1 += mine ? lq : 0.f;
-    if (l0 == 0) {
-      p = lp;
-      q = lq;
-    }
-  }
-  r0 = flat_group_sum(r0, a.width);
+  const bool mine = want && sub < a.S;
+  float p, q;
+  if (!exchange_wait_pair(at + (mine ? sub * stride + col : 0u), mine, tag, polls, trouble, p, q)) return false;
+  r0 = flat_group_sum(mine ? (STATS ? p * flat_pixels(a, sub) : p) : 0.f, a.width);
   if constexpr (STATS) {
     r0 *= a.inv_d;
     const float d = p - r0;
-    r1 = want && sub < a.S ? q + flat_pixels(a, sub) * (d * d) : 0.f;
-#pragma unroll 1
-    for (int l = sub + a.width; l < a.S && want; l += a.width) {  // (read again: all of them are there)
-      const float lp = __builtin_bit_cast(float, static_cast<unsigned>(cl_peek(at + l * stride + col)));
-      const float lq = __builtin_bit_cast(float, static_cast<unsigned>(cl_peek(at + l * stride + col + 1)));
-      const float ld = lp - r0;
-      r1 += lq + flat_pixels(a, l) * (ld * ld);
+    q += flat_pixels(a, sub) * (d * d);
+  }
+  r1 = flat_group_sum(mine ? q : 0.f, a.width);
+  return true;
+}
+
+// The same by the whole workgroup, for more slabs than a wave has lanes: thread t takes the slabs t, t +
+// threads.  All threads call it, and all get the result; buf: 3 * 16 floats.
+template <bool STATS>
+__device__ __forceinline__ bool flat_fold_wide(const FlatArgs& a, unsigned tag, int64_t n, int c, int nt, int polls,
+                                               unsigned* trouble, float* buf, float& r0, float& r1) {
+#pragma clang fp contract(off)
+  constexpr int R = kFlatMaxSlabs / 256;
+  const unsigned stride = static_cast<unsigned>(a.C) * 2;
+  const cl_word* const at = a.tagged + (n * a.S * a.C + c) * 2;
+  const int wave = threadIdx.x / kWave, nw = nt / kWave;
+  float p[R], q[R];
+  float s0 = 0.f, s1 = 0.f;
+  bool ok = true;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    p[r] = q[r] = 0.f;
+    const int l = static_cast<int>(threadIdx.x) + r * nt;
+    if (ok && r * nt < a.S) {  // (wave-uniform)
+      ok = exchange_wait_pair(at + (l < a.S ? l * stride : 0u), l < a.S, tag, polls, trouble, p[r], q[r]);
+      s0 += l < a.S ? (STATS ? p[r] * flat_pixels(a, l) : p[r]) : 0.f;
+      if constexpr (!STATS) s1 += l < a.S ? q[r] : 0.f;
     }
   }
-  r1 = flat_group_sum(r1, a.width);
-  return true;
+  s0 = group_sum<kWave>(s0);
+  if constexpr (!STATS) s1 = group_sum<kWave>(s1);
+  __syncthreads();
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    buf[wave] = s0;
+    buf[16 + wave] = s1;
+    buf[32 + wave] = ok ? 0.f : 1.f;
+  }
+  __syncthreads();
+  r0 = buf[0];
+  r1 = buf[16];
+  float bad = buf[32];
+  for (int w = 1; w < nw; ++w) {
+    r0 += buf[w];
+    r1 += buf[16 + w];
+    bad += buf[32 + w];
+  }
+  if constexpr (STATS) {
+    r0 *= a.inv_d;
+    s1 = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int l = static_cast<int>(threadIdx.x) + r * nt;
+      const float d = p[r] - r0;
+      s1 += l < a.S ? q[r] + flat_pixels(a, l) * (d * d) : 0.f;
+    }
+    s1 = group_sum<kWave>(s1);
+    __syncthreads();
+    if ((threadIdx.x & (kWave - 1)) == 0) buf[wave] = s1;
+    __syncthreads();
+    r1 = buf[0];
+    for (int w = 1; w < nw; ++w) r1 += buf[w];
+  }
+  return flat_uniform(bad > 0.f) == 0;
 }
 
 __device__ __forceinline__ void flat_publish(cl_word* pair, float v0, float v1, unsigned tag, bool local) {
@@ -394,23 +435,35 @@ __device__ __forceinline__ void flat_publish(cl_word* pair, float v0, float v1, 
 
 struct FlatShared {  // in LDS
   int fail;
+  float buf[48];
 };
 
-// The exchange of instance n by its workgroup s; *sm_fail: whether a wait ran out.  OP: result(n, c, r0, r1)
+// The exchange of instance n by its workgroup s; sm.fail: whether a wait ran out.  OP: result(n, c, r0, r1)
 // (what the instance's folded pair means: outputs, and the pair to publish), constants(n, c, r0, r1) (in
 // LDS, from the published pair).
 template <bool STATS, typename Op>
-__device__ __forceinline__ void flat_exchange(const FlatArgs& a, Op& op, int* sm_fail, int nt, unsigned tag, int64_t n,
+__device__ __forceinline__ void flat_exchange(const FlatArgs& a, Op& op, FlatShared& sm, int nt, unsigned tag, int64_t n,
                                               int s) {
   const int polls = a.ex.max_polls;
   unsigned* const trouble = a.ex.trouble;
   const int lane = threadIdx.x & (kWave - 1), wave = flat_uniform(threadIdx.x / kWave), nw = nt / kWave;
   const int at_once = kWave / a.width;  // channels of a wave
-  if (threadIdx.x == 0) *sm_fail = 0;
+  if (threadIdx.x == 0) sm.fail = 0;
   __syncthreads();
   bool fail = false;
+  if (a.S > kWave) {
 #pragma unroll 1
-  for (int c0 = s + wave * at_once * a.S; c0 < a.C && !fail; c0 += nw * at_once * a.S) {
+    for (int c = s; c < a.C && !fail; c += a.S) {  // (the same in every wave)
+      float r0, r1;
+      fail = !flat_fold_wide<STATS>(a, tag, n, c, nt, polls, trouble, sm.buf, r0, r1);
+      if (!fail && threadIdx.x == 0) {
+        op.result(n, c, r0, r1);
+        flat_publish(a.finals + (n * a.C + c) * 2, r0, r1, tag, a.local);
+      }
+    }
+  }
+#pragma unroll 1
+  for (int c0 = a.S > kWave ? a.C : s + wave * at_once * a.S; c0 < a.C && !fail; c0 += nw * at_once * a.S) {
     const int c = c0 + lane / a.width * a.S;
     float r0, r1;
     fail = !flat_fold<STATS>(a, tag, n, c, c < a.C, polls, trouble, r0, r1);
@@ -426,7 +479,7 @@ __device__ __forceinline__ void flat_exchange(const FlatArgs& a, Op& op, int* sm
     fail = !exchange_wait_pair(a.finals + (n * a.C + (c < a.C ? c : 0)) * 2, c < a.C, tag, polls, trouble, r0, r1);
     if (!fail && c < a.C) op.constants(n, c, r0, r1);
   }
-  if (fail && lane == 0) *sm_fail = 1;
+  if (fail && lane == 0) sm.fail = 1;
   __syncthreads();
 }
 
@@ -457,7 +510,16 @@ __device__ __forceinline__ void flat_alone(const FlatArgs& a, Op& op, FlatShared
   }
   __syncthreads();
   // the sums of every slab are there, or in the hands of a running workgroup
-  for (int c0 = wave * at_once; c0 < a.C; c0 += nw * at_once) {
+  for (int c = 0; c < a.C && a.S > kWave; ++c) {
+    float r0, r1;
+    if (!flat_fold_wide<STATS>(a, tag, n, c, nt, kFlatOwnPolls, nullptr, sm.buf, r0, r1)) r0 = r1 = __builtin_nanf("");
+    if (threadIdx.x == 0) {
+      op.result(n, c, r0, r1);
+      flat_publish(a.finals + (n * a.C + c) * 2, r0, r1, tag, a.local);
+      op.constants(n, c, r0, r1);
+    }
+  }
+  for (int c0 = a.S > kWave ? a.C : wave * at_once; c0 < a.C; c0 += nw * at_once) {
     const int c = c0 + lane / a.width;
     float r0, r1;
     if (!flat_fold<STATS>(a, tag, n, c, c < a.C, kFlatOwnPolls, nullptr, r0, r1)) r0 = r1 = __builtin_nanf("");
@@ -520,13 +582,18 @@ struct FlatFwdOp {
     const int c = static_cast<int>(threadIdx.x) < a.C ? threadIdx.x : 0;
     return Params{gamma[c], beta[c]};
   }
+  template <bool MANY = true>  // (more channels than threads)
   __device__ __forceinline__ void keep(int64_t, Params p) const {
     float* k = lds + a.k_at;
+    const int mine = static_cast<int>(threadIdx.x) < a.C ? threadIdx.x : 0;  // (no branch: the others have channel 0's)
+    k[a.C + mine] = p.g;
+    k[2 * a.C + mine] = p.b;
+    if (MANY && a.C > nt) {  // (a loop with loads waits for all others before it)
 #pragma unroll 1
-    for (int c = threadIdx.x; c < a.C; c += nt) {
-      if (c >= nt) p = Params{gamma[c], beta[c]};
-      k[a.C + c] = p.g;
-      k[2 * a.C + c] = p.b;
+      for (int c = threadIdx.x + nt; c < a.C; c += nt) {
+        k[a.C + c] = gamma[c];
+        k[2 * a.C + c] = beta[c];
+      }
     }
   }
   __device__ __forceinline__ void params(int64_t n) const { keep(n, fetch(n)); }
@@ -619,7 +686,7 @@ cl_flat_fwd(const T* __restrict__ x, const float* __restrict__ gamma, const floa
     flat_merge_stats<V>(a, f, flat_pixels(a, s), U, m, q, nt, flat_lds, [&](int c, float cm, float cq) { op.publish(n, s, c, cm, cq); });
   }
   if (a.S > 1) {
-    flat_exchange<true>(a, op, &sm.fail, nt, tag, n, s);
+    flat_exchange<true>(a, op, sm, nt, tag, n, s);
   } else {
     if (threadIdx.x == 0) sm.fail = 0;
     __syncthreads();
@@ -660,14 +727,18 @@ struct FlatBwdOp {
   };
   __device__ __forceinline__ Params fetch(int64_t n) const { return at(n, static_cast<int>(threadIdx.x) < a.C ? threadIdx.x : 0); }
   __device__ __forceinline__ Params at(int64_t n, int c) const { return Params{mean_in[n * a.C + c], gamma[c], rstd_in[n * a.C + c]}; }
+  template <bool MANY = true>  // (more channels than threads)
   __device__ __forceinline__ void keep(int64_t n, Params p) const {
     float* k = lds + a.k_at;
+    auto put = [&](int c, const Params& v) {
+      k[c] = v.m;
+      k[a.C + c] = v.g;
+      k[2 * a.C + c] = v.r;
+    };
+    put(static_cast<int>(threadIdx.x) < a.C ? threadIdx.x : 0, p);  // (no branch: the others have channel 0's)
+    if (MANY && a.C > nt) {  // (a loop with loads waits for all others before it)
 #pragma unroll 1
-    for (int c = threadIdx.x; c < a.C; c += nt) {
-      if (c >= nt) p = at(n, c);
-      k[c] = p.m;
-      k[a.C + c] = p.g;
-      k[2 * a.C + c] = p.r;
+      for (int c = threadIdx.x + nt; c < a.C; c += nt) put(c, at(n, c));
     }
   }
   __device__ __forceinline__ void params(int64_t n) const { keep(n, fetch(n)); }
@@ -794,7 +865,7 @@ cl_flat_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __re
     flat_merge_sums<V>(a, b, d, nt, flat_lds, [&](int c, float cb, float cd) { op.publish(n, s, c, cb, cd); });
   }
   if (a.S > 1) {
-    flat_exchange<false>(a, op, &sm.fail, nt, tag, n, s);
+    flat_exchange<false>(a, op, sm, nt, tag, n, s);
   } else {
     if (threadIdx.x == 0) sm.fail = 0;
     __syncthreads();

@@ -1,7 +1,8 @@
 // Launchers of the flat channels-last kernels, templated on the storage type.
 #pragma once
 
-#include "cl_flat_kernels.hip.h"
+#include "cl_hold_kernels.hip.h"
+#include "large_lds.h"
 #include "plan.h"
 #include "status.h"
 
@@ -27,7 +28,7 @@ inline FlatArgs flat_args(const FlatPlan& p, int64_t N, int64_t C, int64_t D, vo
   a.inv_d = 1.0f / static_cast<float>(D);
   a.px_base = static_cast<float>(int64_t(p.base) * p.pix);
   a.px_more = static_cast<float>((int64_t(p.base) + 1) * p.pix);
-  a.px_last = static_cast<float>(D - (int64_t(p.S - 1) * p.base + p.extra) * p.pix);
+  a.px_last = static_cast<float>(D - (int64_t(p.S - 1) * p.base + std::max(p.extra - 1, 0)) * p.pix);
   a.local = p.local;
   a.k_at = p.k_at;
   a.ex = ExchangeArgs{e.tag, e.at, tuning().cl_flat_polls, e.trouble};
@@ -35,6 +36,23 @@ inline FlatArgs flat_args(const FlatPlan& p, int64_t N, int64_t C, int64_t D, vo
   a.finals = reinterpret_cast<cl_word*>(w + p.off_finals);
   a.claims = reinterpret_cast<unsigned*>(w + p.off_claims);
   return a;
+}
+
+inline HoldArgs hold_args(const FlatPlan& p) { return HoldArgs{p.U, p.R, p.hold_at}; }
+
+template <auto Kernel, typename... Args>
+int hold_launch(const FlatPlan& p, hipStream_t st, const char* name, Args... args) {
+  ATEXN_REQUIRE(allow_large_lds<Kernel>() == hipSuccess, "this device does not give a workgroup %zu bytes of LDS", p.lds);
+  Kernel<<<static_cast<unsigned>(p.grid), p.threads, p.lds, st>>>(args..., hold_args(p));
+  ATEXN_CHECK_LAUNCH(name);
+  return ATEXN_OK;
+}
+// f(K): the kind of the plan's hold kernel as a constant.
+template <size_t N, typename F, size_t... K>
+int hold_kind(const HoldKind (&)[N], const FlatPlan& p, F&& f, std::index_sequence<K...>) {
+  int rc = ATEXN_INVALID_ARGUMENT;
+  (void)((static_cast<int>(K) == p.kind && ((rc = f(std::integral_constant<size_t, K>{})), true)) || ...);
+  return rc;
 }
 
 // Launches the call's kernel unless its workgroups may not exchange results (taken: it did).
@@ -48,6 +66,13 @@ int flat_fwd_v(const FlatPlan& p, const T* x, const float* gamma, const float* b
   if (!taken) return ATEXN_OK;
   const FlatArgs a = flat_args(p, N, C, D, ws, e);
   const unsigned grid = static_cast<unsigned>(p.grid);
+  if (p.hold) {
+    return hold_kind(kPlanHoldFwd, p, [&](auto k) {
+      constexpr HoldKind h = kPlanHoldFwd[k];
+      return hold_launch<cl_hold_fwd<T, V, h.HA, kPlanHoldFwdPass, h.lds, kPlanHoldFwdBatch>>(
+          p, st, "cl_hold_fwd", x, gamma, beta, y, mean, rstd, a, eps);
+    }, std::make_index_sequence<std::size(kPlanHoldFwd)>{});
+  }
 #define ATEXN_FLAT_FWD(U_) \
   case U_: cl_flat_fwd<T, V, U_><<<grid, p.threads, p.lds, st>>>(x, gamma, beta, y, mean, rstd, a, eps); break
   switch (p.U) {
@@ -80,6 +105,15 @@ int flat_bwd_v(const FlatPlan& p, const T* dy, const T* x, const float* gamma, c
   float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + p.off_part);
   float* o0 = N == 1 ? dgamma : part;
   float* o1 = N == 1 ? dbeta : part + C;
+  if (p.hold) {
+    ATEXN_TRY(hold_kind(kPlanHoldBwd, p, [&](auto k) {
+      constexpr HoldKind h = kPlanHoldBwd[k];
+      return hold_launch<cl_hold_bwd<T, V, h.HA, kPlanHoldBwdPass, h.lds, kPlanHoldBwdBatch>>(
+          p, st, "cl_hold_bwd", dy, x, gamma, mean, rstd, dx, o0, o1, 2 * C, a);
+    }, std::make_index_sequence<std::size(kPlanHoldBwd)>{}));
+    if (N > 1) return launch_col_reduce(part, dgamma, dbeta, static_cast<int>(N), C, st);
+    return ATEXN_OK;
+  }
 #define ATEXN_FLAT_BWD(U_) \
   case U_: cl_flat_bwd<T, V, U_><<<grid, p.threads, p.lds, st>>>(dy, x, gamma, mean, rstd, dx, o0, o1, 2 * C, a); break
   switch (p.U) {

@@ -463,7 +463,11 @@ struct ExchangeArgs {
   const unsigned* at;
   int max_polls;
   unsigned* trouble;
-  __device__ __forceinline__ unsigned the_tag() const { return at == nullptr ? tag : *at; }
+  // (Through a pointer that the compiler knows to be global: a flat load on its way makes every later wait
+  // for a vector one for all of them.)
+  __device__ __forceinline__ unsigned the_tag() const {
+    return at == nullptr ? tag : *(const __attribute__((address_space(1))) unsigned*)(at);
+  }
 };
 
 // Loops over strided indices are written in batches of B whose loads are all issued before

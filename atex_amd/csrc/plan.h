@@ -68,6 +68,7 @@ struct Tuning {
   TuneInt cl_single_polls{300};
   TuneInt cl_flat{1};          // channels-last, flat instances (cl_flat_kernels.hip.h); 2: wherever they can
   TuneInt cl_flat_polls{300};  //   their polls
+  TuneInt cl_hold{1};          // channels-last kernels that hold large instances (plan_hold): never, by rule, wherever possible
   TuneInt affine_fold{1};      // channel-first backward, a workgroup per plane: dgamma / dbeta folded over the batch in the row kernel
   TuneInt affine_fold_polls{2000};  //   polls before a workgroup recomputes its peers' plane sums (0: at once)
   // channel-first planes too long for a workgroup: the chunks of a plane on the workgroups of one
@@ -678,6 +679,8 @@ struct FlatPlan {
   int U = 0, threads = 0, P = 0, A = 0, S = 1, base = 0, extra = 0, pix = 1, local = 0, k_at = 0;
   int64_t grid = 0;
   size_t lds = 0, off_tagged = 0, off_finals = 0, off_claims = 0, off_part = 0, off_tag = 0, ws_bytes = 0;
+  bool hold = false;                // cl_hold_kernels.hip.h
+  int kind = 0, R = 0, hold_at = 0;  // which of them; of the U vectors per thread, R are read twice
 };
 constexpr int kPlanFlatMaxSlabs = 512, kPlanFlatMaxThreads = 512, kPlanFlatMaxChannels = 2048;
 constexpr int kPlanFlatUs[] = {16, 12, 8, 6, 4, 3, 2, 1};  // vectors per thread that have a kernel (backward: up to 8)
@@ -692,8 +695,9 @@ inline FlatPlan plan_flat_as(bool bwd, int V, int64_t N, int64_t C, int64_t D, i
   const int64_t m = threads / P, periods = div_up(D, pix);
   if (m < 1 || S < 1 || S > kPlanFlatMaxSlabs || S > periods) return p;
   const int64_t base = periods / S, extra = periods % S;
-  const int64_t last_px = D - (periods - base) * pix;  // the last slab has the fewest pixels
-  if (base + (extra > 0 ? 1 : 0) > U * m || last_px < 1 || last_px < (U - 1) * m * pix) return p;
+  const int64_t most = base + (extra > 0 ? 1 : 0);  // (the last `extra` slabs, the very last may lack pixels)
+  const int64_t last_px = D - (periods - most) * pix;
+  if (most > U * m || base < (U - 1) * m || last_px < 1 || last_px < (U - 1) * m * pix) return p;
   p.U = U;
   p.threads = threads;
   p.P = static_cast<int>(P);
@@ -752,6 +756,68 @@ inline FlatPlan plan_flat(bool bwd, int V, int64_t N, int64_t C, int64_t D, int 
     }
     if (p.on) return p;
   }
+  return p;
+}
+
+// The hold kernels that there are: HA vectors per thread in registers, a last pass of up to Q (kPlanHold*Pass)
+// in registers too; with LDS: Q more there, and any number of passes of Q that are read twice.
+struct HoldKind {
+  int HA;
+  bool lds;
+};
+constexpr int kPlanHoldFwdBatch = 4, kPlanHoldFwdPass = 12, kPlanHoldBwdBatch = 2, kPlanHoldBwdPass = 6;
+constexpr HoldKind kPlanHoldFwd[] = {{12, false}, {24, false}, {36, false}, {36, true}};
+constexpr HoldKind kPlanHoldBwd[] = {{6, false}, {12, false}, {18, false}, {18, true}};
+
+// The hold kernels' plan, whether or not they are the better ones.
+//
+// A thread holds HA + 2 Q vectors (pairs in the backward): 60 or 30 of the 64 that 134 MB of x are on 256 CUs
+// of 512 threads.  As many instances are on the chip at once as that leaves room for (up to a quarter beyond
+// it where that saves a sixth of the rounds: a few vectors read twice cost less than a round whose exchange
+// nothing hides): [8, 524288, 32] fp16 one at a time 148 us forward and 208 us backward, two 107 and 173;
+// [16, 65536, 64] 7 at once, three rounds, 66 us, 8 at once 51 us.  They go on workgroups of 256 threads, two
+// to a CU, so that one instance reads while another one writes.  A single instance at a time goes on 512
+// threads where the exchange of twice the slabs costs more than what the finer slabs even out: backward
+// ([2, 2097152, 32] fp16 190 us against 204), from 128 channels on ([1, 385517, 144] fp32 forward 95.5
+// against 103) and where it does not fit ([2, 2097152, 32] forward 118 against 124; [1, 3000000, 16], which
+// fits, 49 against 46).
+inline FlatPlan plan_hold(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+  FlatPlan p;
+  if (V == 1 || C > kPlanFlatMaxThreads || D * C >= (int64_t(1) << 31) || cus < kPlanXcdCount) return p;
+  int64_t g = V;
+  while (C % g != 0) g /= 2;
+  const int64_t P = C / g, periods = div_up(D, V / g);
+  if (P > kPlanFlatMaxThreads) return p;
+  const int Q = bwd ? kPlanHoldBwdPass : kPlanHoldFwdPass, held = Q * 5;
+  const auto& kinds = bwd ? kPlanHoldBwd : kPlanHoldFwd;
+  const int64_t slots256 = std::min<int64_t>(int64_t(cus) * 2, kPlanFlatMaxSlabs);
+  int threads = C > 256 || 256 / P * 8 < 512 / P * 3 ? 512 : 256;
+  int64_t at_once = 1;
+  if (threads == 256) {
+    const int64_t room = slots256 * (256 / P) * held;
+    auto rounds = [&](int64_t r) { return div_up(N, std::max<int64_t>(1, std::min(N, r / periods))); };
+    const int64_t whole = rounds(room);
+    const int64_t more = rounds(room * 5 / 4);
+    at_once = div_up(N, more * 20 <= whole * 17 ? more : whole);
+    const bool over = room < periods;
+    if (at_once == 1 && (bwd || C >= 128 || (over && C >= 32))) threads = 512;
+  }
+  const int64_t m = threads / P, S0 = threads == 512 ? std::min<int64_t>(cus, kPlanFlatMaxSlabs) : slots256 / at_once;
+  for (int64_t S = S0; S > S0 * 7 / 8 && !p.on; --S) {
+    const int64_t U = div_up(div_up(periods, S), m);
+    if (U > (1 << 20)) return p;
+    p = plan_flat_as(bwd, V, N, C, D, static_cast<int>(U), threads, S, false);
+  }
+  if (!p.on || p.S < 2) return FlatPlan{};
+  if (p.U <= kinds[0].HA) return FlatPlan{};
+  p.kind = 0;
+  while (!kinds[p.kind].lds && p.U > kinds[p.kind].HA + Q) ++p.kind;
+  const bool in_lds = kinds[p.kind].lds;
+  p.R = static_cast<int>(in_lds ? std::max<int64_t>(0, round_up(int64_t(p.U) - kinds[p.kind].HA - 2 * Q, Q)) : 0);
+  p.hold = true;
+  p.hold_at = static_cast<int>(round_up(int64_t(p.lds / sizeof(float)), 4));
+  p.lds = size_t(p.hold_at) * 4 + (in_lds ? size_t(Q) * threads * 16 * (bwd ? 2 : 1) : 0);
+  if (p.lds > kPlanLdsBytes - kPlanBwdLdsReserve) return FlatPlan{};
   return p;
 }
 
@@ -1006,15 +1072,41 @@ inline bool flat_instead(const ClPlan& p, const FlatPlan& f, bool bwd, int V, in
   return V == 8 && p.single && C <= 64 && x2 >= 96;
 }
 
+// Whether that is better than the flat kernels or those of plan_cl_slabs.  (times: those, hold; us)
+// Every slab of every channel costs 32 bytes of pairs, written and read back: not more than one in eight of a
+// pixel's lines, so to speak (S * 128 <= D; [2, 32768, 256] fp16 backward 29.0, 30.1).  Backward: from 17 MiB
+// of x on ([1, 89514, 125] bf16 29.1, 21.4; [2, 12673, 124] fp32, 13 MB, 16.2, 19.5); not the smallest
+// instances of many channels ([38, 3168, 100] fp16 21.5, 22.7), nor 256 channels and more on short slabs
+// ([2, 50000, 320] fp16 52, 63; [3, 100000, 300] bf16 201, 154), nor where the flat kernels' slabs fill each
+// XCD exactly ([64, 16384, 64] bf16 81.5, 85.7; [36, 57624, 16] fp16, where they do not, 49, 40).  Forward: from
+// 24 MiB on and with instances beyond the 4 MiB that one XCD holds ([32, 65536, 32] fp16, of 4 MiB, 44, 48;
+// [9, 72447, 32] bf16, of 4.6 MB, 27.2, 20.8; [16, 65536, 64], of 8 MiB, 65, 51); not in place of the single
+// launch on one XCD where that is whole or fp32 ([5, 15779, 192] fp32 23.7, 30.6), nor with several instances one
+// at a time that leave the chip part empty ([3, 100000, 300] bf16 104, 121; [2, 85000, 133] fp16 28.5, 37.8).
+inline bool hold_instead(const ClPlan& p, const FlatPlan& h, bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+  if (!h.on || int64_t(h.S) * 128 > D) return false;
+  const int64_t inst = C * D * 16 / V, x = N * inst;
+  if (bwd) {
+    const int64_t xcd_slots = int64_t(cus) / kPlanXcdCount * (1024 / std::max(p.flat.threads, 1));
+    if (p.flat.on && p.flat.local && h.R > 0 && N % kPlanXcdCount == 0 && xcd_slots % p.flat.S == 0) return false;
+    return x >= (int64_t(17) << 20) && (inst >= (int64_t(1) << 20) || C <= 64) && (C < 256 || h.U >= 30);
+  }
+  if (p.single && (V == 4 || !p.single_xm || p.xm_resident)) return false;
+  return x >= (int64_t(24) << 20) && inst > (int64_t(4) << 20) && (N == 1 || h.threads == 256 || h.U >= 40);
+}
+
 inline ClPlan plan_cl(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
   ClPlan p = plan_cl_slabs(bwd, V, N, C, D, cus);
-  const int how = tuning().cl_flat;
-  if (how == 0 || (how == 1 && (p.fused || N * C * D < (int64_t(1) << 19)))) return p;  // (flat_instead wants more)
-  const FlatPlan f = plan_flat(bwd, V, N, C, D, cus);
-  if (how == 2 ? f.on : flat_instead(p, f, bwd, V, N, C, D, cus)) {
-    p.flat = f;
-    p.ws_bytes = std::max(p.ws_bytes, f.ws_bytes);
+  const int how = tuning().cl_flat, hold = tuning().cl_hold;
+  if (how != 0 && (how == 2 || !(p.fused || N * C * D < (int64_t(1) << 19)))) {  // (flat_instead wants more)
+    const FlatPlan f = plan_flat(bwd, V, N, C, D, cus);
+    if (how == 2 ? f.on : flat_instead(p, f, bwd, V, N, C, D, cus)) p.flat = f;
   }
+  if (hold != 0 && (hold == 2 || N * C * D * 16 / V >= (int64_t(17) << 20))) {  // (hold_instead wants more)
+    const FlatPlan h = plan_hold(bwd, V, N, C, D, cus);
+    if (hold == 2 ? h.on : hold_instead(p, h, bwd, V, N, C, D, cus)) p.flat = h;
+  }
+  if (p.flat.on) p.ws_bytes = std::max(p.ws_bytes, p.flat.ws_bytes);
   return p;
 }
 

@@ -2,6 +2,7 @@
 // translation unit per dtype instantiates them (rows_launch_*.hip).
 #pragma once
 
+#include "large_lds.h"
 #include "plan.h"
 #include "rows_kernels.hip.h"
 #include "plane_single_kernels.hip.h"
@@ -29,25 +30,6 @@ using BwdResidentFn = void (*)(const T*, const T*, const float*, const float*, c
 
 // Row batching (RB > 1) exists for the vector path and rows of at most one wave; the
 // predicate-free EXACT variants exist for the vector path.
-// The kernels that keep a row (or its accumulators) in LDS ask for more dynamic LDS than a
-// launch gets by default: the limit is raised once per kernel and device.
-template <auto Kernel>
-inline hipError_t allow_large_lds() {
-  static std::atomic<uint64_t> done{0};
-  int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
-    (void)hipGetLastError();
-    dev = -1;
-  }
-  if (dev >= 0 && ((done.load(std::memory_order_acquire) >> dev) & 1)) return hipSuccess;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(Kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           static_cast<int>(kPlanLdsBytes - kPlanBwdLdsReserve));
-  if (e == hipSuccess && dev >= 0) done.fetch_or(uint64_t(1) << dev, std::memory_order_release);
-  if (e != hipSuccess) (void)hipGetLastError();
-  return e;
-}
-
 template <typename T, int V, int TPR, int VPT, bool AFF>
 FwdResidentFn<T, V, AFF> fwd_variant(int rb, bool exact, bool ragged) {
   if constexpr (V > 1) {

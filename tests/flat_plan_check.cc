@@ -1,6 +1,7 @@
-// Host-only check of the plans of the flat channels-last kernels (atex_amd/csrc/plan.h): what the kernels
+// Host-only check of the plans of the flat and hold channels-last kernels (atex_amd/csrc/plan.h): what the kernels
 // assume of them, and that threads, steps and slabs cover every element of an instance once.  Built and run
-// by tests/test_flat_plans.py.  "ok <plans> <with several slabs>" on success.
+// by tests/test_flat_plans.py.  "ok <plans> <with several slabs> <plans that hold
+// more>" on success.
 #include <cstdio>
 #include <vector>
 
@@ -12,7 +13,7 @@ const Tuning& tuning() { return g_tuning; }
 }  // namespace atexn
 using namespace atexn;
 
-static long g_plans = 0, g_split = 0, g_failed = 0;
+static long g_plans = 0, g_split = 0, g_held = 0, g_failed = 0;
 #define EXPECT(cond)                                                                                              \
   do {                                                                                                            \
     if (!(cond) && ++g_failed < 50)                                                                               \
@@ -20,39 +21,49 @@ static long g_plans = 0, g_split = 0, g_failed = 0;
                   (long long)N, (long long)C, (long long)D, cus, p.U, p.threads, p.S);                            \
   } while (0)
 
-static void check(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
-  const FlatPlan p = plan_flat(bwd, V, N, C, D, cus);
+static void check(bool hold, bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+  const FlatPlan p = hold ? plan_hold(bwd, V, N, C, D, cus) : plan_flat(bwd, V, N, C, D, cus);
   if (!p.on) return;
-  ++g_plans;
-  if (p.S > 1) ++g_split;
+  ++(hold ? g_held : g_plans);
+  if (!hold && p.S > 1) ++g_split;
   EXPECT(p.threads == 256 || p.threads == 512);
   EXPECT(p.A <= p.threads && p.A % p.P == 0 && int64_t(p.P) * V == C * p.pix && V % p.pix == 0);
   bool built = false;
   for (const int u : kPlanFlatUs) built = built || (p.U == u && (u <= 8 || !bwd));
-  EXPECT(built);
+  EXPECT(p.hold == hold && (built || hold));
+  if (hold) {  // every vector but the last one is whole, and the passes are what the kernel of that kind has
+    const int Q = bwd ? kPlanHoldBwdPass : kPlanHoldFwdPass, B = bwd ? kPlanHoldBwdBatch : kPlanHoldFwdBatch;
+    const HoldKind k = bwd ? kPlanHoldBwd[p.kind] : kPlanHoldFwd[p.kind];
+    const int before = k.HA + (k.lds ? Q : 0) + p.R;  // vectors before the last pass
+    EXPECT(p.S > 1 && C <= p.threads && p.R >= 0 && p.R % Q == 0 && (k.lds || p.R == 0) && Q % B == 0 && k.HA % B == 0);
+    EXPECT(before < p.U && p.U <= before + Q && p.U >= Q);
+    EXPECT(p.hold_at % 4 == 0 && p.hold_at >= p.k_at + int(bwd ? 4 : 3) * C);
+    EXPECT(p.lds == size_t(4) * p.hold_at + (k.lds ? size_t(Q) * p.threads * 16 * (bwd ? 2 : 1) : 0) && p.lds <= 160 * 1024 - 512);
+    EXPECT(int64_t(p.U) * p.A * 16 < (int64_t(1) << 32));
+  }
   // the slabs are the instance's periods; every step of every slab but the last is whole
   const int64_t E = D * C, step = int64_t(p.A) * V;
   int64_t at = 0, least = E;
   for (int s = 0; s < p.S; ++s) {
-    const int64_t p0 = int64_t(s) * p.base + std::min(s, p.extra), k = p.base + (s < p.extra ? 1 : 0);
+    const int64_t p0 = int64_t(s) * p.base + std::max(s - (p.S - p.extra), 0), k = p.base + (s >= p.S - p.extra ? 1 : 0);
     const int64_t px0 = p0 * p.pix, px1 = std::min(px0 + k * p.pix, D);
     EXPECT(px0 * C == at && px1 > px0);
     const int64_t n = (px1 - px0) * C;
-    EXPECT(n <= p.U * step && n >= (p.U - 1) * step && n < (int64_t(1) << 24));
+    EXPECT(n <= p.U * step && n >= (p.U - 1) * step && (hold || n < (int64_t(1) << 24)) && (k * p.pix < (1 << 24) || hold));
     // pixel counts as the fold takes them
-    const int64_t said = s == p.S - 1 ? D - (int64_t(p.S - 1) * p.base + p.extra) * p.pix
-                                      : (int64_t(p.base) + (s < p.extra ? 1 : 0)) * p.pix;
+    const int64_t said = s == p.S - 1 ? D - (int64_t(p.S - 1) * p.base + std::max(p.extra - 1, 0)) * p.pix
+                                      : (int64_t(p.base) + (s >= p.S - p.extra ? 1 : 0)) * p.pix;
     EXPECT(said == px1 - px0);
     at += n;
     least = std::min(least, n);
   }
   EXPECT(at == E && least > 0);
   // an instance's slabs are on the chip (the XCD) together; 32-bit positions in its pairs
-  const int64_t slots = int64_t(cus) * (1024 / p.threads);
+  const int64_t slots = int64_t(cus) * ((hold ? 512 : 1024) / p.threads);
   EXPECT(p.S <= (p.local ? slots / 8 : slots) && 4 * int64_t(p.S) * C < (int64_t(1) << 32));
   EXPECT(p.grid == (p.local ? round_up(N, 8) : N) * p.S && p.grid * p.threads < (int64_t(1) << 32));
   EXPECT(size_t(p.k_at) >= 2 * size_t(step) + 2 * size_t(std::max<int64_t>(p.threads, C)));
-  EXPECT(p.lds >= sizeof(float) * (size_t(p.k_at) + size_t(bwd ? 4 : 3) * size_t(C)) && p.lds + 2048 <= 65536 + 1536);
+  EXPECT(p.lds >= sizeof(float) * (size_t(p.k_at) + size_t(bwd ? 4 : 3) * size_t(C)) && (hold || p.lds + 2048 <= 65536 + 1536));
   const size_t pairs = p.S > 1 ? size_t(16) * N * p.S * C : 0, finals = p.S > 1 ? size_t(16) * N * C : 0;
   EXPECT(p.off_tagged == 0 && p.off_finals >= pairs && p.off_claims >= p.off_finals + finals);
   EXPECT(p.off_part >= p.off_claims + (p.S > 1 ? size_t(4) * N * p.S : 0));
@@ -76,10 +87,10 @@ int main() {
         for (const int cus : {256, 304, 64, 8, 7})
           for (const int V : {8, 4}) {
             if (C < V) continue;
-            check(false, V, N, C, D, cus);
-            check(true, V, N, C, D, cus);
+            for (const bool hold : {false, true})
+              for (const bool bwd : {false, true}) check(hold, bwd, V, N, C, D, cus);
           }
   if (g_failed) return 1;
-  std::printf("ok %ld %ld\n", g_plans, g_split);
+  std::printf("ok %ld %ld %ld\n", g_plans, g_split, g_held);
   return 0;
 }

@@ -1,4 +1,4 @@
-"""Plans of the flat channels-last kernels against what the kernels assume of them, on the CPU."""
+"""Plans of the flat and hold channels-last kernels against what the kernels assume of them, on the CPU."""
 import os
 import subprocess
 
@@ -12,5 +12,5 @@ def test_flat_plans_cover_every_instance_once(tmp_path):
                    check=True, capture_output=True, text=True)
     run = subprocess.run([exe], capture_output=True, text=True)
     assert run.returncode == 0, run.stdout[-4000:]
-    plans, split = (int(v) for v in run.stdout.split()[1:])
-    assert plans > 100_000 and split > 50_000
+    plans, split, held = (int(v) for v in run.stdout.split()[1:])
+    assert plans > 100_000 and split > 50_000 and held > 20_000
