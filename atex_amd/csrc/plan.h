@@ -1078,7 +1078,9 @@ inline bool flat_instead(const ClPlan& p, const FlatPlan& f, bool bwd, int V, in
 // of x on ([1, 89514, 125] bf16 29.1, 21.4; [2, 12673, 124] fp32, 13 MB, 16.2, 19.5); not the smallest
 // instances of many channels ([38, 3168, 100] fp16 21.5, 22.7), nor 256 channels and more on short slabs
 // ([2, 50000, 320] fp16 52, 63; [3, 100000, 300] bf16 201, 154), nor where the flat kernels' slabs fill each
-// XCD exactly ([64, 16384, 64] bf16 81.5, 85.7; [36, 57624, 16] fp16, where they do not, 49, 40).  Forward: from
+// XCD exactly ([64, 16384, 64] bf16 81.5, 85.7; [36, 57624, 16] fp16, where they do not, 49, 40), nor in place of
+// the single launch on one XCD where all lanes have a vector and all XCDs the same work ([8, 16384, 64] fp32
+// 20.4, 25.5, [16, 8192, 128] fp16 24.4, 28.1; else [24, 16384, 48] bf16 34.6, 26.7, [20, 16384, 64] fp16 35, 28).  Forward: from
 // 24 MiB on and with instances beyond the 4 MiB that one XCD holds ([32, 65536, 32] fp16, of 4 MiB, 44, 48;
 // [9, 72447, 32] bf16, of 4.6 MB, 27.2, 20.8; [16, 65536, 64], of 8 MiB, 65, 51); not in place of the single
 // launch on one XCD where that is whole or fp32 ([5, 15779, 192] fp32 23.7, 30.6), nor with several instances one
@@ -1088,6 +1090,7 @@ inline bool hold_instead(const ClPlan& p, const FlatPlan& h, bool bwd, int V, in
   const int64_t inst = C * D * 16 / V, x = N * inst;
   if (bwd) {
     const int64_t xcd_slots = int64_t(cus) / kPlanXcdCount * (1024 / std::max(p.flat.threads, 1));
+    if (p.single && !p.flat.on && p.TPP * p.CT == p.CV && N * p.CT % kPlanXcdCount == 0) return false;
     if (p.flat.on && p.flat.local && h.R > 0 && N % kPlanXcdCount == 0 && xcd_slots % p.flat.S == 0) return false;
     return x >= (int64_t(17) << 20) && (inst >= (int64_t(1) << 20) || C <= 64) && (C < 256 || h.U >= 30);
   }
