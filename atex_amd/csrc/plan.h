@@ -1073,8 +1073,8 @@ inline bool flat_instead(const ClPlan& p, const FlatPlan& f, bool bwd, int V, in
 }
 
 // Whether that is better than the flat kernels or those of plan_cl_slabs.  (times: those, hold; us)
-// Every slab of every channel costs 32 bytes of pairs, written and read back: not more than one in eight of a
-// pixel's lines, so to speak (S * 128 <= D; [2, 32768, 256] fp16 backward 29.0, 30.1).  Backward: from 17 MiB
+// A channel's pair costs 32 bytes a slab, written and read back: slabs of at least 128 pixels, whose channel is
+// 256 bytes in fp16 ([5, 15779, 192] fp32 on slabs of 123 backward 46, 56).  Backward: from 17 MiB
 // of x on ([1, 89514, 125] bf16 29.1, 21.4; [2, 12673, 124] fp32, 13 MB, 16.2, 19.5); not the smallest
 // instances of many channels ([38, 3168, 100] fp16 21.5, 22.7), nor 256 channels and more on short slabs
 // ([2, 50000, 320] fp16 52, 63; [3, 100000, 300] bf16 201, 154), nor where the flat kernels' slabs fill each
