@@ -267,10 +267,10 @@ int atexn_bench_describe_bwd(int op, int dtype, int layout, int64_t N, int64_t C
   if (op == 1 && layout == ATEXN_LAYOUT_N_C) {
     const ClPlan p = plan_cl(true, C >= vec ? vec : 1, N, C, D, cus);
     if (p.flat.on && p.flat.hold)
-      n = snprintf(out, out_bytes, "cl_hold_bwd (S=%d slabs, U=%d, %d read twice, grid %lld x %d threads; cl_bwd_sums and two stages when dx == dy)%s; alone=0",
+      n = snprintf(out, out_bytes, "cl_hold_bwd (S=%d slabs, U=%d, %d read twice, grid %lld x %d threads; the slab kernels when dx == dy)%s; alone=0",
                    p.flat.S, p.flat.U, p.flat.R, (long long)p.flat.grid, p.flat.threads, N > 1 ? " + col_reduce" : "");
     else if (p.flat.on)
-      n = snprintf(out, out_bytes, "cl_flat_bwd (S=%d slabs, U=%d, grid %lld x %d threads%s; two stages when dx == dy)%s; alone=0", p.flat.S,
+      n = snprintf(out, out_bytes, "cl_flat_bwd (S=%d slabs, U=%d, grid %lld x %d threads%s; the slab kernels when dx == dy)%s; alone=0", p.flat.S,
                    p.flat.U, (long long)p.flat.grid, p.flat.threads, p.flat.local ? ", instances on one XCD" : "", N > 1 ? " + col_reduce" : "");
     else if (p.fused)
       n = snprintf(out, out_bytes, "cl_bwd_fused (u=%d, grid %lld x %d)%s; alone=0", p.fused_u, (long long)N,

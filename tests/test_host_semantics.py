@@ -273,7 +273,16 @@ def test_every_planning_parameter_is_settable_in_the_benchmark_build():
     assert L.atexn_bench_describe_bwd(1, 1, 1, 8, 64, 16384, buf, 256) > 0
     assert b"cl_bwd_single" in buf.value and b"alone=0" in buf.value
     assert L.atexn_bench_describe_bwd(1, 1, 1, 2, 32, 2097152, buf, 256) > 0
-    assert b"cl_bwd_sums" in buf.value and b"alone=0" in buf.value
+    assert buf.value.startswith(b"cl_hold_bwd (") and buf.value.endswith(b"alone=0")
+    assert b"cl_bwd_sums" not in buf.value  # (what a call in place takes is not what this one does)
+    for off in (b"cl_hold", b"cl_flat"):
+        assert L.atexn_set_tuning(off, 0) == 0
+    try:
+        assert L.atexn_bench_describe_bwd(1, 1, 1, 2, 32, 2097152, buf, 256) > 0
+        assert buf.value.startswith(b"cl_bwd_sums + ") and buf.value.endswith(b"alone=0")
+    finally:
+        for off in (b"cl_hold", b"cl_flat"):
+            assert L.atexn_set_tuning(off, 1) == 0
     assert L.atexn_bench_describe_bwd(1, 1, 0, 2, 32, 2097152, buf, 256) > 0
     assert b"plane_bwd_single (S=64" in buf.value and b"folded over the batch" in buf.value
     # planes of any length: the split kernels' plan (few planes) and the staged kernels' (many) carry it
