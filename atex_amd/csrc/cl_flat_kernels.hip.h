@@ -666,7 +666,7 @@ template <typename T, int V, int U>
 __global__ void __launch_bounds__(kFlatMaxThreads, 4)
 cl_flat_fwd(const T* __restrict__ x, const float* __restrict__ gamma, const float* __restrict__ beta,
             T* __restrict__ y, float* __restrict__ mean_out, float* __restrict__ rstd_out, FlatArgs a, float eps) {
-  extern __shared__ float flat_lds[];
+  extern __shared__ __attribute__((aligned(16))) float flat_lds[];
   __shared__ FlatShared sm;
   const int nt = block_threads();
   const unsigned tag = a.S > 1 ? a.ex.the_tag() : 0;
@@ -841,7 +841,7 @@ __global__ void __launch_bounds__(kFlatMaxThreads, 4)
 cl_flat_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __restrict__ gamma,
             const float* __restrict__ mean_in, const float* __restrict__ rstd_in, T* __restrict__ dx,
             float* __restrict__ o0, float* __restrict__ o1, int64_t o_stride, FlatArgs a) {
-  extern __shared__ float flat_lds[];
+  extern __shared__ __attribute__((aligned(16))) float flat_lds[];
   __shared__ FlatShared sm;
   const int nt = block_threads();
   const unsigned tag = a.S > 1 ? a.ex.the_tag() : 0;

@@ -24,7 +24,7 @@ namespace atexn {
 
 struct HoldArgs {
   int U, R;     // vectors per thread: all, read twice (a multiple of Q)
-  int hold_at;  // where in LDS (floats) the held vectors are
+  int hold_at;  // where in LDS (floats, a multiple of 4) the held vectors are
 };
 
 // Mean and squared deviations of a thread's V streams over the vectors from, ..., B - 1 of a batch (the last
@@ -219,7 +219,7 @@ cl_hold_fwd(const T* __restrict__ x, const float* __restrict__ gamma, const floa
             HoldArgs h) {
   static_assert(HA % B == 0 && Q % B == 0, "whole batches");
   constexpr int NB = Q / B;
-  extern __shared__ float flat_lds[];
+  extern __shared__ __attribute__((aligned(16))) float flat_lds[];
   __shared__ FlatShared sm;
   const int nt = block_threads();
   const unsigned tag = a.ex.the_tag();
@@ -316,7 +316,7 @@ cl_hold_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __re
             float* __restrict__ o0, float* __restrict__ o1, int64_t o_stride, FlatArgs a, HoldArgs h) {
   static_assert(HA % B == 0 && Q % B == 0, "whole batches");
   constexpr int NB = Q / B;
-  extern __shared__ float flat_lds[];
+  extern __shared__ __attribute__((aligned(16))) float flat_lds[];
   __shared__ FlatShared sm;
   const int nt = block_threads();
   const unsigned tag = a.ex.the_tag();

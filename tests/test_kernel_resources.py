@@ -86,6 +86,16 @@ def test_the_configurations_kernels_use_no_scratch_memory(kernels):
             assert kernels[n]["scratch_bytes_per_lane"] == 0, f"{n}: {kernels[n]}"
 
 
+def test_held_vectors_lie_on_16_bytes_in_lds(kernels):
+    """The dynamic LDS of the flat and held kernels holds 16-byte vectors at multiples of 16 bytes from its
+    start (hold_at, a multiple of 4 floats): what lies before it must be as many bytes, and fit the 512 that the
+    planner leaves for it."""
+    ours = {n: r for n, r in kernels.items() if re.search(r"cl_(flat|hold)_(fwd|bwd)I", n)}
+    assert len(ours) >= 2 * 3 * 4
+    for name, r in ours.items():
+        assert r["lds_bytes"] % 16 == 0 and r["lds_bytes"] <= 512, f"{name}: {r}"
+
+
 def test_bf16_builds_need_no_more_scratch_than_fp16_plus_a_little(kernels):
     """bf16 has no mixed-precision arithmetic (conversions cost registers); a twin far above its
     fp16 kernel means the code keeps converted copies alive."""
