@@ -37,6 +37,11 @@ namespace atexn {
 constexpr int kFlatMaxThreads = 512;
 constexpr int kFlatMaxSlabs = 512;
 constexpr int kFlatOwnPolls = 1 << 16;  // for values known to be published: bounds the wait only
+// Polls of a wait that is cut short (exchange_wait_pair).  The slabs of an instance that is on the chip
+// together end some microseconds apart, the more the larger they are: after 24 polls of about 0.15 us most
+// workgroups of held instances took running peers for absent ones (fp16 [2, 128^3, 32] on a free GPU, forward
+// 121 us -> 570, backward [8, 524288, 32] 175 -> 1078), after 48 some still did, after 99 none.
+constexpr int kFlatHastyPolls = 160;
 
 // A value that is the same in every thread, as the compiler's scalar: a branch on it keeps no copy of the
 // held vectors for lanes that might not take it.
@@ -358,7 +363,7 @@ __device__ __forceinline__ bool flat_fold(const FlatArgs& a, unsigned tag, int64
   const unsigned col = want ? 2u * c : 0u;
   const bool mine = want && sub < a.S;
   float p, q;
-  if (!exchange_wait_pair(at + (mine ? sub * stride + col : 0u), mine, tag, polls, trouble, p, q)) return false;
+  if (!exchange_wait_pair(at + (mine ? sub * stride + col : 0u), mine, tag, polls, trouble, p, q, kFlatHastyPolls)) return false;
   r0 = flat_group_sum(mine ? (STATS ? p * flat_pixels(a, sub) : p) : 0.f, a.width);
   if constexpr (STATS) {
     r0 *= a.inv_d;
@@ -387,7 +392,8 @@ __device__ __forceinline__ bool flat_fold_wide(const FlatArgs& a, unsigned tag, 
     p[r] = q[r] = 0.f;
     const int l = static_cast<int>(threadIdx.x) + r * nt;
     if (ok && r * nt < a.S) {  // (wave-uniform)
-      ok = exchange_wait_pair(at + (l < a.S ? l * stride : 0u), l < a.S, tag, polls, trouble, p[r], q[r]);
+      ok = exchange_wait_pair(at + (l < a.S ? l * stride : 0u), l < a.S, tag, polls, trouble, p[r], q[r],
+                              kFlatHastyPolls);
       s0 += l < a.S ? (STATS ? p[r] * flat_pixels(a, l) : p[r]) : 0.f;
       if constexpr (!STATS) s1 += l < a.S ? q[r] : 0.f;
     }
@@ -476,7 +482,8 @@ __device__ __forceinline__ void flat_exchange(const FlatArgs& a, Op& op, FlatSha
   for (int c0 = wave * kWave; c0 < a.C && !fail; c0 += nt) {
     const int c = c0 + lane;
     float r0, r1;
-    fail = !exchange_wait_pair(a.finals + (n * a.C + (c < a.C ? c : 0)) * 2, c < a.C, tag, polls, trouble, r0, r1);
+    fail = !exchange_wait_pair(a.finals + (n * a.C + (c < a.C ? c : 0)) * 2, c < a.C, tag, polls, trouble, r0, r1,
+                               kFlatHastyPolls);
     if (!fail && c < a.C) op.constants(n, c, r0, r1);
   }
   if (fail && lane == 0) sm.fail = 1;

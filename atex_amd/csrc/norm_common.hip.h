@@ -438,13 +438,15 @@ constexpr int kExchangeHastyPolls = 24;
 constexpr unsigned kExchangeTroubleCalls = 256;  // (consecutive calls' tags are two apart)
 // cl_wait_pair under that rule.  All 64 lanes of the wave must call it; the result is the same
 // in all of them.  trouble == nullptr or a limit below kExchangePatientPolls: the plain wait.
+// hasty: the polls of a kernel whose resident peers may need longer than kExchangeHastyPolls.
 __device__ __forceinline__ bool exchange_wait_pair(const cl_word* pair, bool want, unsigned tag, int max_polls,
-                                                   unsigned* trouble, float& a, float& b) {
+                                                   unsigned* trouble, float& a, float& b,
+                                                   int hasty = kExchangeHastyPolls) {
   a = b = 0.f;
   const bool adaptive = trouble != nullptr && max_polls >= kExchangePatientPolls;
   for (int poll = 0; poll < max_polls; ++poll) {
     // (the record is fetched along with the poll's own loads: one round trip, not two)
-    const bool decide = adaptive && poll == kExchangeHastyPolls - 1;
+    const bool decide = adaptive && poll == hasty - 1;
     unsigned seen = 0;
     if (decide) seen = __hip_atomic_load(trouble, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (cl_try_pair(pair, want, tag, a, b)) return true;

@@ -174,6 +174,55 @@ def test_random_shapes_beside_the_occupier(seed):
         L.atexn_bench_mark_exchange_trouble(0)
 
 
+def _median_us(call, before, reps=7):
+    """Median duration of single calls behind a busy stretch of the stream, the first left out."""
+    import torch
+
+    times = []
+    for _ in range(reps):
+        torch.cuda.synchronize()
+        before()
+        torch.cuda._sleep(400000)
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        call()
+        e1.record()
+        torch.cuda.synchronize()
+        times.append(e0.elapsed_time(e1) * 1e3)
+    return float(np.median(times[1:]))
+
+
+def _channels_last_calls(capi, N, S, C, dtype):
+    import torch
+
+    gen = torch.Generator(device="cuda").manual_seed(79)
+    x, dy = (torch.randn((N, S, C), device="cuda", generator=gen).to(util.torch_dtype(dtype)) for _ in range(2))
+    gamma = torch.rand(C, device="cuda", generator=gen) + 0.5
+    beta = torch.randn(C, device="cuda", generator=gen) * 0.1
+    _, m, r = capi.in_fwd(x, gamma, beta, EPS, dtype, False)
+    return (lambda: capi.in_fwd(x, gamma, beta, EPS, dtype, False),
+            lambda: capi.in_bwd(dy, x, gamma, m, r, dtype, False))
+
+
+# held instances one and two at a time, flat ones on one XCD each and over all of them
+@pytest.mark.parametrize("N,S,C,dtype", [(2, 2097152, 32, "f16"), (8, 524288, 32, "f16"), (1, 385517, 144, "f32"),
+                                         (36, 36288, 29, "bf16"), (1, 598464, 17, "f16")])
+def test_waits_cut_short_find_peers_that_are_running(N, S, C, dtype):
+    """After a wait that ran out, on a GPU that is free again: slabs of hundreds of KB end microseconds apart,
+    and a wait cut short still lasts that long (or every workgroup redoes its peers' work: 4 to 6 times the
+    duration, where 1.4 is allowed)."""
+    capi = util.Capi(bench=True)
+    calls = _channels_last_calls(capi, N, S, C, dtype)
+    try:
+        for what, call in zip(("forward", "backward"), calls):
+            patient = _median_us(call, lambda: capi.L.atexn_bench_mark_exchange_trouble(0))
+            short = _median_us(call, lambda: capi.L.atexn_bench_mark_exchange_trouble(1))
+            print(f"{what} [{N}, {S}, {C}] {dtype}: patient {patient:.1f} us, cut short {short:.1f} us", flush=True)
+            assert short < 1.4 * patient + 5.0, what
+    finally:
+        capi.L.atexn_bench_mark_exchange_trouble(0)
+
+
 def test_the_occupier_leaves_in_time():
     import time
 
