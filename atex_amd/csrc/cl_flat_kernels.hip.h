@@ -22,12 +22,15 @@
 //
 // Nothing depends on which workgroups are on the chip together.  A workgroup publishes its slab's sums
 // before it waits for anything, and every wait is a bounded number of polls.  A workgroup whose wait runs
-// out helps itself: it computes the slabs whose sums it cannot see, to the same bits, a vector at a time
-// through memory, each slab by the one workgroup that claims it (an atomic compare-and-swap on a word per
-// slab), folds all channels of the instance and normalises its slab, again through memory.  That is code of
-// its own, outside the kernel: compiled into it, it doubled the registers of the held vectors, and what a
-// kernel runs only once in a while comes from memory cold, some microseconds of instruction fetches.  The
-// outputs must not alias x (the slabs are read again).
+// out looks which slabs have no sums, all at once, claims one of them (an atomic exchange on a word per slab),
+// computes its sums, to the same bits, and looks again until nothing is left to claim: every slab's sums are
+// there or in the hands of a running workgroup.  It does the duties of the slabs that it has computed (the
+// channels that they fold) besides its own, so that every channel's fold is a running workgroup's, waits for
+// those, and reads its own slab a second time to normalise it.  That is code of its own, outside the kernel:
+// compiled into it, it doubled the registers of the held vectors (the look and the claim alone, for workgroups
+// that find nothing to claim to go on with theirs, spilled 25), and what a kernel runs only once in a while
+// comes from memory cold, some microseconds of instruction fetches.  The outputs must not alias x (the slabs are
+// read again).
 #pragma once
 
 #include "norm_common.hip.h"
@@ -36,6 +39,7 @@ namespace atexn {
 
 constexpr int kFlatMaxThreads = 512;
 constexpr int kFlatMaxSlabs = 512;
+constexpr int kFlatFwdMost = 16, kFlatBwdMost = 8;  // vectors per thread
 constexpr int kFlatOwnPolls = 1 << 16;  // for values known to be published: bounds the wait only
 // Polls of a wait that is cut short (exchange_wait_pair).  The slabs of an instance that is on the chip
 // together end some microseconds apart, the more the larger they are: after 24 polls of about 0.15 us most
@@ -133,46 +137,52 @@ __device__ __forceinline__ void flat_advance(unsigned& at, unsigned step) {
   at += step;
   asm volatile("" : "+v"(at));
 }
-// The thread's U vectors of a slab.  All steps but the last are whole (the planner sees to it); nv: the
-// thread's valid elements of the last one, the others read as zero.
-template <typename T, int V, int U, bool LAST>
-__device__ __forceinline__ void flat_load(const T* src, int A, int n_el, u32x4 (&raw)[U], int& nv) {
+// The thread's U vectors of a slab (at most MAX; the last one in the last place).  All steps but the last are
+// whole (the planner sees to it); nv: the thread's valid elements of the last one, the others read as zero.
+template <typename T, int V, int MAX, bool LAST>
+__device__ __forceinline__ void flat_load(const T* src, int A, int n_el, int U, u32x4 (&raw)[MAX], int& nv) {
   const int t = static_cast<int>(threadIdx.x);
   const unsigned step = static_cast<unsigned>(A) * V;
   unsigned at = static_cast<unsigned>(t) * V;
   const int left = n_el - static_cast<int>((U - 1) * step + at);
   nv = t >= A || left <= 0 ? 0 : (left < V ? left : V);
 #pragma unroll
-  for (int u = 0; u < U; ++u) raw[u] = u32x4{};
+  for (int u = 0; u < MAX; ++u) raw[u] = u32x4{};
   if (t < A) {
 #pragma unroll
-    for (int u = 0; u < U - 1; ++u) {
-      raw[u] = flat_bits(LAST ? load_pack_last<T, V>(src + at) : load_pack<T, V>(src + at));
-      flat_advance(at, step);
+    for (int u = 0; u < MAX - 1; ++u) {
+      if (u < U - 1) {
+        raw[u] = flat_bits(LAST ? load_pack_last<T, V>(src + at) : load_pack<T, V>(src + at));
+        flat_advance(at, step);
+      }
     }
     if (nv == V) {
-      raw[U - 1] = flat_bits(LAST ? load_pack_last<T, V>(src + at) : load_pack<T, V>(src + at));
-    } else if (nv > 0) {
+      raw[MAX - 1] = flat_bits(LAST ? load_pack_last<T, V>(src + at) : load_pack<T, V>(src + at));
+    }
+    // (an `else` puts these loads, and the wait for them, ahead of the whole vector's)
+    if (nv > 0 && nv < V) {
       Pack<T, V> part;
 #pragma unroll
       for (int i = 0; i < V; ++i) part.v[i] = i < nv ? src[at + i] : T(0);
-      raw[U - 1] = flat_bits(part);
+      raw[MAX - 1] = flat_bits(part);
     }
   }
   __builtin_amdgcn_sched_barrier(0);  // every load is on its way before the first use
 }
-template <typename T, int V, int U, typename F>
-__device__ __forceinline__ void flat_store(T* dst, int A, int nv, F&& value) {
+template <typename T, int V, int MAX, typename F>
+__device__ __forceinline__ void flat_store(T* dst, int A, int U, int nv, F&& value) {
   const int t = static_cast<int>(threadIdx.x);
   const unsigned step = static_cast<unsigned>(A) * V;
   unsigned at = static_cast<unsigned>(t) * V;
   if (t >= A) return;
 #pragma unroll
-  for (int u = 0; u < U - 1; ++u) {
-    store_pack<T, V>(dst + at, value(u));
-    flat_advance(at, step);
+  for (int u = 0; u < MAX - 1; ++u) {
+    if (u < U - 1) {
+      store_pack<T, V>(dst + at, value(u));
+      flat_advance(at, step);
+    }
   }
-  if (nv > 0) store_pack_n<T, V>(dst + at, value(U - 1), nv);
+  if (nv > 0) store_pack_n<T, V>(dst + at, value(MAX - 1), nv);
 }
 
 // How the workgroup's threads share the entries of the channels: thread (q, c) of Q * C, or with more
@@ -213,31 +223,35 @@ __device__ __forceinline__ void flat_each(const float* l, int first, int end, in
   }
 }
 
-// The thread's V streams over its U vectors (the last one nv elements): mean and squared deviations, an
-// exact two-pass over the registers.  vector(u): the u-th.
-template <typename T, int V, int UNROLL, typename Vector>
+// The thread's V streams over its U vectors (placed as flat_load has them; the last one nv elements): mean and
+// squared deviations, an exact two-pass over the registers.
+template <typename T, int V, int MAX, typename Vector>
 __device__ __forceinline__ void flat_lane_stats(int U, int nv, Vector&& vector, float (&m)[V], float (&q)[V]) {
-#pragma clang fp contract(off)  // (a thread's sums have the same bits from its registers and through memory)
+#pragma clang fp contract(off)  // (a thread's sums have the same bits wherever they are computed)
   const float one = mix_one();
 #pragma unroll
   for (int i = 0; i < V; ++i) m[i] = q[i] = 0.f;
-#pragma unroll UNROLL
-  for (int u = 0; u < U; ++u) {
-    const Pack<T, V> x = vector(u);
 #pragma unroll
-    for (int i = 0; i < V; ++i) m[i] = add_f32<T>(m[i], x.v[i], one);
+  for (int u = 0; u < MAX; ++u) {
+    if (u < U - 1 || u == MAX - 1) {
+      const Pack<T, V> x = vector(u);
+#pragma unroll
+      for (int i = 0; i < V; ++i) m[i] = add_f32<T>(m[i], x.v[i], one);
+    }
   }
   const float whole = 1.0f / static_cast<float>(U), less = U > 1 ? 1.0f / static_cast<float>(U - 1) : 0.f;
 #pragma unroll
   for (int i = 0; i < V; ++i) m[i] *= i < nv ? whole : less;
-#pragma unroll UNROLL
-  for (int u = 0; u < U; ++u) {
-    const Pack<T, V> x = vector(u);
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
-      float d = sub_f32<T>(x.v[i], m[i], one);
-      if (u == U - 1) d = i < nv ? d : 0.f;
-      q[i] = __builtin_fmaf(d, d, q[i]);
+  for (int u = 0; u < MAX; ++u) {
+    if (u < U - 1 || u == MAX - 1) {
+      const Pack<T, V> x = vector(u);
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        float d = sub_f32<T>(x.v[i], m[i], one);
+        if (u == MAX - 1) d = i < nv ? d : 0.f;
+        q[i] = __builtin_fmaf(d, d, q[i]);
+      }
     }
   }
 }
@@ -290,21 +304,23 @@ __device__ __forceinline__ void flat_merge_stats(const FlatArgs& a, const FlatSl
 }
 
 // The same for the backward's sums: b = sum dy * (x - mu), s = sum dy.
-template <typename T, int V, int UNROLL, typename Vx, typename Vd>
+template <typename T, int V, int MAX, typename Vx, typename Vd>
 __device__ __forceinline__ void flat_lane_sums(int U, Vx&& vx, Vd&& vd, const float (&mu)[V], float (&b)[V],
                                                float (&s)[V]) {
 #pragma clang fp contract(off)
   const float one = mix_one();
 #pragma unroll
   for (int i = 0; i < V; ++i) b[i] = s[i] = 0.f;
-#pragma unroll UNROLL
-  for (int u = 0; u < U; ++u) {
-    const Pack<T, V> x = vx(u), d = vd(u);
 #pragma unroll
-    for (int i = 0; i < V; ++i) {
-      // (what the last step does not have reads as dy = 0)
-      b[i] = __builtin_fmaf(to_f32(d.v[i]), sub_f32<T>(x.v[i], mu[i], one), b[i]);
-      s[i] = add_f32<T>(s[i], d.v[i], one);
+  for (int u = 0; u < MAX; ++u) {
+    if (u < U - 1 || u == MAX - 1) {
+      const Pack<T, V> x = vx(u), d = vd(u);
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        // (what the last step does not have reads as dy = 0)
+        b[i] = __builtin_fmaf(to_f32(d.v[i]), sub_f32<T>(x.v[i], mu[i], one), b[i]);
+        s[i] = add_f32<T>(s[i], d.v[i], one);
+      }
     }
   }
 }
@@ -440,124 +456,153 @@ __device__ __forceinline__ void flat_publish(cl_word* pair, float v0, float v1, 
 }
 
 struct FlatShared {  // in LDS
-  int fail;
+  int fail;  // a wait has run out
+  int pick;  // the slab that the workgroup has claimed then
   float buf[48];
+  unsigned open[kFlatMaxSlabs / 32], mine[kFlatMaxSlabs / 32];  // slabs: nobody's, computed by this workgroup
 };
 
-// The exchange of instance n by its workgroup s; sm.fail: whether a wait ran out.  OP: result(n, c, r0, r1)
-// (what the instance's folded pair means: outputs, and the pair to publish), constants(n, c, r0, r1) (in
-// LDS, from the published pair).
-template <bool STATS, typename Op>
-__device__ __forceinline__ void flat_exchange(const FlatArgs& a, Op& op, FlatShared& sm, int nt, unsigned tag, int64_t n,
-                                              int s) {
-  const int polls = a.ex.max_polls;
-  unsigned* const trouble = a.ex.trouble;
+// The fold of the channels of slab `sk` by the workgroup, published as the instance's; whether a wait of the
+// wave ran out.  OP: result(n, c, r0, r1) (what the instance's folded pair means: outputs, and the pair to
+// publish).  CERTAIN: for sums that are on their way; should they not show up after all, the results are
+// marked (NaN).
+template <bool STATS, bool CERTAIN, typename Op>
+__device__ __forceinline__ bool flat_own(const FlatArgs& a, Op& op, FlatShared& sm, int nt, unsigned tag, int64_t n, int sk,
+                                         int polls, unsigned* trouble) {
   const int lane = threadIdx.x & (kWave - 1), wave = flat_uniform(threadIdx.x / kWave), nw = nt / kWave;
   const int at_once = kWave / a.width;  // channels of a wave
-  if (threadIdx.x == 0) sm.fail = 0;
-  __syncthreads();
   bool fail = false;
-  if (a.S > kWave) {
-#pragma unroll 1
-    for (int c = s; c < a.C && !fail; c += a.S) {  // (the same in every wave)
-      float r0, r1;
-      fail = !flat_fold_wide<STATS>(a, tag, n, c, nt, polls, trouble, sm.buf, r0, r1);
-      if (!fail && threadIdx.x == 0) {
-        op.result(n, c, r0, r1);
-        flat_publish(a.finals + (n * a.C + c) * 2, r0, r1, tag, a.local);
-      }
+  auto done = [&](int c, bool mine, float r0, float r1) {
+    if (CERTAIN && fail) {
+      r0 = r1 = __builtin_nanf("");
+      fail = false;
     }
-  }
-#pragma unroll 1
-  for (int c0 = a.S > kWave ? a.C : s + wave * at_once * a.S; c0 < a.C && !fail; c0 += nw * at_once * a.S) {
-    const int c = c0 + lane / a.width * a.S;
-    float r0, r1;
-    fail = !flat_fold<STATS>(a, tag, n, c, c < a.C, polls, trouble, r0, r1);
-    if (!fail && c < a.C && (lane & (a.width - 1)) == 0) {
+    if (!fail && mine) {
       op.result(n, c, r0, r1);
       flat_publish(a.finals + (n * a.C + c) * 2, r0, r1, tag, a.local);
     }
+  };
+  if (a.S > kWave) {
+#pragma unroll 1
+    for (int c = sk; c < a.C && !fail; c += a.S) {  // (the same in every wave)
+      float r0, r1;
+      fail = !flat_fold_wide<STATS>(a, tag, n, c, nt, polls, trouble, sm.buf, r0, r1);
+      done(c, threadIdx.x == 0, r0, r1);
+    }
+  } else {
+#pragma unroll 1
+    for (int c0 = sk + wave * at_once * a.S; c0 < a.C && !fail; c0 += nw * at_once * a.S) {
+      const int c = c0 + lane / a.width * a.S;
+      float r0, r1;
+      fail = !flat_fold<STATS>(a, tag, n, c, c < a.C, polls, trouble, r0, r1);
+      done(c, c < a.C && (lane & (a.width - 1)) == 0, r0, r1);
+    }
   }
+  return fail;
+}
+// The instance's pairs as constants(n, c, r0, r1) in LDS, a lane per channel; whether a wait of the wave ran out.
+template <bool CERTAIN, typename Op>
+__device__ __forceinline__ bool flat_finals(const FlatArgs& a, Op& op, int nt, unsigned tag, int64_t n, int polls,
+                                            unsigned* trouble) {
+  const int lane = threadIdx.x & (kWave - 1), wave = flat_uniform(threadIdx.x / kWave);
+  bool fail = false;
 #pragma unroll 1
   for (int c0 = wave * kWave; c0 < a.C && !fail; c0 += nt) {
     const int c = c0 + lane;
     float r0, r1;
     fail = !exchange_wait_pair(a.finals + (n * a.C + (c < a.C ? c : 0)) * 2, c < a.C, tag, polls, trouble, r0, r1,
                                kFlatHastyPolls);
+    if (CERTAIN && fail) {
+      r0 = r1 = __builtin_nanf("");
+      fail = false;
+    }
     if (!fail && c < a.C) op.constants(n, c, r0, r1);
   }
-  if (fail && lane == 0) sm.fail = 1;
+  return fail;
+}
+
+// The exchange of instance n by its workgroup s; sm.fail: whether a wait ran out.
+template <bool STATS, typename Op>
+__device__ __forceinline__ void flat_exchange(const FlatArgs& a, Op& op, FlatShared& sm, int nt, unsigned tag, int64_t n,
+                                              int s) {
+  if (threadIdx.x == 0) sm.fail = 0;
+  __syncthreads();
+  const bool fail = flat_own<STATS, false>(a, op, sm, nt, tag, n, s, a.ex.max_polls, a.ex.trouble) ||
+                    flat_finals<false>(a, op, nt, tag, n, a.ex.max_polls, a.ex.trouble);
+  if (fail && (threadIdx.x & (kWave - 1)) == 0) sm.fail = 1;
   __syncthreads();
 }
 
-// A workgroup whose wait has run out, to its end.  OP has also params(n) (the channels' parameters into LDS) and
-// sums(n, l) and apply(n, l), which take slab l through memory.
+// A slab of instance n whose sums are neither there nor anybody's to compute, claimed for this workgroup; -1
+// when there is none (left).  A slab's workgroup publishes all of its channels without waiting, so one of them
+// tells.  Every round in which another workgroup was quicker claims a slab: there are at most S.  The claims
+// of workgroups that look at the same time spread over the open slabs.  Contains barriers.
+__device__ __forceinline__ int flat_claim(const FlatArgs& a, FlatShared& sm, int nt, unsigned tag, int64_t n, int s) {
+  constexpr int WORDS = kFlatMaxSlabs / 32;
+  const int t = static_cast<int>(threadIdx.x);
+  unsigned* const claims = a.claims + n * a.S;
+#pragma unroll 1
+  for (int round = 0; round < a.S; ++round) {
+    __syncthreads();
+    if (t < WORDS) sm.open[t] = 0;
+    __syncthreads();
+#pragma unroll 1
+    for (int l = t; l < a.S; l += nt) {
+      const cl_word* const pair = a.tagged + ((n * a.S + l) * a.C + a.C - 1) * 2;
+      const cl_word w0 = cl_peek(pair), w1 = cl_peek(pair + 1);
+      const unsigned whose = __hip_atomic_load(claims + l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const bool there = static_cast<unsigned>(w0 >> 32) == tag && static_cast<unsigned>(w1 >> 32) == ~tag;
+      if (l != s && !there && whose != tag) atomicOr(&sm.open[l / 32], 1u << l % 32);
+    }
+    __syncthreads();
+    if (t == 0) {
+      int total = 0;
+#pragma unroll 1
+      for (int w = 0; w < WORDS; ++w) total += __popc(sm.open[w]);
+      int pick = -1;
+      if (total > 0) {
+        int k = s % total, w = 0;
+#pragma unroll 1
+        while (k >= __popc(sm.open[w])) k -= __popc(sm.open[w++]);
+        unsigned bits = sm.open[w];
+#pragma unroll 1
+        for (; k > 0; --k) bits &= bits - 1;
+        const int l = w * 32 + __ffs(bits) - 1;
+        pick = atomicExch(claims + l, tag) != tag ? l : -2;
+      }
+      sm.pick = pick;
+    }
+    __syncthreads();
+    const int pick = flat_uniform(sm.pick);
+    if (pick != -2) return pick;
+  }
+  return -1;
+}
+
+// A workgroup whose wait has run out, to its end.  OP has also params(n) (the channels' parameters into LDS),
+// sums(n, l) (slab l's, published) and apply(n, l).
 template <bool STATS, typename Op>
 __device__ __forceinline__ void flat_alone(const FlatArgs& a, Op& op, FlatShared& sm, int nt, unsigned tag, int64_t n, int s) {
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, nw = nt / kWave;
-  const int at_once = kWave / a.width;
-  __syncthreads();
+  constexpr int WORDS = kFlatMaxSlabs / 32;
+  if (threadIdx.x < WORDS) sm.mine[threadIdx.x] = 0;
   op.params(n);
-  for (int i = 1; i < a.S; ++i) {  // (from behind its own slab on: the workgroups spread over the missing ones)
-    const int l = s + i < a.S ? s + i : s + i - a.S;
-    __syncthreads();
-    if (threadIdx.x == 0) sm.fail = 0;
-    __syncthreads();
-    for (int c = threadIdx.x; c < a.C; c += nt) {
-      const cl_word* pair = a.tagged + ((n * a.S + l) * a.C + c) * 2;
-      const cl_word w0 = cl_peek(pair), w1 = cl_peek(pair + 1);
-      if (static_cast<unsigned>(w0 >> 32) != tag || static_cast<unsigned>(w1 >> 32) != ~tag) sm.fail = 1;
-    }
-    __syncthreads();
-    if (flat_uniform(sm.fail) == 0) continue;
-    __syncthreads();
-    if (threadIdx.x == 0) sm.fail = atomicExch(a.claims + n * a.S + l, tag) != tag;
-    __syncthreads();
-    if (flat_uniform(sm.fail)) op.sums(n, l);
+#pragma unroll 1
+  for (int l; (l = flat_claim(a, sm, nt, tag, n, s)) >= 0;) {
+    if (threadIdx.x == 0) sm.mine[l / 32] |= 1u << l % 32;
+    op.sums(n, l);
   }
   __syncthreads();
-  // the sums of every slab are there, or in the hands of a running workgroup
-  for (int c = 0; c < a.C && a.S > kWave; ++c) {
-    float r0, r1;
-    if (!flat_fold_wide<STATS>(a, tag, n, c, nt, kFlatOwnPolls, nullptr, sm.buf, r0, r1)) r0 = r1 = __builtin_nanf("");
-    if (threadIdx.x == 0) {
-      op.result(n, c, r0, r1);
-      flat_publish(a.finals + (n * a.C + c) * 2, r0, r1, tag, a.local);
-      op.constants(n, c, r0, r1);
+#pragma unroll 1
+  for (int w = 0; w < WORDS; ++w) {
+    unsigned bits = static_cast<unsigned>(flat_uniform(static_cast<int>(sm.mine[w] | (w == s / 32 ? 1u << s % 32 : 0u))));
+#pragma unroll 1
+    for (; bits != 0; bits &= bits - 1) {
+      flat_own<STATS, true>(a, op, sm, nt, tag, n, w * 32 + __ffs(bits) - 1, kFlatOwnPolls, nullptr);
     }
   }
-  for (int c0 = a.S > kWave ? a.C : wave * at_once; c0 < a.C; c0 += nw * at_once) {
-    const int c = c0 + lane / a.width;
-    float r0, r1;
-    if (!flat_fold<STATS>(a, tag, n, c, c < a.C, kFlatOwnPolls, nullptr, r0, r1)) r0 = r1 = __builtin_nanf("");
-    if (c < a.C && (lane & (a.width - 1)) == 0) {
-      op.result(n, c, r0, r1);
-      flat_publish(a.finals + (n * a.C + c) * 2, r0, r1, tag, a.local);
-      op.constants(n, c, r0, r1);
-    }
-  }
+  flat_finals<true>(a, op, nt, tag, n, kFlatOwnPolls, nullptr);
   __syncthreads();
   op.apply(n, s);
-}
-
-// One vector of a slab, through memory: the thread's u-th of U.
-template <typename T, int V>
-__device__ __forceinline__ Pack<T, V> flat_vector(const T* src, int A, int u, int U, int nv) {
-  const unsigned at = (static_cast<unsigned>(u) * A + threadIdx.x) * V;
-  Pack<T, V> p{};
-  if (static_cast<int>(threadIdx.x) < A) {
-    if (u < U - 1 || nv == V) {
-      p = load_pack<T, V>(src + at);
-    } else {
-#pragma unroll
-      for (int i = 0; i < V; ++i) p.v[i] = i < nv ? src[at + i] : T(0);
-    }
-  }
-  return flat_pinned<T, V>(p);
-}
-__device__ __forceinline__ int flat_valid(int A, int V, int U, int n_el) {
-  const int left = n_el - static_cast<int>((U - 1) * A + threadIdx.x) * V;
-  return static_cast<int>(threadIdx.x) >= A || left <= 0 ? 0 : (left < V ? left : V);
 }
 
 // ------------------------------------------------------------------------------ forward
@@ -640,26 +685,23 @@ struct FlatFwdOp {
       constants(n, c, m, q);
     }
   }
-  // through memory
+  // as the kernel has them
   __device__ __forceinline__ void sums(int64_t n, int l) const {
     const FlatSlab f = flat_slab<V>(a, l);
-    const T* src = x + n * a.E + f.e0;
-    const int nv = flat_valid(a.A, V, U, f.n_el);
+    u32x4 raw[kFlatFwdMost];
+    int nv;
+    flat_load<T, V, kFlatFwdMost, false>(x + n * a.E + f.e0, a.A, f.n_el, U, raw, nv);
     float m[V], q[V];
-    flat_lane_stats<T, V, 1>(U, nv, [&](int u) { return flat_vector<T, V>(src, a.A, u, U, nv); }, m, q);
+    flat_lane_stats<T, V, kFlatFwdMost>(U, nv, [&](int u) { return flat_pack<T, V>(raw[u]); }, m, q);
     flat_merge_stats<V>(a, f, flat_pixels(a, l), U, m, q, nt, lds, [&](int c, float cm, float cq) { publish(n, l, c, cm, cq); });
   }
   __device__ __forceinline__ void apply(int64_t n, int l) const {
     const FlatSlab f = flat_slab<V>(a, l);
-    const int nv = flat_valid(a.A, V, U, f.n_el);
     const Coef k = coef();
-    if (static_cast<int>(threadIdx.x) >= a.A) return;
-#pragma unroll 1
-    for (int u = 0; u < U; ++u) {
-      const unsigned at = (static_cast<unsigned>(u) * a.A + threadIdx.x) * V;
-      const int cnt = u < U - 1 ? V : nv;
-      if (cnt > 0) store_pack_n<T, V>(y + n * a.E + f.e0 + at, k(flat_vector<T, V>(x + n * a.E + f.e0, a.A, u, U, nv)), cnt);
-    }
+    u32x4 raw[kFlatFwdMost];
+    int nv;
+    flat_load<T, V, kFlatFwdMost, true>(x + n * a.E + f.e0, a.A, f.n_el, U, raw, nv);
+    flat_store<T, V, kFlatFwdMost>(y + n * a.E + f.e0, a.A, U, nv, [&](int u) { return k(flat_pinned<T, V>(flat_pack<T, V>(raw[u]))); });
   }
 };
 
@@ -685,7 +727,7 @@ cl_flat_fwd(const T* __restrict__ x, const float* __restrict__ gamma, const floa
   const FlatSlab f = flat_slab<V>(a, s);
   u32x4 raw[U];
   int nv;
-  flat_load<T, V, U, false>(x + n * a.E + f.e0, a.A, f.n_el, raw, nv);
+  flat_load<T, V, U, false>(x + n * a.E + f.e0, a.A, f.n_el, U, raw, nv);
   op.keep(n, params);
   {
     float m[V], q[V];
@@ -701,7 +743,7 @@ cl_flat_fwd(const T* __restrict__ x, const float* __restrict__ gamma, const floa
   if (flat_uniform(sm.fail) == 0) {
     flat_forget(raw);
     const typename FlatFwdOp<T, V>::Coef k = op.coef();
-    flat_store<T, V, U>(y + n * a.E + f.e0, a.A, nv, [&](int u) { return k(flat_pack<T, V>(raw[u])); });
+    flat_store<T, V, U>(y + n * a.E + f.e0, a.A, U, nv, [&](int u) { return k(flat_pack<T, V>(raw[u])); });
   }
   asm volatile("" ::: "memory");  // (asked for again, so that nothing of the slab lives across the call)
   if (flat_uniform(sm.fail) != 0) {
@@ -809,32 +851,29 @@ struct FlatBwdOp {
       constants(n, c, b, d);
     }
   }
-  // through memory
+  // as the kernel has them
   __device__ __forceinline__ void sums(int64_t n, int l) const {
     const FlatSlab f = flat_slab<V>(a, l);
-    const int nv = flat_valid(a.A, V, U, f.n_el);
-    const T* sx = x + n * a.E + f.e0;
-    const T* sd = dy + n * a.E + f.e0;
+    u32x4 rx[kFlatBwdMost], rd[kFlatBwdMost];
+    int nv;
+    flat_load<T, V, kFlatBwdMost, false>(x + n * a.E + f.e0, a.A, f.n_el, U, rx, nv);
+    flat_load<T, V, kFlatBwdMost, false>(dy + n * a.E + f.e0, a.A, f.n_el, U, rd, nv);
     float mu[V], b[V], d[V];
     means(mu);
-    flat_lane_sums<T, V, 1>(U, [&](int u) { return flat_vector<T, V>(sx, a.A, u, U, nv); },
-                         [&](int u) { return flat_vector<T, V>(sd, a.A, u, U, nv); }, mu, b, d);
+    flat_lane_sums<T, V, kFlatBwdMost>(U, [&](int u) { return flat_pack<T, V>(rx[u]); },
+                                       [&](int u) { return flat_pack<T, V>(rd[u]); }, mu, b, d);
     flat_merge_sums<V>(a, b, d, nt, lds, [&](int c, float cb, float cd) { publish(n, l, c, cb, cd); });
   }
   __device__ __forceinline__ void apply(int64_t n, int l) const {
     const FlatSlab f = flat_slab<V>(a, l);
-    const int nv = flat_valid(a.A, V, U, f.n_el);
     const Coef k = coef();
-    if (static_cast<int>(threadIdx.x) >= a.A) return;
-    const int64_t e = n * a.E + f.e0;
-#pragma unroll 1
-    for (int u = 0; u < U; ++u) {
-      const unsigned at = (static_cast<unsigned>(u) * a.A + threadIdx.x) * V;
-      const int cnt = u < U - 1 ? V : nv;
-      if (cnt > 0) {
-        store_pack_n<T, V>(dx + e + at, k(flat_vector<T, V>(x + e, a.A, u, U, nv), flat_vector<T, V>(dy + e, a.A, u, U, nv)), cnt);
-      }
-    }
+    u32x4 rx[kFlatBwdMost], rd[kFlatBwdMost];
+    int nv;
+    flat_load<T, V, kFlatBwdMost, true>(x + n * a.E + f.e0, a.A, f.n_el, U, rx, nv);
+    flat_load<T, V, kFlatBwdMost, true>(dy + n * a.E + f.e0, a.A, f.n_el, U, rd, nv);
+    flat_store<T, V, kFlatBwdMost>(dx + n * a.E + f.e0, a.A, U, nv, [&](int u) {
+      return k(flat_pinned<T, V>(flat_pack<T, V>(rx[u])), flat_pinned<T, V>(flat_pack<T, V>(rd[u])));
+    });
   }
 };
 
@@ -860,8 +899,8 @@ cl_flat_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __re
   const FlatSlab f = flat_slab<V>(a, s);
   u32x4 rx[U], rd[U];
   int nv;
-  flat_load<T, V, U, true>(x + n * a.E + f.e0, a.A, f.n_el, rx, nv);
-  flat_load<T, V, U, true>(dy + n * a.E + f.e0, a.A, f.n_el, rd, nv);
+  flat_load<T, V, U, true>(x + n * a.E + f.e0, a.A, f.n_el, U, rx, nv);
+  flat_load<T, V, U, true>(dy + n * a.E + f.e0, a.A, f.n_el, U, rd, nv);
   op.keep(n, params);
   __syncthreads();
   {
@@ -881,7 +920,7 @@ cl_flat_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __re
     flat_forget(rx);
     flat_forget(rd);
     const typename FlatBwdOp<T, V>::Coef k = op.coef();
-    flat_store<T, V, U>(dx + n * a.E + f.e0, a.A, nv, [&](int u) { return k(flat_pack<T, V>(rx[u]), flat_pack<T, V>(rd[u])); });
+    flat_store<T, V, U>(dx + n * a.E + f.e0, a.A, U, nv, [&](int u) { return k(flat_pack<T, V>(rx[u]), flat_pack<T, V>(rd[u])); });
   }
   asm volatile("" ::: "memory");  // (asked for again, so that nothing of the slab lives across the call)
   if (flat_uniform(sm.fail) != 0) {

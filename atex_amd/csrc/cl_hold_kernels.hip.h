@@ -131,7 +131,12 @@ struct HoldLane {
   // batch b of pass p
   template <bool LAST>
   __device__ __forceinline__ void load(u32x4 (&ring)[Q], int p, int b, const T* src) const {
-    unsigned o = at(p, b);
+    load_from<LAST>(ring, p < P ? HA + p * Q : U - Q, b, src);
+  }
+  // batch b of the Q vectors from the u-th on
+  template <bool LAST>
+  __device__ __forceinline__ void load_from(u32x4 (&ring)[Q], int u, int b, const T* src) const {
+    unsigned o = from(u + b * B);
 #pragma unroll
     for (int i = 0; i < B; ++i) {
       if (b == NB - 1 && i == B - 1) o = o < end ? o : end;
@@ -170,6 +175,26 @@ struct HoldLane {
     }
     __builtin_amdgcn_sched_barrier(0);
   }
+  // All U vectors in passes of Q, in order, through the registers of one: batch(u, b) has the b-th batch from
+  // the u-th vector on, last(b) that of the last pass.  ring(f): f(registers, where they come from) for all arrays.
+  template <bool LAST, typename Ring, typename Batch, typename Last>
+  __device__ __forceinline__ void through(Ring&& ring, Batch&& batch, Last&& last) const {
+    auto load = [&](int u, int b) { ring([&](u32x4 (&r)[Q], const T* src) { load_from<LAST>(r, u, b, src); }); };
+    const int main = HA + P * Q;  // vectors before the last pass
+#pragma unroll
+    for (int b = 0; b < NB; ++b) load(0, b);
+#pragma unroll 1
+    for (int u = 0; u < main; u += Q) {
+#pragma unroll
+      for (int b = 0; b < NB; ++b) {
+        batch(u, b);
+        load(u + Q < main ? u + Q : U - Q, b);
+      }
+    }
+    ring([&](u32x4 (&r)[Q], const T*) { settle(r[Q - 1]); });
+#pragma unroll
+    for (int b = 0; b < NB; ++b) last(b);
+  }
   // N vectors from the u-th on
   template <int N, typename Value>
   __device__ __forceinline__ void store_own(int u, T* dst, Value&& value) const {
@@ -184,31 +209,55 @@ struct HoldLane {
 };
 
 // ------------------------------------------------------------------------------ forward
+// One batch after another.
 template <typename T, int V, int B>
+__device__ __forceinline__ void hold_stats_now(const u32x4* batch, int skip, int nv, float& n, float (&m)[V], float (&q)[V]) {
+  hold_stats<T, V, B, B>(skip, nv, [&](int u) { return flat_pack<T, V>(batch[u]); }, n, m, q);
+  hold_now(m);
+  hold_now(q);
+}
+
+template <typename T, int V, int HA, int Q, bool LDS, int B>
 struct HoldFwdOp : FlatFwdOp<T, V> {
-  int main;  // vectors before the last pass
-  // through memory, in the kernel's order
+  HoldArgs h;
+  using Lane = HoldLane<T, V, HA, Q, LDS, B>;
+  // in the kernel's order, in passes through one pass's registers
   __device__ __forceinline__ void sums(int64_t n, int l) const {
     const FlatArgs& a = this->a;
     const FlatSlab f = flat_slab<V>(a, l);
-    const T* src = this->x + n * a.E + f.e0;
-    const int U = this->U, nv = flat_valid(a.A, V, U, f.n_el);
+    const T* const src = this->x + n * a.E + f.e0;
+    const Lane w(a, h, f.n_el);
+    u32x4 r[Q];
     float m[V], q[V], cnt = 0.f;
 #pragma unroll
     for (int i = 0; i < V; ++i) m[i] = q[i] = 0.f;
-#pragma unroll 1
-    for (int u0 = 0; u0 < U;) {
-      const int k = u0 < main ? B : (U - u0 - 1) % B + 1;  // (the last pass's batches count from its end)
-      hold_stats<T, V, B, 1>(B - k, u0 + k == U ? nv : V, [&](int u) { return flat_vector<T, V>(src, a.A, u0 + u - (B - k), U, nv); }, cnt, m, q);
-      u0 += k;
-    }
-    flat_merge_stats<V>(a, f, flat_pixels(a, l), U, m, q, this->nt, this->lds,
+    w.template through<false>([&](auto&& f) { f(r, src); },
+                              [&](int, int b) { hold_stats_now<T, V, B>(r + b * B, 0, V, cnt, m, q); },
+                              [&](int b) {
+                                const int skip = w.skip - b * B;
+                                if (skip < B) hold_stats_now<T, V, B>(r + b * B, skip > 0 ? skip : 0, b == Lane::NB - 1 ? w.nv : V, cnt, m, q);
+                              });
+    flat_merge_stats<V>(a, f, flat_pixels(a, l), h.U, m, q, this->nt, this->lds,
                         [&](int c, float cm, float cq) { this->publish(n, l, c, cm, cq); });
+  }
+  __device__ __forceinline__ void apply(int64_t n, int l) const {
+    const FlatArgs& a = this->a;
+    const FlatSlab f = flat_slab<V>(a, l);
+    const T* const src = this->x + n * a.E + f.e0;
+    T* const dst = this->y + n * a.E + f.e0;
+    const Lane w(a, h, f.n_el);
+    const typename FlatFwdOp<T, V>::Coef coef = this->coef();
+    if (static_cast<int>(threadIdx.x) >= a.A) return;
+    u32x4 r[Q];
+    auto value = [&](int i) { return coef(flat_pinned<T, V>(flat_pack<T, V>(r[i]))); };
+    w.template through<true>([&](auto&& f) { f(r, src); },
+                             [&](int u, int b) { w.template store_own<B>(u + b * B, dst, [&](int i) { return value(b * B + i); }); },
+                             [&](int b) { w.store(w.P, b, dst, value); });
   }
 };
 
-template <typename T, int V, int B>
-__device__ __attribute__((noinline)) void hold_fwd_alone(const HoldFwdOp<T, V, B>* op, FlatShared* sm, int64_t n, int s) {
+template <typename Op>
+__device__ __attribute__((noinline)) void hold_fwd_alone(const Op* op, FlatShared* sm, int64_t n, int s) {
   flat_alone<true>(op->a, *op, *sm, op->nt, op->tag, n, s);
 }
 
@@ -241,11 +290,7 @@ cl_hold_fwd(const T* __restrict__ x, const float* __restrict__ gamma, const floa
   float m[V], q[V], cnt = 0.f;
 #pragma unroll
   for (int i = 0; i < V; ++i) m[i] = q[i] = 0.f;
-  auto stats = [&](const u32x4* batch, int skip, int nv) {
-    hold_stats<T, V, B, B>(skip, nv, [&](int u) { return flat_pack<T, V>(batch[u]); }, cnt, m, q);
-    hold_now(m);
-    hold_now(q);
-  };
+  auto stats = [&](const u32x4* batch, int skip, int nv) { hold_stats_now<T, V, B>(batch, skip, nv, cnt, m, q); };
 #pragma unroll
   for (int u = 0; u < HA; u += B) stats(own + u, 0, V);
   if constexpr (LDS) {
@@ -303,12 +348,78 @@ cl_hold_fwd(const T* __restrict__ x, const float* __restrict__ gamma, const floa
   asm volatile("" ::: "memory");  // (asked for again, so that nothing of the slab lives across the call)
   if (flat_uniform(sm.fail) != 0) {
     const FlatArgs args = a;
-    const HoldFwdOp<T, V, B> copy{{args, x, gamma, beta, y, mean_out, rstd_out, eps, nt, h.U, tag, flat_lds}, HA + (LDS ? Q : 0) + h.R};
-    hold_fwd_alone<T, V, B>(&copy, &sm, n, s);
+    const HoldFwdOp<T, V, HA, Q, LDS, B> copy{{args, x, gamma, beta, y, mean_out, rstd_out, eps, nt, h.U, tag, flat_lds}, h};
+    hold_fwd_alone(&copy, &sm, n, s);
   }
 }
 
 // ----------------------------------------------------------------------------- backward
+// One pair of vectors after another (flat_lane_sums).
+template <typename T, int V>
+__device__ __forceinline__ void hold_sums_now(const u32x4& bx, const u32x4& bd, const float (&mu)[V], float (&b)[V], float (&s)[V]) {
+#pragma clang fp contract(off)
+  const float one = mix_one();
+  const Pack<T, V> vx = flat_pack<T, V>(bx), vd = flat_pack<T, V>(bd);
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    b[i] = __builtin_fmaf(to_f32(vd.v[i]), sub_f32<T>(vx.v[i], mu[i], one), b[i]);
+    s[i] = add_f32<T>(s[i], vd.v[i], one);
+  }
+  hold_now(b);
+  hold_now(s);
+}
+
+template <typename T, int V, int HA, int Q, bool LDS, int B>
+struct HoldBwdOp : FlatBwdOp<T, V> {
+  HoldArgs h;
+  using Lane = HoldLane<T, V, HA, Q, LDS, B>;
+  // in the kernel's order, in passes through one pass's registers
+  __device__ __forceinline__ void sums(int64_t n, int l) const {
+    const FlatArgs& a = this->a;
+    const FlatSlab f = flat_slab<V>(a, l);
+    const T* const sx = this->x + n * a.E + f.e0;
+    const T* const sd = this->dy + n * a.E + f.e0;
+    const Lane w(a, h, f.n_el);
+    u32x4 rx[Q], rd[Q];
+    float mu[V], b[V], d[V];
+    this->means(mu);
+#pragma unroll
+    for (int i = 0; i < V; ++i) b[i] = d[i] = 0.f;
+    w.template through<false>([&](auto&& f) { f(rx, sx); f(rd, sd); },
+                              [&](int, int k) {
+#pragma unroll
+                                for (int r = k * B; r < (k + 1) * B; ++r) hold_sums_now<T, V>(rx[r], rd[r], mu, b, d);
+                              },
+                              [&](int k) {
+#pragma unroll
+                                for (int r = k * B; r < (k + 1) * B; ++r) {
+                                  if (r >= w.skip) hold_sums_now<T, V>(rx[r], rd[r], mu, b, d);
+                                }
+                              });
+    flat_merge_sums<V>(a, b, d, this->nt, this->lds, [&](int c, float cb, float cd) { this->publish(n, l, c, cb, cd); });
+  }
+  __device__ __forceinline__ void apply(int64_t n, int l) const {
+    const FlatArgs& a = this->a;
+    const FlatSlab f = flat_slab<V>(a, l);
+    const T* const sx = this->x + n * a.E + f.e0;
+    const T* const sd = this->dy + n * a.E + f.e0;
+    T* const dst = this->dx + n * a.E + f.e0;
+    const Lane w(a, h, f.n_el);
+    const typename FlatBwdOp<T, V>::Coef coef = this->coef();
+    if (static_cast<int>(threadIdx.x) >= a.A) return;
+    u32x4 rx[Q], rd[Q];
+    auto value = [&](int i) { return coef(flat_pinned<T, V>(flat_pack<T, V>(rx[i])), flat_pinned<T, V>(flat_pack<T, V>(rd[i]))); };
+    w.template through<true>([&](auto&& f) { f(rx, sx); f(rd, sd); },
+                             [&](int u, int k) { w.template store_own<B>(u + k * B, dst, [&](int i) { return value(k * B + i); }); },
+                             [&](int k) { w.store(w.P, k, dst, value); });
+  }
+};
+
+template <typename Op>
+__device__ __attribute__((noinline)) void hold_bwd_alone(const Op* op, FlatShared* sm, int64_t n, int s) {
+  flat_alone<false>(op->a, *op, *sm, op->nt, op->tag, n, s);
+}
+
 template <typename T, int V, int HA, int Q, bool LDS, int B>
 __global__ void __launch_bounds__(kFlatMaxThreads, 2)
 cl_hold_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __restrict__ gamma,
@@ -346,18 +457,7 @@ cl_hold_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __re
   op.means(mu);
 #pragma unroll
   for (int i = 0; i < V; ++i) sb[i] = ss[i] = 0.f;
-  const float one = mix_one();
-  auto sums = [&](const u32x4& bx, const u32x4& bd) {
-#pragma clang fp contract(off)
-    const Pack<T, V> vx = flat_pack<T, V>(bx), vd = flat_pack<T, V>(bd);
-#pragma unroll
-    for (int i = 0; i < V; ++i) {  // (flat_lane_sums)
-      sb[i] = __builtin_fmaf(to_f32(vd.v[i]), sub_f32<T>(vx.v[i], mu[i], one), sb[i]);
-      ss[i] = add_f32<T>(ss[i], vd.v[i], one);
-    }
-    hold_now(sb);
-    hold_now(ss);
-  };
+  auto sums = [&](const u32x4& bx, const u32x4& bd) { hold_sums_now<T, V>(bx, bd, mu, sb, ss); };
 #pragma unroll
   for (int u = 0; u < HA; ++u) sums(ox[u], od[u]);
   if constexpr (LDS) {
@@ -423,8 +523,8 @@ cl_hold_bwd(const T* __restrict__ dy, const T* __restrict__ x, const float* __re
   asm volatile("" ::: "memory");  // (asked for again, so that nothing of the slab lives across the call)
   if (flat_uniform(sm.fail) != 0) {
     const FlatArgs args = a;
-    const FlatBwdOp<T, V> copy{args, dy, x, gamma, mean_in, rstd_in, dx, o0, o1, o_stride, nt, h.U, tag, flat_lds};
-    flat_bwd_alone<T, V>(&copy, &sm, n, s);
+    const HoldBwdOp<T, V, HA, Q, LDS, B> copy{{args, dy, x, gamma, mean_in, rstd_in, dx, o0, o1, o_stride, nt, h.U, tag, flat_lds}, h};
+    hold_bwd_alone(&copy, &sm, n, s);
   }
 }
 

@@ -192,6 +192,27 @@ def _median_us(call, before, reps=7):
     return float(np.median(times[1:]))
 
 
+def _stream_beside(L):
+    """A stream whose work runs beside the current stream's (streams share a few hardware queues)."""
+    import torch
+
+    word = torch.zeros(1, device="cuda")
+    for _ in range(16):
+        side = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        assert L.atexn_bench_occupy(1, 5.0, side.cuda_stream) == 0
+        over, here = torch.cuda.Event(), torch.cuda.Event()
+        over.record(side)
+        word.add_(1.0)
+        here.record()
+        here.synchronize()
+        beside = not over.query()
+        torch.cuda.synchronize()
+        if beside:
+            return side
+    raise AssertionError("no stream runs beside the current one")
+
+
 def _channels_last_calls(capi, N, S, C, dtype):
     import torch
 
@@ -205,8 +226,55 @@ def _channels_last_calls(capi, N, S, C, dtype):
 
 
 # held instances one and two at a time, flat ones on one XCD each and over all of them
-@pytest.mark.parametrize("N,S,C,dtype", [(2, 2097152, 32, "f16"), (8, 524288, 32, "f16"), (1, 385517, 144, "f32"),
-                                         (36, 36288, 29, "bf16"), (1, 598464, 17, "f16")])
+HELD_AND_FLAT = [(2, 2097152, 32, "f16"), (8, 524288, 32, "f16"), (1, 385517, 144, "f32"), (36, 36288, 29, "bf16"),
+                 (1, 598464, 17, "f16")]
+
+
+@pytest.mark.parametrize("N,S,C,dtype", HELD_AND_FLAT)
+def test_held_and_flat_instances_beside_the_occupier(N, S, C, dtype):
+    """One CU taken is enough for held instances never to be on the chip together.  The bits of a run alone; and
+    the workgroups that are there share out what is missing in at most three times the duration of the slab
+    kernels, which need no company (each walking through an instance's slabs on its own: 5 to 10 times)."""
+    import torch
+
+    capi = util.Capi(bench=True)
+    L = capi.L
+    calls = _channels_last_calls(capi, N, S, C, dtype)
+    side = _stream_beside(L)
+    alone = [call() for call in calls]
+    torch.cuda.synchronize()
+    switches = (b"cl_hold", b"cl_flat", b"cl_single")
+    try:
+        assert L.atexn_bench_mark_exchange_trouble(0) == 0
+        for wgs in (1, 192):
+            def occupy():
+                assert L.atexn_bench_occupy(wgs, 8.0, side.cuda_stream) == 0
+
+            for what, call, want in zip(("forward", "backward"), calls, alone):
+                for _ in range(2):
+                    torch.cuda.synchronize()
+                    occupy()
+                    torch.cuda._sleep(400000)  # the occupier gets its CUs first
+                    got = call()
+                    torch.cuda.synchronize()
+                    for a, b in zip(got, want):
+                        assert torch.equal(_bits(a), _bits(b)), f"{what} beside {wgs} occupied CUs differs"
+                shared = _median_us(call, occupy)
+                for s in switches:
+                    assert L.atexn_set_tuning(s, 0) == 0
+                slabs = _median_us(call, occupy)
+                for s in switches:
+                    assert L.atexn_set_tuning(s, 1) == 0
+                print(f"{what} [{N}, {S}, {C}] {dtype} beside {wgs}: {shared:.1f} us, slab kernels {slabs:.1f} us", flush=True)
+                assert shared < 3.0 * slabs + 20.0, f"{what} beside {wgs} occupied CUs"
+    finally:
+        torch.cuda.synchronize()
+        for s in switches:
+            L.atexn_set_tuning(s, 1)
+        L.atexn_bench_mark_exchange_trouble(0)
+
+
+@pytest.mark.parametrize("N,S,C,dtype", HELD_AND_FLAT)
 def test_waits_cut_short_find_peers_that_are_running(N, S, C, dtype):
     """After a wait that ran out, on a GPU that is free again: slabs of hundreds of KB end microseconds apart,
     and a wait cut short still lasts that long (or every workgroup redoes its peers' work: 4 to 6 times the
