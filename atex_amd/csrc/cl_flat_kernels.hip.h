@@ -41,11 +41,12 @@ constexpr int kFlatMaxThreads = 512;
 constexpr int kFlatMaxSlabs = 512;
 constexpr int kFlatFwdMost = 16, kFlatBwdMost = 8;  // vectors per thread
 constexpr int kFlatOwnPolls = 1 << 16;  // for values known to be published: bounds the wait only
-// Polls of a wait that is cut short (exchange_wait_pair).  The slabs of an instance that is on the chip
-// together end some microseconds apart, the more the larger they are: after 24 polls of about 0.15 us most
-// workgroups of held instances took running peers for absent ones (fp16 [2, 128^3, 32] on a free GPU, forward
-// 121 us -> 570, backward [8, 524288, 32] 175 -> 1078), after 48 some still did, after 99 none.
-constexpr int kFlatHastyPolls = 160;
+// How long a wait lasts, in polls of about 0.15 us (exchange_wait_pair), besides one for each vector of a thread:
+// the slabs of an instance that is on the chip together end the further apart the larger they are.  After 24
+// polls most workgroups of held instances took running peers for absent ones (fp16 [2, 128^3, 32], 64 vectors, on
+// a free GPU with waits cut short: forward 121 us -> 570), 99 were enough there, 159 for 128 vectors, not 300 for
+// 512 and 1024 (backward [1, 2^24, 64] bf16 2230 us, 1880 with 600), 600 were.
+constexpr int kFlatHastyPolls = 112;
 
 // A value that is the same in every thread, as the compiler's scalar: a branch on it keeps no copy of the
 // held vectors for lanes that might not take it.
@@ -60,6 +61,7 @@ struct FlatArgs {
   float inv_d;         // 1 / D
   float px_more, px_base, px_last;  // pixels of the last `extra` slabs, of the others, of the very last one
   int local;           // the slabs of an instance on one XCD
+  int hasty;           // polls of a wait that is cut short
   int k_at;            // where in LDS the channels' parameters, then constants, are: behind the sums
   ExchangeArgs ex;
   cl_word* tagged;      // [N][S][C] pairs: the slabs' sums
@@ -379,7 +381,7 @@ __device__ __forceinline__ bool flat_fold(const FlatArgs& a, unsigned tag, int64
   const unsigned col = want ? 2u * c : 0u;
   const bool mine = want && sub < a.S;
   float p, q;
-  if (!exchange_wait_pair(at + (mine ? sub * stride + col : 0u), mine, tag, polls, trouble, p, q, kFlatHastyPolls)) return false;
+  if (!exchange_wait_pair(at + (mine ? sub * stride + col : 0u), mine, tag, polls, trouble, p, q, a.hasty)) return false;
   r0 = flat_group_sum(mine ? (STATS ? p * flat_pixels(a, sub) : p) : 0.f, a.width);
   if constexpr (STATS) {
     r0 *= a.inv_d;
@@ -409,7 +411,7 @@ __device__ __forceinline__ bool flat_fold_wide(const FlatArgs& a, unsigned tag, 
     const int l = static_cast<int>(threadIdx.x) + r * nt;
     if (ok && r * nt < a.S) {  // (wave-uniform)
       ok = exchange_wait_pair(at + (l < a.S ? l * stride : 0u), l < a.S, tag, polls, trouble, p[r], q[r],
-                              kFlatHastyPolls);
+                              a.hasty);
       s0 += l < a.S ? (STATS ? p[r] * flat_pixels(a, l) : p[r]) : 0.f;
       if constexpr (!STATS) s1 += l < a.S ? q[r] : 0.f;
     }
@@ -511,7 +513,7 @@ __device__ __forceinline__ bool flat_finals(const FlatArgs& a, Op& op, int nt, u
     const int c = c0 + lane;
     float r0, r1;
     fail = !exchange_wait_pair(a.finals + (n * a.C + (c < a.C ? c : 0)) * 2, c < a.C, tag, polls, trouble, r0, r1,
-                               kFlatHastyPolls);
+                               a.hasty);
     if (CERTAIN && fail) {
       r0 = r1 = __builtin_nanf("");
       fail = false;

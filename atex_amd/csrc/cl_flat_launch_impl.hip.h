@@ -31,7 +31,9 @@ inline FlatArgs flat_args(const FlatPlan& p, int64_t N, int64_t C, int64_t D, vo
   a.px_last = static_cast<float>(D - (int64_t(p.S - 1) * p.base + std::max(p.extra - 1, 0)) * p.pix);
   a.local = p.local;
   a.k_at = p.k_at;
-  a.ex = ExchangeArgs{e.tag, e.at, tuning().cl_flat_polls, e.trouble};
+  const int polls = tuning().cl_flat_polls;
+  a.ex = ExchangeArgs{e.tag, e.at, polls < kExchangePatientPolls ? polls : polls + p.U, e.trouble};
+  a.hasty = kFlatHastyPolls + p.U;
   a.tagged = reinterpret_cast<cl_word*>(w + p.off_tagged);
   a.finals = reinterpret_cast<cl_word*>(w + p.off_finals);
   a.claims = reinterpret_cast<unsigned*>(w + p.off_claims);

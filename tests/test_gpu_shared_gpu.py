@@ -291,6 +291,27 @@ def test_waits_cut_short_find_peers_that_are_running(N, S, C, dtype):
         capi.L.atexn_bench_mark_exchange_trouble(0)
 
 
+@pytest.mark.parametrize("N,S,C,dtype", [(2, 2097152, 32, "f32"), (1, 1 << 24, 64, "bf16")])
+def test_patience_grows_with_the_slabs(N, S, C, dtype):
+    """Instances of 268 MB and 2 GB on a free GPU: nobody runs out of a wait, cut short or not, whose slab is merely
+    large (a fifth more time where some did; a tenth is allowed)."""
+    capi = util.Capi(bench=True)
+    L = capi.L
+    calls = _channels_last_calls(capi, N, S, C, dtype)
+    try:
+        for what, call in zip(("forward", "backward"), calls):
+            assert L.atexn_set_tuning(b"cl_flat_polls", 10000) == 0
+            endless = _median_us(call, lambda: L.atexn_bench_mark_exchange_trouble(0))
+            assert L.atexn_set_tuning(b"cl_flat_polls", 300) == 0
+            patient = _median_us(call, lambda: L.atexn_bench_mark_exchange_trouble(0))
+            short = _median_us(call, lambda: L.atexn_bench_mark_exchange_trouble(1))
+            print(f"{what} [{N}, {S}, {C}] {dtype}: {endless:.1f} us, patient {patient:.1f}, cut short {short:.1f}", flush=True)
+            assert max(patient, short) < 1.1 * endless, what
+    finally:
+        L.atexn_set_tuning(b"cl_flat_polls", 300)
+        L.atexn_bench_mark_exchange_trouble(0)
+
+
 def test_the_occupier_leaves_in_time():
     import time
 
