@@ -388,7 +388,12 @@ int rows_bwd_v(const T* dy, const T* x, const float* gamma, const float* mean, c
   float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + p.off_part);
   const int64_t W = AFF ? C : D;
   if constexpr (!AFF && V > 1) {
-    if (p.lr.on && static_cast<const void*>(dx) != static_cast<const void*>(dy) && bwd_stage_mask() == 3) {
+    const bool one_launch = static_cast<const void*>(dx) != static_cast<const void*>(dy) && bwd_stage_mask() == 3;
+    if (one_launch) {
+      const PairPlan pair = plan_pair(V, n_rows, D);
+      if (pair.on) return pair_bwd_launch<T>(pair, dy, x, gamma, mean, rstd, n_rows, D, dx, dgamma, dbeta, st);
+    }
+    if (p.lr.on && one_launch) {
       ExchangeTag tag;
       ATEXN_TRY(exchange_tag(st, static_cast<char*>(ws) + p.lr.off_tag, tag));
       if (tag.ok) return long_rows_bwd_launch<T>(p.lr, tag, dy, x, gamma, mean, rstd, n_rows, D, dx, dgamma, dbeta, ws, st);
@@ -546,10 +551,6 @@ int rows_bwd_t(bool affine, const void* dy_, const void* x_, const float* gamma,
   }
   if (route.tiles) {
     return tiles_bwd<T>(dy, x, gamma, mean, rstd, n_rows, D, dx, dgamma, dbeta, ws, ws_bytes, st);
-  }
-  if (!affine && route.V > 1 && static_cast<const void*>(dx) != static_cast<const void*>(dy) && bwd_stage_mask() == 3) {
-    const PairPlan p = plan_pair(VEC, n_rows, D);
-    if (p.on) return pair_bwd_launch<T>(p, dy, x, gamma, mean, rstd, n_rows, D, dx, dgamma, dbeta, st);
   }
   if (route.V > 1) {
     return affine ? rows_bwd_v<T, VEC, true>(dy, x, gamma, mean, rstd, n_rows, D, C, dx, dgamma, dbeta, ws, ws_bytes, st)

@@ -227,6 +227,12 @@ def test_kernel_level_validation(L):
     assert L.atexn_layer_norm_bwd(1, FAKE, 0x2000, FAKE, FAKE, FAKE, 8192, 1024, 0x3000, FAKE, FAKE,
                                   0x4000, need - 256, None) == 1
     assert b"workspace too small" in L.atexn_last_error()
+    for rows, cols in ((32, 1024), (768, 4104)):  # (the launch that these take leaves the workspace alone)
+        need = L.atexn_layer_norm_bwd_workspace_bytes(1, rows, cols)
+        assert need > 0
+        assert L.atexn_layer_norm_bwd(1, FAKE, 0x2000, FAKE, FAKE, FAKE, rows, cols, 0x3000, FAKE, FAKE,
+                                      0x4000, need - 256, None) == 1
+        assert b"workspace too small" in L.atexn_last_error()
     # the product library has no process-wide settings at all
     assert not hasattr(L, "atexn_set_tuning")
     # the static-scratch backward refuses what does not fit its buffer before it touches a device
