@@ -55,6 +55,43 @@ def test_few_rows_in_one_launch(coracle, N, D, dtype):
     check(capi.ln_bwd(dyd, xd, gd, m, r, dtype, dx=dyd))  # in place: the row kernels
 
 
+@pytest.mark.parametrize("N,D,dtype", [(32, 1024, "f16"), (512, 4096, "bf16"), (200, 2051, "f32")])
+def test_gradients_over_the_weights_keep_the_row_kernels(N, D, dtype):
+    """dgamma written over gamma (dbeta over gamma, or into its second half): the bits of the row kernels, which
+    write them when everything is read."""
+    import torch
+
+    capi = util.Capi(bench=True)
+    L, code = capi.L, O.DTYPE_CODE[dtype]
+    x, gamma, beta, dy = util.ln_inputs("plain", N, D, dtype, 141)
+    xd, dyd, gd = util.to_device(x, dtype), util.to_device(dy, dtype), torch.from_numpy(gamma).cuda()
+    _, m, r = capi.ln_fwd(xd, gd, torch.from_numpy(beta).cuda(), EPS, dtype)
+    need = L.atexn_layer_norm_bwd_workspace_bytes(code, N, D)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+
+    def run(place):
+        buf = torch.zeros(3 * D, device="cuda")
+        buf[:D] = gd
+        dx = torch.empty_like(xd)
+        dg, db = (buf[o:o + D] for o in place)
+        assert L.atexn_layer_norm_bwd(code, dyd.data_ptr(), xd.data_ptr(), buf.data_ptr(), m.data_ptr(), r.data_ptr(), N, D,
+                                      dx.data_ptr(), dg.data_ptr(), db.data_ptr(), ws.data_ptr(), need,
+                                      torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return dx, dg.clone(), db.clone()
+
+    try:
+        assert L.atexn_set_tuning(b"pair_rows", 0) == 0
+        want = run((D, 2 * D))
+    finally:
+        assert L.atexn_set_tuning(b"pair_rows", 1) == 0
+    print(f"dgamma / dbeta over gamma N={N} D={D} {dtype}", flush=True)
+    assert not all(bool((a == b).all()) for a, b in zip(run((D, 2 * D)), want))  # (rows_bwd_pair sums differently)
+    for place in ((0, D), (D, 0), (D // 2, 2 * D)):
+        for name, a, b in zip(("dx", "dgamma", "dbeta"), run(place), want):
+            assert bool((a == b).all()), f"{place}: {name}"
+
+
 def test_more_rows_stay_on_the_row_kernels():
     capi = util.Capi(bench=True)
     for N, D, dtype in ((1025, 64, "f16"), (513, 1024, "f16"), (769, 8192, "f16"), (513, 8192, "f32"), (8, 16392, "f16")):
