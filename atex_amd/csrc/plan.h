@@ -1057,19 +1057,25 @@ inline ClPlan plan_cl_slabs(bool bwd, int V, int64_t N, int64_t C, int64_t D, in
 // [15, 5488, 104] 24.7 -> 17.5; [12, 3408, 448] 27.9 -> 29.2, [11, 20592, 128] 35.6 -> 37.9); and where even
 // the kernels of resident slabs need several rounds, both ways ([33, 23808, 64] bf16 55.9 / 89.1 ->
 // 39.2 / 77.3, [36, 30000, 32] 35.9 / 58.0 -> 26.9 / 50.2; [32, 6976, 64] 15.0 -> 15.1).
-inline bool flat_instead(const ClPlan& p, const FlatPlan& f, bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
-  if (!f.on || p.fused || f.S < 2) return false;
-  if (int64_t(f.S) * 32 > D) return false;  // a slab's pairs: more than a sixteenth (f32: an eighth) of its bytes
+// The sizes alone, asked first: most calls stay on plan p, and a step plans four times (the plans that were made
+// and then refused cost a call of [8, 16384, 64] 0.13 us beside the 0.065 of its own).
+inline bool flat_may(const ClPlan& p, bool bwd, int V, int64_t N, int64_t C, int64_t D) {
+  if (p.fused || V == 1) return false;
   const int64_t x2 = N * C * D / (V / 2) >> 16;  // MiB of x, times two
+  if (C % V != 0 && V == 8) return x2 >= (bwd ? 14 : (N >= kPlanXcdCount ? 4 : 10));
+  if (C > 128) return false;
+  return !bwd && !p.single ? x2 >= 40 : V == 8 && p.single && C <= 64 && x2 >= 96;
+}
+inline bool flat_instead(const ClPlan& p, const FlatPlan& f, bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+  if (!f.on || f.S < 2 || !flat_may(p, bwd, V, N, C, D)) return false;
+  if (int64_t(f.S) * 32 > D) return false;  // a slab's pairs: more than a sixteenth (f32: an eighth) of its bytes
   const int64_t slots = int64_t(cus) * (1024 / f.threads);
   if (C % V != 0 && V == 8) {
-    if (bwd) return f.local && x2 >= 14 && (f.grid <= slots || C <= 64 || (C <= 160 && f.grid * 20 > slots * 23));
-    if (f.local) return N >= kPlanXcdCount && x2 >= 4;
-    return x2 >= 10 && (f.grid <= slots ? C <= 300 : C <= 80 && f.grid <= slots * 2);
+    if (bwd) return f.local && (f.grid <= slots || C <= 64 || (C <= 160 && f.grid * 20 > slots * 23));
+    if (f.local) return N >= kPlanXcdCount;
+    return N * C * D >= (int64_t(10) << 18) && (f.grid <= slots ? C <= 300 : C <= 80 && f.grid <= slots * 2);
   }
-  if (!f.local || C > 128 || (f.grid > slots && f.grid * 2 < slots * 3)) return false;
-  if (!bwd && !p.single) return x2 >= 40;
-  return V == 8 && p.single && C <= 64 && x2 >= 96;
+  return f.local && (f.grid <= slots || f.grid * 2 >= slots * 3);
 }
 
 // Whether that is better than the flat kernels or those of plan_cl_slabs.  (times: those, hold; us)
@@ -1085,27 +1091,31 @@ inline bool flat_instead(const ClPlan& p, const FlatPlan& f, bool bwd, int V, in
 // [9, 72447, 32] bf16, of 4.6 MB, 27.2, 20.8; [16, 65536, 64], of 8 MiB, 65, 51); not in place of the single
 // launch on one XCD where that is whole or fp32 ([5, 15779, 192] fp32 23.7, 30.6), nor with several instances one
 // at a time that leave the chip part empty ([3, 100000, 300] bf16 104, 121; [2, 85000, 133] fp16 28.5, 37.8).
-inline bool hold_instead(const ClPlan& p, const FlatPlan& h, bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
-  if (!h.on || int64_t(h.S) * 128 > D) return false;
+inline bool hold_may(const ClPlan& p, bool bwd, int V, int64_t N, int64_t C, int64_t D) {  // (the sizes alone)
+  if (V == 1 || C > kPlanFlatMaxThreads) return false;
   const int64_t inst = C * D * 16 / V, x = N * inst;
+  if (bwd) return x >= (int64_t(17) << 20) && (inst >= (int64_t(1) << 20) || C <= 64);
+  return x >= (int64_t(24) << 20) && inst > (int64_t(4) << 20) && !(p.single && (V == 4 || !p.single_xm || p.xm_resident));
+}
+inline bool hold_instead(const ClPlan& p, const FlatPlan& h, bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
+  if (!h.on || !hold_may(p, bwd, V, N, C, D) || int64_t(h.S) * 128 > D) return false;
   if (bwd) {
     const int64_t xcd_slots = int64_t(cus) / kPlanXcdCount * (1024 / std::max(p.flat.threads, 1));
     if (p.single && !p.flat.on && p.TPP * p.CT == p.CV && N * p.CT % kPlanXcdCount == 0) return false;
     if (p.flat.on && p.flat.local && h.R > 0 && N % kPlanXcdCount == 0 && xcd_slots % p.flat.S == 0) return false;
-    return x >= (int64_t(17) << 20) && (inst >= (int64_t(1) << 20) || C <= 64) && (C < 256 || h.U >= 30);
+    return C < 256 || h.U >= 30;
   }
-  if (p.single && (V == 4 || !p.single_xm || p.xm_resident)) return false;
-  return x >= (int64_t(24) << 20) && inst > (int64_t(4) << 20) && (N == 1 || h.threads == 256 || h.U >= 40);
+  return N == 1 || h.threads == 256 || h.U >= 40;
 }
 
 inline ClPlan plan_cl(bool bwd, int V, int64_t N, int64_t C, int64_t D, int cus) {
   ClPlan p = plan_cl_slabs(bwd, V, N, C, D, cus);
   const int how = tuning().cl_flat, hold = tuning().cl_hold;
-  if (how != 0 && (how == 2 || !(p.fused || N * C * D < (int64_t(1) << 19)))) {  // (flat_instead wants more)
+  if (how == 2 || (how != 0 && flat_may(p, bwd, V, N, C, D))) {
     const FlatPlan f = plan_flat(bwd, V, N, C, D, cus);
     if (how == 2 ? f.on : flat_instead(p, f, bwd, V, N, C, D, cus)) p.flat = f;
   }
-  if (hold != 0 && (hold == 2 || N * C * D * 16 / V >= (int64_t(17) << 20))) {  // (hold_instead wants more)
+  if (hold == 2 || (hold != 0 && hold_may(p, bwd, V, N, C, D))) {
     const FlatPlan h = plan_hold(bwd, V, N, C, D, cus);
     if (hold == 2 ? h.on : hold_instead(p, h, bwd, V, N, C, D, cus)) p.flat = h;
   }

@@ -74,7 +74,23 @@ static void check(bool hold, bool bwd, int V, int64_t N, int64_t C, int64_t D, i
   EXPECT(!c.flat.on || (c.ws_bytes >= c.flat.ws_bytes && c.ws_bytes >= plan_cl_slabs(bwd, V, N, C, D, cus).ws_bytes));
 }
 
+// Calls that stay on the slab kernels are told by their sizes, before a plan is made that would be refused.
+static void check_refused_early(int V, int64_t N, int64_t C, int64_t D) {
+  for (const bool bwd : {false, true}) {
+    const int cus = 256;
+    const ClPlan c = plan_cl(bwd, V, N, C, D, cus);
+    const FlatPlan& p = c.flat;
+    EXPECT(!p.on && !flat_may(c, bwd, V, N, C, D) && !hold_may(c, bwd, V, N, C, D));
+  }
+}
+
 int main() {
+  check_refused_early(8, 8, 64, 16384);
+  check_refused_early(8, 2, 320, 216);
+  check_refused_early(8, 100, 64, 2048 / 2);
+  check_refused_early(8, 24, 57, 800);
+  check_refused_early(4, 16, 64, 4096);
+  check_refused_early(4, 46, 60, 100);
   std::vector<int64_t> channels;
   for (int64_t c = 4; c <= 80; ++c) channels.push_back(c);
   for (int64_t c = 81; c <= 2100; c += c < 600 ? 5 : 61) channels.push_back(c);
