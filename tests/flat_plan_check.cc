@@ -88,7 +88,7 @@ int main() {
   check_refused_early(8, 8, 64, 16384);
   check_refused_early(8, 2, 320, 216);
   check_refused_early(8, 100, 64, 2048 / 2);
-  check_refused_early(8, 24, 57, 800);
+  check_refused_early(8, 5, 57, 800);
   check_refused_early(4, 16, 64, 4096);
   check_refused_early(4, 46, 60, 100);
   std::vector<int64_t> channels;
