@@ -1058,20 +1058,21 @@ inline ClPlan plan_cl_slabs(bool bwd, int V, int64_t N, int64_t C, int64_t D, in
 }
 
 // Whether the flat kernels take a call that would otherwise run plan p: the classes of drawn shapes where
-// they were faster (us of the old kernels against theirs).
+// they were faster (us of the other kernels -> theirs; fp16 where nothing else is said).
 // 16-bit pixels that are no whole number of vectors, which the other kernels read in overlapping pieces and
-// twice.  Forward from 2 MB of x ([22, 14280, 17] fp16 20.1 -> 11.2, [51, 7684, 87] bf16 49.1 -> 32.3,
-// [28, 1275, 162] 16.2 -> 13.5; [48, 304, 74], 2.2 MB with few pixels, 7.5 -> 9.0); over all XCDs from 5 MB and
-// while the pairs that are exchanged are few ([1, 598464, 17] 31.1 -> 20.2, [2, 85000, 133] 37.4 -> 32.4;
-// [4, 1664, 428] 14.4 -> 17.1, [3, 14016, 428] 31.0 -> 41.0, [5, 75264, 116] 48 -> 53).  Backward, which holds half as much and leaves
-// the fold over the instances to a launch, from 7 MB on one XCD each ([24, 9384, 57] 28.8 -> 20.4,
-// [36, 36288, 29] 104 -> 61; [50, 1248, 53], 6.6 MB, 13.3 -> 13.6), not where a few workgroups are left for
-// another round or there are several rounds of many channels ([20, 2920, 175] 26.8 -> 30.0, [11, 7104, 190]
-// 33.0 -> 39.5).
-// Other pixels: forward in place of two stages from 20 MB ([28, 92880, 16] 47.3 -> 34.3, f32
-// [15, 5488, 104] 24.7 -> 17.5; [12, 3408, 448] 27.9 -> 29.2, [11, 20592, 128] 35.6 -> 37.9); and where even
-// the kernels of resident slabs need several rounds, both ways ([33, 23808, 64] bf16 55.9 / 89.1 ->
-// 39.2 / 77.3, [36, 30000, 32] 35.9 / 58.0 -> 26.9 / 50.2; [32, 6976, 64] 15.0 -> 15.1).
+// twice.  Forward from 2 MB of x ([22, 14280, 17] 20.6 -> 11.4, [51, 7684, 87] bf16 49.5 -> 31.5,
+// [28, 1275, 162] 16.9 -> 12.4; [48, 304, 74], 2.2 MB with few pixels, 7.6 -> 8.3); over all XCDs from 5 MB and
+// while the pairs that are exchanged are few ([1, 598464, 17] 31.6 -> 18.6, [2, 85000, 133] 38.1 -> 29.4;
+// [4, 1664, 428] 14.6 -> 16.6, [3, 14016, 428] 31.1 -> 31.4, [5, 75264, 116] 53.3 -> 55.9).  Backward, which holds half
+// as much and leaves the fold over the instances to a launch, from 7 MB on one XCD each ([22, 14280, 17]
+// 22.9 -> 14.3, [38, 3328, 85] 30.7 -> 18.9; [50, 1248, 53], 6.6 MB, 13.4 -> 13.5), not where a few workgroups are
+// left for another round or there are several rounds of many channels ([20, 2920, 175] 27.1 -> 29.1,
+// [11, 7104, 190] 33.4 -> 38.8).  (What hold_instead has of these it takes.)
+// Other pixels: forward in place of two stages from 20 MB ([33, 23808, 64] bf16 56.0 -> 38.9, f32
+// [15, 5488, 104] 24.9 -> 17.5; [12, 3408, 448] 27.6 -> 28.7); and where even the kernels of resident slabs
+// need several rounds, both ways ([64, 16384, 64] bf16 65.8 / 86.3 -> 46.8 / 80.9, forward [32, 65536, 32]
+// 64.9 -> 44.8).  Not on grids of 1 to 1.5 rounds, where both happens: forward [11, 20592, 128] 36.4 -> 38.8, but
+// [28, 92880, 16] 47.4 -> 33.9 and [36, 30000, 32] 33.5 -> 26.8, which stay where they were.
 // The sizes alone, asked first: most calls stay on plan p, and a step plans four times (the plans that were made
 // and then refused cost a call of [8, 16384, 64] 0.13 us beside the 0.065 of its own).
 inline bool flat_may(const ClPlan& p, bool bwd, int V, int64_t N, int64_t C, int64_t D) {
@@ -1095,17 +1096,17 @@ inline bool flat_instead(const ClPlan& p, const FlatPlan& f, bool bwd, int V, in
 
 // Whether that is better than the flat kernels or those of plan_cl_slabs.  (times: those, hold; us)
 // A channel's pair costs 32 bytes a slab, written and read back: slabs of at least 128 pixels, whose channel is
-// 256 bytes in fp16 ([5, 15779, 192] fp32 on slabs of 123 backward 46, 56).  Backward: from 17 MiB
-// of x on ([1, 89514, 125] bf16 29.1, 21.4; [2, 12673, 124] fp32, 13 MB, 16.2, 19.5); not the smallest
-// instances of many channels ([38, 3168, 100] fp16 21.5, 22.7), nor 256 channels and more on short slabs
-// ([2, 50000, 320] fp16 52, 63; [3, 100000, 300] bf16 201, 154), nor where the flat kernels' slabs fill each
-// XCD exactly ([64, 16384, 64] bf16 81.5, 85.7; [36, 57624, 16] fp16, where they do not, 49, 40), nor in place of
+// 256 bytes in fp16 (backward [5, 15779, 192] fp32 on slabs of 154 46.8, 44.7, [3, 14016, 428] fp16 of 54 38.3,
+// 60.5).  Backward: from 17 MiB of x on ([1, 89514, 125] bf16 29.7, 21.7; [2, 12673, 124] fp32, 13 MB, 16.3, 20.0);
+// not the smallest instances of many channels ([38, 3168, 100] fp16 21.0, 23.2), nor 256 channels and more on short
+// slabs ([2, 50000, 320] fp16 52.4, 62.5; [3, 100000, 300] bf16 201, 153), nor where the flat kernels' slabs fill each
+// XCD exactly ([64, 16384, 64] bf16 80.9, 85.2; [36, 57624, 16] fp16, where they do not, 47.3, 39.7), nor in place of
 // the single launch on one XCD where all lanes have a vector and all XCDs the same work ([8, 16384, 64] fp32
-// 20.4, 25.5, [16, 8192, 128] fp16 24.4, 28.1; else [24, 16384, 48] bf16 34.6, 26.7, [20, 16384, 64] fp16 35, 28).  Forward: from
-// 24 MiB on and with instances beyond the 4 MiB that one XCD holds ([32, 65536, 32] fp16, of 4 MiB, 44, 48;
-// [9, 72447, 32] bf16, of 4.6 MB, 27.2, 20.8; [16, 65536, 64], of 8 MiB, 65, 51); not in place of the single
-// launch on one XCD where that is whole or fp32 ([5, 15779, 192] fp32 23.7, 30.6), nor with several instances one
-// at a time that leave the chip part empty ([3, 100000, 300] bf16 104, 121; [2, 85000, 133] fp16 28.5, 37.8).
+// 20.2, 26.0, [16, 8192, 128] fp16 24.7, 28.8; else [24, 16384, 48] bf16 35.2, 28.3, [20, 16384, 64] fp16 35.1, 30.0).
+// Forward: from 24 MiB on and with instances beyond the 4 MiB that one XCD holds ([32, 65536, 32] fp16, of 4 MiB,
+// 44.8, 47.5; [9, 72447, 32] bf16, of 4.6 MB, 27.5, 21.1; [16, 65536, 64], of 8 MiB, 64.7, 49.3); not in place of the
+// single launch on one XCD where that is whole or fp32 ([5, 15779, 192] fp32 23.8, 31.3), nor with several instances
+// one at a time that leave the chip part empty ([3, 100000, 300] bf16 105, 122; [2, 85000, 133] fp16 29.4, 37.8).
 inline bool hold_may(const ClPlan& p, bool bwd, int V, int64_t N, int64_t C, int64_t D) {  // (the sizes alone)
   if (V == 1 || C > kPlanFlatMaxThreads) return false;
   const int64_t inst = C * D * 16 / V, x = N * inst;

@@ -84,7 +84,57 @@ static void check_refused_early(int V, int64_t N, int64_t C, int64_t D) {
   }
 }
 
+// The kernels of shapes that the rules' comments quote, forward and backward: slabs, flat or held.
+static void check_kernel(int V, int64_t N, int64_t D, int64_t C, const char* want) {
+  for (const bool bwd : {false, true}) {
+    const int cus = 256;
+    const FlatPlan p = plan_cl(bwd, V, N, C, D, cus).flat;
+    const char got = !p.on ? 's' : (p.hold ? 'h' : 'f');
+    EXPECT(got == want[bwd]);
+  }
+}
+static void check_quoted() {
+  check_kernel(8, 22, 14280, 17, "ff");
+  check_kernel(8, 51, 7684, 87, "fh");
+  check_kernel(8, 28, 1275, 162, "ff");
+  check_kernel(8, 48, 304, 74, "ss");
+  check_kernel(8, 1, 598464, 17, "fh");
+  check_kernel(8, 2, 85000, 133, "fh");
+  check_kernel(8, 4, 1664, 428, "ss");
+  check_kernel(8, 3, 14016, 428, "ss");
+  check_kernel(8, 5, 75264, 116, "hh");
+  check_kernel(8, 38, 3328, 85, "ff");
+  check_kernel(8, 50, 1248, 53, "fs");
+  check_kernel(8, 20, 2920, 175, "fs");
+  check_kernel(8, 11, 7104, 190, "fh");
+  check_kernel(8, 33, 23808, 64, "fh");
+  check_kernel(4, 15, 5488, 104, "fh");
+  check_kernel(8, 12, 3408, 448, "ss");
+  check_kernel(8, 64, 16384, 64, "ff");
+  check_kernel(8, 32, 65536, 32, "fh");
+  check_kernel(8, 11, 20592, 128, "hh");
+  check_kernel(8, 17, 30940, 57, "fh");
+  check_kernel(8, 28, 92880, 16, "sh");
+  check_kernel(8, 36, 30000, 32, "sh");
+  check_kernel(4, 5, 15779, 192, "sh");
+  check_kernel(8, 1, 89514, 125, "fh");
+  check_kernel(4, 2, 12673, 124, "ss");
+  check_kernel(8, 38, 3168, 100, "ff");
+  check_kernel(8, 2, 50000, 320, "ss");
+  check_kernel(8, 3, 100000, 300, "sh");
+  check_kernel(8, 36, 57624, 16, "sh");
+  check_kernel(4, 8, 16384, 64, "ss");
+  check_kernel(8, 16, 8192, 128, "ss");
+  check_kernel(8, 24, 16384, 48, "sh");
+  check_kernel(8, 20, 16384, 64, "sh");
+  check_kernel(8, 9, 72447, 32, "hh");
+  check_kernel(8, 16, 65536, 64, "hh");
+  check_kernel(8, 8, 524288, 32, "hh");
+  check_kernel(8, 2, 2097152, 32, "hh");
+}
+
 int main() {
+  check_quoted();
   check_refused_early(8, 8, 64, 16384);
   check_refused_early(8, 2, 320, 216);
   check_refused_early(8, 100, 64, 2048 / 2);
