@@ -40,9 +40,19 @@ HOT = [
     "13cl_bwd_singleIDF16_Li8ELi8ELb1ELb0EE",
     "16plane_fwd_singleIDF16_Li8ELi8ELb1ELb1EE",                # IN [2, 32, 128^3] channel-first
     "16plane_fwd_singleIDF16bLi8ELi8ELb1ELb1EE",                # ... in bf16
-    "12cl_fwd_statsIDF16_Li8ELi0E", "11cl_bwd_sumsIDF16_Li8ELi0E",  # IN [2, 128^3, 32] channels-last
+    "12cl_fwd_statsIDF16_Li8ELi0E", "11cl_bwd_sumsIDF16_Li8ELi0E",  # IN [2, 128^3, 32] channels-last, in place
     "12cl_fwd_applyIDF16_Li8ELi0E", "12cl_bwd_applyIDF16_Li8ELi0E",
+    "13rows_bwd_pairIDF16_Li8ELi64ELi2ELi4E",                   # LN [32, 1024] backward
 ]
+
+# Kernels whose fallback is a function of its own: its frame is reserved, and used only there.  (pattern, bytes of
+# it, waves per SIMD that the rest of the kernel is built for)
+OUT_OF_LINE = [
+    (r"11cl_flat_(fwd|bwd)I", 272, 4),
+    (r"11cl_hold_(fwd|bwd)I", 288, 2),
+]
+# ... of which the configurations run
+HOT_OUT_OF_LINE = ["11cl_hold_fwdIDF16_Li8ELi36ELi12ELb1ELi4EE", "11cl_hold_bwdIDF16_Li8ELi18ELi6ELb1ELi2EE"]  # IN [2, 128^3, 32] channels-last
 
 
 @pytest.fixture(scope="module")
@@ -61,6 +71,7 @@ def kernels():
 def test_the_report_covers_the_library(kernels):
     units = {r["unit"] for r in kernels.values()}
     assert {"rows_launch_f32", "rows_launch_f16", "rows_launch_bf16", "cl_launch", "dispatch"} <= units
+    assert {"cl_flat_launch_f32", "cl_flat_launch_f16", "cl_flat_launch_bf16"} <= units
     assert len(kernels) > 1000
     for name, r in kernels.items():
         assert {"vgprs", "sgprs", "scratch_bytes_per_lane", "vgpr_spills", "waves_per_simd"} <= set(r), name
@@ -84,6 +95,25 @@ def test_the_configurations_kernels_use_no_scratch_memory(kernels):
         assert hits, f"no kernel matches {frag}: has an instantiation been renamed?"
         for n in hits:
             assert kernels[n]["scratch_bytes_per_lane"] == 0, f"{n}: {kernels[n]}"
+
+
+def test_fallbacks_out_of_line_keep_to_their_frame(kernels):
+    """The flat and held kernels keep their vectors in registers: nothing is spilled, and the scratch memory is
+    that of the call which a workgroup makes when its wait has run out."""
+    for pattern, frame, waves in OUT_OF_LINE:
+        ours = {n: r for n, r in kernels.items() if re.search(pattern, n)}
+        assert len(ours) >= 3 * 8
+        for name, r in ours.items():
+            assert r["vgpr_spills"] == 0 and r["scratch_bytes_per_lane"] <= frame and r["waves_per_simd"] >= waves, f"{name}: {r}"
+    for frag in HOT_OUT_OF_LINE:
+        assert any(frag in n for n in kernels), f"no kernel matches {frag}: has an instantiation been renamed?"
+
+
+def test_no_other_kernel_calls_out_of_line(kernels):
+    for name, r in kernels.items():
+        if any(re.search(pattern, name) for pattern, _, _ in OUT_OF_LINE) or r["vgpr_spills"] > 0:
+            continue
+        assert r["scratch_bytes_per_lane"] == 0, f"{name}: {r}"
 
 
 def test_held_vectors_lie_on_16_bytes_in_lds(kernels):
