@@ -583,7 +583,7 @@ def shared_gpu_reference(name, occupier_wgs=128, hold_ms=20.0, reps=7):
             return e0.elapsed_time(e1) * 1e3
 
         for knob, label in ((1, "exchange"), (0, "two_launch")):
-            for nm in (b"cl_single", b"plane_single", b"affine_fold"):
+            for nm in (b"cl_single", b"cl_flat", b"cl_hold", b"plane_single", b"affine_fold"):
                 L.atexn_set_tuning(nm, knob)
             L.atexn_bench_mark_exchange_trouble(0)
             case.fwd(0)
@@ -595,7 +595,7 @@ def shared_gpu_reference(name, occupier_wgs=128, hold_ms=20.0, reps=7):
                           "bwd_first_us": b[0], "bwd_us": float(np.median(b[1:]))}
         del case
     finally:
-        for nm in (b"cl_single", b"plane_single", b"affine_fold"):
+        for nm in (b"cl_single", b"cl_flat", b"cl_hold", b"plane_single", b"affine_fold"):
             L.atexn_set_tuning(nm, 1)
         L.atexn_bench_mark_exchange_trouble(0)
         USE_BENCH_LIB_EVERYWHERE = saved
