@@ -11,6 +11,14 @@ namespace atexn {
 static_assert(kPlanFlatMaxSlabs == kFlatMaxSlabs && kPlanFlatMaxThreads == kFlatMaxThreads,
               "the planner and the flat kernels must agree on their limits");
 
+// float32 backwards go on the held kernels or stay on the slabs' (flat_may): the flat ones are built only where
+// a switch can ask for them.
+#ifdef ATEXN_BENCH_BUILD
+constexpr bool kFlatBwdAnyWidth = true;
+#else
+constexpr bool kFlatBwdAnyWidth = false;
+#endif
+
 inline FlatArgs flat_args(const FlatPlan& p, int64_t N, int64_t C, int64_t D, void* ws, const ExchangeTag& e) {
   char* w = static_cast<char*>(ws);
   FlatArgs a;
@@ -116,18 +124,22 @@ int flat_bwd_v(const FlatPlan& p, const T* dy, const T* x, const float* gamma, c
     if (N > 1) return launch_col_reduce(part, dgamma, dbeta, static_cast<int>(N), C, st);
     return ATEXN_OK;
   }
+  if constexpr (V == 8 || kFlatBwdAnyWidth) {
 #define ATEXN_FLAT_BWD(U_) \
   case U_: cl_flat_bwd<T, V, U_><<<grid, p.threads, p.lds, st>>>(dy, x, gamma, mean, rstd, dx, o0, o1, 2 * C, a); break
-  switch (p.U) {
-    ATEXN_FLAT_BWD(1);
-    ATEXN_FLAT_BWD(2);
-    ATEXN_FLAT_BWD(3);
-    ATEXN_FLAT_BWD(4);
-    ATEXN_FLAT_BWD(6);
-    ATEXN_FLAT_BWD(8);
-    default: return set_error(ATEXN_INVALID_ARGUMENT, "no kernel for %d vectors per thread", p.U);
-  }
+    switch (p.U) {
+      ATEXN_FLAT_BWD(1);
+      ATEXN_FLAT_BWD(2);
+      ATEXN_FLAT_BWD(3);
+      ATEXN_FLAT_BWD(4);
+      ATEXN_FLAT_BWD(6);
+      ATEXN_FLAT_BWD(8);
+      default: return set_error(ATEXN_INVALID_ARGUMENT, "no kernel for %d vectors per thread", p.U);
+    }
 #undef ATEXN_FLAT_BWD
+  } else {
+    return set_error(ATEXN_INVALID_ARGUMENT, "no flat backward for vectors of %d elements", V);
+  }
   ATEXN_CHECK_LAUNCH("cl_flat_bwd");
   if (N > 1) return launch_col_reduce(part, dgamma, dbeta, static_cast<int>(N), C, st);
   return ATEXN_OK;

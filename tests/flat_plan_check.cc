@@ -71,6 +71,7 @@ static void check(bool hold, bool bwd, int V, int64_t N, int64_t C, int64_t D, i
   EXPECT(p.off_finals % 16 == 0 && p.off_claims % 16 == 0 && p.off_part % 16 == 0 && p.off_tag % 4 == 0);
   // the call's plan has room for it and for the kernels that serve y == x
   const ClPlan c = plan_cl(bwd, V, N, C, D, cus);
+  EXPECT(!c.flat.on || c.flat.hold || !bwd || V == 8);  // (the product has no other flat backward)
   EXPECT(!c.flat.on || (c.ws_bytes >= c.flat.ws_bytes && c.ws_bytes >= plan_cl_slabs(bwd, V, N, C, D, cus).ws_bytes));
 }
 

@@ -105,6 +105,7 @@ def test_fallbacks_out_of_line_keep_to_their_frame(kernels):
         assert len(ours) >= 3 * 8
         for name, r in ours.items():
             assert r["vgpr_spills"] == 0 and r["scratch_bytes_per_lane"] <= frame and r["waves_per_simd"] >= waves, f"{name}: {r}"
+    assert not any("11cl_flat_bwdIf" in n for n in kernels)  # (no rule chooses them)
     for frag in HOT_OUT_OF_LINE:
         assert any(frag in n for n in kernels), f"no kernel matches {frag}: has an instantiation been renamed?"
 
