@@ -291,6 +291,40 @@ def test_waits_cut_short_find_peers_that_are_running(N, S, C, dtype):
         capi.L.atexn_bench_mark_exchange_trouble(0)
 
 
+@pytest.mark.parametrize("N,S,C,dtype", [(2, 2097152, 32, "f16"), (3, 703459, 23, "bf16")])
+def test_held_calls_on_two_streams(N, S, C, dtype):
+    """Two calls at a time, each of which wants the whole chip: their instances take CUs from each other between
+    two instances of a call.  The bits of calls one after another."""
+    import torch
+
+    capi = util.Capi(bench=True)
+    calls = _channels_last_calls(capi, N, S, C, dtype)
+    side = _stream_beside(capi.L)
+    alone = [call() for call in calls]
+    torch.cuda.synchronize()
+    main = torch.cuda.current_stream()
+    e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    for first, second in ((0, 0), (0, 1), (1, 1)):
+        got = []
+        torch.cuda.synchronize()
+        torch.cuda._sleep(400000)
+        e[0].record()
+        side.wait_stream(main)
+        for _ in range(4):
+            got.append((first, calls[first]()))
+            with torch.cuda.stream(side):
+                got.append((second, calls[second]()))
+        main.wait_stream(side)
+        e[1].record()
+        torch.cuda.synchronize()
+        print(f"[{N}, {S}, {C}] {dtype}: eight calls on two streams {e[0].elapsed_time(e[1]) * 1e3:.0f} us", flush=True)
+        for which, out in got:
+            for a, b in zip(out, alone[which]):
+                assert torch.equal(_bits(a), _bits(b))
+        del got
+    capi.L.atexn_bench_mark_exchange_trouble(0)
+
+
 @pytest.mark.parametrize("N,S,C,dtype", [(2, 2097152, 32, "f32"), (1, 1 << 24, 64, "bf16")])
 def test_patience_grows_with_the_slabs(N, S, C, dtype):
     """Instances of 268 MB and 2 GB on a free GPU: nobody runs out of a wait, cut short or not, whose slab is merely
