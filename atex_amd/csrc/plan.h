@@ -221,36 +221,21 @@ struct PairPlan {
   int strip = 4;         // vectors of a column workgroup (4 or 8)
   int row_blocks = 0, grid = 0;
 };
-// How many rows at most, by the vectors of a row: the second read of x and dy against the partial rows of the row
-// kernels and the launch that folds them, which fare differently with rows of whole vectors and others (masks).
-// Measured with operands that the L2s do not have (96 MB of them in turn) at 32 to 1024 rows of 2 to 2048 vectors; a
-// line lies where the sides cross (us, row kernels -> this).  16 bits: [256, 256] 5.5 -> 5.2, beyond the line
-// [1024, 256] 6.1 -> 8.5, [1024, 255] 6.3 -> 9.3, [512, 512] 6.0 -> 7.3; [512, 4096] 11.4 -> 10.0; [768, 10503]
-// 31.1 -> 22.2, [640, 16384] 24.9 -> 23.5; the worst of those taken [512, 2560] 10.2 -> 10.6.  float32, whose column
-// workgroups read twice the bytes: [160, 256] 5.3 -> 5.2, beyond the line [512, 256] 5.6 -> 7.5, [512, 1028]
-// 7.9 -> 10.5, [512, 2048] 8.5 -> 10.0; [192, 2048] 7.9 -> 6.5, [448, 4096] 12.3 -> 10.2.  Rows of 17 to 24 vectors
-// leave the row kernels' lanes partly idle: [768, 192] fp16 7.8 -> 7.0.
-// Strips of 8 vectors, whole cache lines, where that leaves enough workgroups: [256, 10501] 13.5 -> 9.8.
-struct PairRows {
-  int vectors, whole, ragged;  // rows of up to so many vectors: at most so many rows
-};
-constexpr PairRows kPlanPair16[] = {{6, 896, 192},   {16, 448, 128},  {24, 1024, 704}, {32, 320, 192},  {48, 512, 512},  {63, 416, 192},
-                                    {64, 192, 192},  {127, 512, 480}, {128, 352, 480}, {512, 512, 512}, {1023, 768, 640}, {2048, 768, 768}};
-constexpr PairRows kPlanPair32[] = {{4, 1024, 1024}, {8, 352, 576},   {16, 288, 192},  {24, 448, 224},  {32, 192, 160},  {63, 320, 192},
-                                    {64, 160, 192},  {127, 256, 192}, {128, 160, 192}, {256, 192, 224}, {319, 416, 224}, {512, 192, 224},
-                                    {1023, 480, 480}, {2048, 448, 512}};
-inline int64_t pair_most_rows(int V, int64_t n_vec, bool ragged) {
-  const PairRows* r = V == 8 ? kPlanPair16 : kPlanPair32;
-  while (n_vec > r->vectors) ++r;
-  return ragged ? r->ragged : r->whole;
-}
+// How many rows: the second read of x and dy against the partial rows of the row kernels and the launch
+// that folds them (us, row kernels -> this).  Up to 512: fp16 [32, 1024] 7.7 -> 4.9, [128, 10501] 20.1 ->
+// 8.4, [256, 13845] 22.2 -> 11.0, [512, 4096] 11.4 -> 10.4, float32 [512, 1024] 8.3 -> 8.1, [512, 7575] 22.0 ->
+// 21.0; more where a row of 16-bit data is long ([768, 10501] 31.0 -> 23.6; [768, 4096] 12.5 -> 12.9, float32
+// [768, 7575] 25.3 -> 30.2) or so short that the launches are all there is ([1024, 256] 8.9 -> 8.1;
+// [1024, 1024] 8.6 -> 10.1).  Strips of 8 vectors, whole cache lines, where that leaves enough workgroups:
+// [256, 10501] 13.5 -> 9.8.
 inline PairPlan plan_pair(int V, int64_t n_rows, int64_t D) {
   PairPlan p;
   const int how = tuning().pair_rows;
   const int64_t n_vec = div_up(D, V);
   if (how == 0 || V == 1 || D < V || n_vec > 2048) return p;
   if (!tuning().long_rows && n_vec > 1536) return p;  // (a switch: such rows on the kernels that serve dx == dy)
-  if (n_rows > (how == 2 ? 65536 : pair_most_rows(V, n_vec, D % V != 0))) return p;
+  const int64_t most = n_vec <= 32 ? 1024 : (V == 8 && n_vec > 512 ? 768 : 512);
+  if (n_rows > (how == 2 ? 65536 : most)) return p;
   p.tpr = n_vec <= 256 ? 64 : 512;
   p.vpt = n_vec <= p.tpr ? 1 : (n_vec <= 2 * p.tpr ? 2 : 4);
   p.strip = n_vec > 512 ? 8 : 4;

@@ -20,15 +20,6 @@ def _describe(capi, N, D, dtype):
     return text.value.decode()
 
 
-@pytest.fixture
-def wherever():
-    """The kernel beyond the lines of the product's rule too."""
-    capi = util.Capi(bench=True)
-    assert capi.L.atexn_set_tuning(b"pair_rows", 2) == 0
-    yield capi
-    capi.L.atexn_set_tuning(b"pair_rows", 1)
-
-
 # strips of 4 and 8 vectors and what is left of one; rows of 1 to 2048 vectors on a wave (up to 256) and on a
 # workgroup; 1, 8, 9 rows, around 64 / 128 rows at once and around a batch of 8 steps
 @pytest.mark.parametrize("N,D,dtype", [
@@ -36,10 +27,10 @@ def wherever():
     (127, 2048, "f16"), (512, 2049, "f16"), (1024, 250, "bf16"), (65, 4096, "f16"), (513, 4097, "bf16"), (33, 4104, "f16"),
     (10, 8191, "f16"), (768, 8200, "f16"), (5, 16384, "bf16"), (31, 8189, "f32"), (2, 8192, "f32"),
 ])
-def test_few_rows_in_one_launch(wherever, coracle, N, D, dtype):
+def test_few_rows_in_one_launch(coracle, N, D, dtype):
     import torch
 
-    capi = wherever
+    capi = util.Capi(bench=True)
     what = _describe(capi, N, D, dtype)
     print(f"pair rows N={N} D={D} {dtype}: {what}", flush=True)
     assert what.startswith("rows_bwd_pair")

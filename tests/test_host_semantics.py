@@ -297,23 +297,6 @@ def test_every_planning_parameter_is_settable_in_the_benchmark_build():
         assert buf.value.startswith(b"plane_bwd_ragged") and buf.value.endswith(b"alone=0"), buf.value
 
 
-def test_few_rows_take_one_launch_where_it_is_the_faster_one():
-    """Both sides of the lines of the LayerNorm backward's rule, by dtype, rows of whole vectors and others."""
-    L = _capi.bench_lib()
-    buf = ctypes.create_string_buffer(256)
-
-    def one_launch(dtype, rows, cols):
-        assert L.atexn_bench_describe_bwd(0, dtype, 0, rows, 0, cols, buf, 256) > 0
-        return buf.value.startswith(b"rows_bwd_pair")
-
-    for dtype, rows, cols in ((1, 256, 256), (1, 192, 255), (1, 1024, 192), (2, 512, 4096), (1, 768, 10504), (1, 640, 16384),
-                              (1, 1, 8), (0, 160, 256), (0, 192, 2048), (0, 416, 1028), (0, 448, 4096), (0, 2, 8192)):
-        assert one_launch(dtype, rows, cols), (dtype, rows, cols)
-    for dtype, rows, cols in ((1, 1024, 256), (1, 1024, 255), (2, 512, 512), (1, 513, 4096), (1, 769, 10504), (1, 641, 5001),
-                              (0, 512, 256), (0, 512, 1028), (0, 512, 2048), (0, 449, 4096), (0, 1024, 128), (1, 8, 16392)):
-        assert not one_launch(dtype, rows, cols), (dtype, rows, cols)
-
-
 def test_workspace_queries_without_gpu(L):
     """Usable on a host without a GPU (they assume 256 CUs) and monotone in the obvious way."""
     assert L.atexn_layer_norm_fwd_workspace_bytes(1, 8192, 1024) == 0       # register-resident rows
