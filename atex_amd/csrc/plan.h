@@ -222,12 +222,16 @@ struct PairPlan {
   int row_blocks = 0, grid = 0;
 };
 // How many rows: the second read of x and dy against the partial rows of the row kernels and the launch
-// that folds them (us, row kernels -> this).  Up to 512: fp16 [32, 1024] 7.7 -> 4.9, [128, 10501] 20.1 ->
-// 8.4, [256, 13845] 22.2 -> 11.0, [512, 4096] 11.4 -> 10.4, float32 [512, 1024] 8.3 -> 8.1, [512, 7575] 22.0 ->
-// 21.0; more where a row of 16-bit data is long ([768, 10501] 31.0 -> 23.6; [768, 4096] 12.5 -> 12.9, float32
-// [768, 7575] 25.3 -> 30.2) or so short that the launches are all there is ([1024, 256] 8.9 -> 8.1;
-// [1024, 1024] 8.6 -> 10.1).  Strips of 8 vectors, whole cache lines, where that leaves enough workgroups:
-// [256, 10501] 13.5 -> 9.8.
+// that folds them.  What decides is the call as a program makes it, where a launch costs more than what it does: the
+// step of forward and backward, back to back, with the row kernels -> with this (us): fp16 [1024, 256] 13.7 -> 10.7,
+// [512, 512] 14.1 -> 11.4, bf16 [1024, 255] 14.1 -> 11.2, float32 [512, 1028] 14.9 -> 12.6, [512, 2048] 13.8 -> 12.9,
+// [512, 4100] 18.6 -> 15.8.  Backward calls alone: fp16 [32, 1024] 7.7 -> 4.9, [128, 10501] 20.1 -> 8.4,
+// [256, 13845] 22.2 -> 11.0, float32 [512, 7575] 22.0 -> 21.0; more rows where one of 16-bit data is long
+// ([768, 10501] 31.0 -> 23.6; at its edge [640, 4104] 14.2 -> 13.1, [768, 4104] 15.3 -> 15.5; [768, 4096] 12.5 -> 12.9,
+// float32 [768, 7575] 25.3 -> 30.2) or so short that the launches are all there is ([1024, 256] 8.9 -> 8.1;
+// [1024, 1024] 8.6 -> 10.1).  The kernels' own time, which is what a recorded graph has, is the other way round where
+// neither a launch nor traffic is saved: [1024, 256] 5.8 against 7.7, float32 [512, 1028] 8.0 against 10.2.
+// Strips of 8 vectors, whole cache lines, where that leaves enough workgroups: [256, 10501] 13.5 -> 9.8.
 inline PairPlan plan_pair(int V, int64_t n_rows, int64_t D) {
   PairPlan p;
   const int how = tuning().pair_rows;
