@@ -17,7 +17,7 @@
 //
 // Bound by memory with data, by the exchange's two hops (about 4 us with the merges in LDS) without:
 // forward [28, 13300, 29] bf16 13.7 us (two stages 26.7; 43 MB at 5.5 TB/s: 7.9), [36, 36288, 29] fp16 31.6
-// (59.1; 27.6), backward 61.4 (104; 41.3).  128 registers, four waves per SIMD: what a launch can hold at
+// (59.1; 27.6), backward [22, 14280, 17] fp16 14.3 (22.9; 5.8).  128 registers, four waves per SIMD: what a launch can hold at
 // once counts for more than the next slab's loads in flight.
 //
 // Nothing depends on which workgroups are on the chip together.  A workgroup publishes its slab's sums

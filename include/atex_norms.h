@@ -32,9 +32,11 @@
  *     call on kernels that need no group of workgroups resident on the GPU together (for some
  *     InstanceNorm shapes two launches per direction instead of one, for LayerNorm rows of more
  *     than one workgroup three or four; same results up to the order of a few float32 additions,
- *     same workspace sizes) -- for processes that keep other kernels running on more than half
- *     of the GPU's compute units all the time, under which the one-launch kernels are correct but
- *     two to three times slower than the others;
+ *     same workspace sizes) -- for processes that keep other kernels running on the GPU all the
+ *     time.  Beside such a kernel the one-launch kernels are correct but slower than the others:
+ *     two to three times when it holds more than half of the compute units; channels-last
+ *     instances of some 20 MiB and more, which take the whole GPU, 1.4 to 2 times as soon as it
+ *     holds one;
  *   - the device the stream belongs to must be the calling thread's current device: launch
  *     plans and workspace sizes are made for the current device's compute-unit count;
  *   - data pointers need only the alignment of their element type (2 or 4 bytes): the
@@ -96,7 +98,8 @@ int atexn_layer_norm_fwd(int dtype, const void* x, const float* gamma, const flo
                          void* stream);
 
 /* Replaces functor::FusedLayerNormGrad<GPUDevice,T,U>::operator()
- * (cc/kernels/fused_layer_norm_op.cu:895-1030). dx may alias dy (in-place gradient), not x. */
+ * (cc/kernels/fused_layer_norm_op.cu:895-1030). dx may alias dy (in-place gradient), not x; dgamma
+ * and dbeta must not overlap any input. */
 size_t atexn_layer_norm_bwd_workspace_bytes(int dtype, int64_t N, int64_t D);
 int atexn_layer_norm_bwd(int dtype, const void* dy, const void* x, const float* gamma,
                          const float* mean, const float* inv_std, int64_t N, int64_t D,
@@ -134,8 +137,8 @@ int atexn_instance_norm_fwd(int dtype, int layout, const void* x, const float* g
                             void* workspace, size_t workspace_bytes, void* stream);
 
 /* Replaces functor::FusedInstanceNormGrad<GPUDevice,T,U>::operator()
- * (cc/kernels/fused_instance_norm_op.cu:1519-1561). dgamma / dbeta are [C]; dx may alias dy,
- * not x. */
+ * (cc/kernels/fused_instance_norm_op.cu:1519-1561). dgamma / dbeta are [C] and must not overlap any
+ * input; dx may alias dy, not x. */
 size_t atexn_instance_norm_bwd_workspace_bytes(int dtype, int layout, int64_t N, int64_t C,
                                                int64_t D);
 int atexn_instance_norm_bwd(int dtype, int layout, const void* dy, const void* x,
