@@ -22,15 +22,15 @@ unsigned next_call_tag();
 
 // Whether a call on stream `st` may take the InstanceNorm kernels whose workgroups exchange partial
 // results under a tag from the host.  Not while the stream is being captured (a graph replay would
-// repeat the call's tag; LayerNorm's long rows and ragged planes take theirs from exchange_tag below and
-// are recorded as they are), and neither these nor those in a process started with ATEXN_NO_EXCHANGE set
+// repeat the call's tag; LayerNorm's long rows, ragged planes and flat and held channels-last instances take
+// theirs from exchange_tag below and are recorded as they are), and neither these nor those in a process started with ATEXN_NO_EXCHANGE set
 // to anything but "0": such kernels need the workgroups of one instance / plane on the chip together, which a process that
 // keeps other kernels resident on the same GPU (communication kernels overlapped with compute)
 // may never give them; every wait then runs out and every workgroup recomputes its peers' share.
 // The results are the same; the time is not.  The variable is read once, at the first call.
 bool exchange_allowed(void* st);
 
-// The current device's word for exchange_polls / exchange_gave_up (norm_common.hip.h): a static
+// The current device's word for exchange_wait_pair (norm_common.hip.h): a static
 // device variable of the library, looked up once per device.  nullptr if that fails (the kernels
 // then always wait patiently).
 unsigned* exchange_trouble_word();
