@@ -356,16 +356,17 @@ int tiles_bwd(const T* dy, const T* x, const float* gamma, const float* mean, co
   return launch_col_reduce(part, dgamma, dbeta, p.sums_RS, D, st);
 }
 
-// rows_bwd_pair reads gamma and the statistics while it writes dgamma and dbeta; the row kernels write them last.
-inline bool pair_outputs_apart(const float* gamma, const float* mean, const float* rstd, int64_t n_rows, int64_t D,
-                               const float* dgamma, const float* dbeta) {
+// rows_bwd_pair reads its inputs while it writes dgamma and dbeta; the row kernels write them last.
+template <typename T>
+inline bool pair_outputs_apart(const T* dy, const T* x, const float* gamma, const float* mean, const float* rstd,
+                               int64_t n_rows, int64_t D, const float* dgamma, const float* dbeta) {
   bool apart = true;
   for (const float* out : {dgamma, dbeta}) {
-    auto from = [&](const float* in, int64_t n) {
+    auto from = [&](const auto* in, int64_t n) {
       const uintptr_t o = reinterpret_cast<uintptr_t>(out), i = reinterpret_cast<uintptr_t>(in);
-      return o >= i + sizeof(float) * static_cast<size_t>(n) || i >= o + sizeof(float) * static_cast<size_t>(D);
+      return o >= i + sizeof(*in) * static_cast<size_t>(n) || i >= o + sizeof(float) * static_cast<size_t>(D);
     };
-    apart = apart && from(gamma, D) && from(mean, n_rows) && from(rstd, n_rows);
+    apart = apart && from(gamma, D) && from(mean, n_rows) && from(rstd, n_rows) && from(x, n_rows * D) && from(dy, n_rows * D);
   }
   return apart;
 }
@@ -405,7 +406,7 @@ int rows_bwd_v(const T* dy, const T* x, const float* gamma, const float* mean, c
     const bool one_launch = static_cast<const void*>(dx) != static_cast<const void*>(dy) && bwd_stage_mask() == 3;
     if (one_launch) {
       const PairPlan pair = plan_pair(V, n_rows, D);
-      if (pair.on && pair_outputs_apart(gamma, mean, rstd, n_rows, D, dgamma, dbeta)) return pair_bwd_launch<T>(pair, dy, x, gamma, mean, rstd, n_rows, D, dx, dgamma, dbeta, st);
+      if (pair.on && pair_outputs_apart(dy, x, gamma, mean, rstd, n_rows, D, dgamma, dbeta)) return pair_bwd_launch<T>(pair, dy, x, gamma, mean, rstd, n_rows, D, dx, dgamma, dbeta, st);
     }
     if (p.lr.on && one_launch) {
       ExchangeTag tag;

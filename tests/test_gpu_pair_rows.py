@@ -57,8 +57,8 @@ def test_few_rows_in_one_launch(coracle, N, D, dtype):
 
 @pytest.mark.parametrize("N,D,dtype", [(32, 1024, "f16"), (512, 4096, "bf16"), (200, 2051, "f32")])
 def test_gradients_over_the_weights_keep_the_row_kernels(N, D, dtype):
-    """dgamma written over gamma (dbeta over gamma, or into its second half): the bits of the row kernels, which
-    write them when everything is read."""
+    """dgamma written over gamma (dbeta over gamma, or into its second half) or over x or dy: the bits of the row
+    kernels, which write them when everything is read."""
     import torch
 
     capi = util.Capi(bench=True)
@@ -90,6 +90,19 @@ def test_gradients_over_the_weights_keep_the_row_kernels(N, D, dtype):
     for place in ((0, D), (D, 0), (D // 2, 2 * D)):
         for name, a, b in zip(("dx", "dgamma", "dbeta"), run(place), want):
             assert bool((a == b).all()), f"{place}: {name}"
+    # ... and over x and dy
+    half = 2 * D if dtype != "f32" else D  # elements that D floats cover
+    for over_x, over_dy in ((True, False), (False, True), (True, True)):
+        ops = {True: xd.clone(), False: dyd.clone()}
+        out = [ops[k].view(-1)[:half].view(torch.float32) if over else torch.empty(D, device="cuda")
+               for k, over in ((True, over_x), (False, over_dy))]
+        dx = torch.empty_like(xd)
+        assert L.atexn_layer_norm_bwd(code, ops[False].data_ptr(), ops[True].data_ptr(), gd.data_ptr(), m.data_ptr(), r.data_ptr(),
+                                      N, D, dx.data_ptr(), out[0].data_ptr(), out[1].data_ptr(), ws.data_ptr(), need,
+                                      torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        for name, a, b in zip(("dx", "dgamma", "dbeta"), (dx, *out), want):
+            assert bool((a == b).all()), f"over x {over_x}, over dy {over_dy}: {name}"
 
 
 def test_more_rows_stay_on_the_row_kernels():
